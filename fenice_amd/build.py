@@ -18,7 +18,8 @@ LIB = os.path.join(HERE, "libfvg.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("FVG_ARCH", "gfx950")
 
-SOURCES = ["fvg_kernels_f64.hip", "fvg_kernels_f32.hip", "fvg_kernels_f4.hip", "fvg_kernels.hip", "fvg_api.hip", "fvg_batch.hip", "fvg_learned.hip", "fvg_noalloc.hip",
+SOURCES = ["fvg_kernels_f64.hip", "fvg_fused_f64.hip", "fvg_learned_f64.hip", "fvg_batch.hip", "fvg_fused_f32.hip", "fvg_kernels_f32.hip",
+           "fvg_kernels_f4.hip", "fvg_learned_f32.hip", "fvg_kernels.hip", "fvg_api.hip", "fvg_learned.hip", "fvg_noalloc.hip",
            "fvg_config.cpp", "fvg_checkpoint.cpp", "fvg_npz.cpp"]
 COMMON = ["-O3", "-std=c++17", "-fPIC", "-ffp-contract=off", "-fno-fast-math", "-Wall",
           "-I" + os.path.join(ROOT, "include")]
@@ -48,7 +49,7 @@ def build(verbose: bool = False) -> str:
         objs.append(obj)
         if verbose:
             print(" ".join(cmds[-1]), flush=True)
-    with ThreadPoolExecutor(max_workers=min(6, len(cmds))) as ex:
+    with ThreadPoolExecutor(max_workers=min(8, len(cmds))) as ex:
         list(ex.map(_run, cmds))
     tmp = LIB + ".tmp"
     _run([HIPCC, "-shared", f"--offload-arch={ARCH}", "-o", tmp, *objs])

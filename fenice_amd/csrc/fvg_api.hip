@@ -21,10 +21,10 @@
 namespace fvg {
 template <int NV, typename T> __global__ void k_cells(KP);
 template <int NV> __global__ void k_hancock(KP);
-template <int NV, int D, int MODE, typename T> __global__ void k_faces(KP);
+template <int NV, int D, int MODE, int RECON, bool PER, typename T> __global__ void k_faces(KP);
 template <int NV, int UPD, typename T> __global__ void k_update(KP, const double*, const double*, double*);
 template <int NV, int WHAT> __global__ void k_totals_partial(const double*, long long, double*);
-template <int NV, int D, int USE, typename T> __global__ void k_faces_learned(KP);
+template <int NV, int D, int USE, bool PER, typename T> __global__ void k_faces_learned(KP);
 template <int NV, int MODE, int USE, typename T> __global__ void k_xacc(KP);
 template <int NV, int D, int MODE, int USE, int UPD, typename T> __global__ void k_lacc(KP, const double*, const double*, double*);
 template <int NV> __global__ void k_axpy(KP, const double*, const double*, double*);
@@ -213,6 +213,41 @@ int enqueue_massflow(fvg_ctx* c, const KP& p) {
     return rc;
 }
 
+// the faces normal to D in the variant of the configuration: the reconstruction, and whether the axis has a periodic halo
+template <int NV, int D, int MODE, int RECON, typename T>
+int launch_faces_recon(fvg_ctx* c, const KP& p) {
+    const dim3 g(faces_grid(c, D)), b(faces_block(c, D));
+    return launch(c, FAM_FACES_X + D, [&] {
+        if (p.wrap[D]) hipLaunchKernelGGL((k_faces<NV, D, MODE, RECON, true, T>), g, b, 0, c->stream, p);
+        else hipLaunchKernelGGL((k_faces<NV, D, MODE, RECON, false, T>), g, b, 0, c->stream, p);
+    });
+}
+template <int NV, int D, typename T>
+int launch_faces(fvg_ctx* c, const KP& p, int mode) {
+    if (mode == MODE_FIRST_ORDER)
+        return launch(c, FAM_FACES_X + D, [&] {
+            hipLaunchKernelGGL((k_faces<NV, D, MODE_FIRST_ORDER, 0, false, T>), dim3(faces_grid(c, D)), dim3(faces_block(c, D)), 0, c->stream, p);
+        });
+    switch (p.recon) {
+    case FVG_RECON_MUSCL: return launch_faces_recon<NV, D, MODE_PLAIN, FVG_RECON_MUSCL, T>(c, p);
+    case FVG_RECON_WENO3: return launch_faces_recon<NV, D, MODE_PLAIN, FVG_RECON_WENO3, T>(c, p);
+    default: return launch_faces_recon<NV, D, MODE_PLAIN, FVG_RECON_WENO5, T>(c, p);
+    }
+}
+template <int NV, int D, typename T>
+int launch_faces_learned(fvg_ctx* c, const KP& p, bool reuse) {
+    const dim3 g(faces_grid(c, D)), b(faces_block(c, D));
+    return launch(c, FAM_FACES_X + D, [&] {
+        if (p.wrap[D]) {
+            if (reuse) hipLaunchKernelGGL((k_faces_learned<NV, D, LF_KEPT, true, T>), g, b, 0, c->stream, p);
+            else hipLaunchKernelGGL((k_faces_learned<NV, D, LF_STORE, true, T>), g, b, 0, c->stream, p);
+        } else {
+            if (reuse) hipLaunchKernelGGL((k_faces_learned<NV, D, LF_KEPT, false, T>), g, b, 0, c->stream, p);
+            else hipLaunchKernelGGL((k_faces_learned<NV, D, LF_STORE, false, T>), g, b, 0, c->stream, p);
+        }
+    });
+}
+
 // reuse (learned indicator, Runge-Kutta stages 2 and 3): the faces take the decisions the network made on the step's
 // first stage instead of running it again
 template <int NV, typename T>
@@ -225,21 +260,15 @@ int enqueue_residual_nv(fvg_ctx* c, const double* Uin, int mode, bool audit, boo
     if (mode == MODE_LEARNED) {
 #define LFACES(KERNEL, FAM, D, GRID, BLOCK) \
     launch(c, FAM, [&] { hipLaunchKernelGGL((KERNEL<NV, D, T>), dim3(GRID), dim3(BLOCK), 0, c->stream, p); })
-#define LEARNED(FAM, D)                                                                                                            \
-    launch(c, FAM, [&] {                                                                                                         \
-        if (reuse) hipLaunchKernelGGL((k_faces_learned<NV, D, LF_KEPT, T>), dim3(faces_grid(c, D)), dim3(faces_block(c, D)), 0, c->stream, p); \
-        else hipLaunchKernelGGL((k_faces_learned<NV, D, LF_STORE, T>), dim3(faces_grid(c, D)), dim3(faces_block(c, D)), 0, c->stream, p);     \
-    })
         if (audit) {
             if ((rc = LFACES(k_audit, FAM_AUDIT, 0, grid_for(c->nfa[0]), kBlock)) || (rc = LFACES(k_audit, FAM_AUDIT, 1, grid_for(c->nfa[1]), kBlock)))
                 return rc;
             if constexpr (NV == 5)
                 if ((rc = LFACES(k_audit, FAM_AUDIT, 2, grid_for(c->nfa[2]), kBlock))) return rc;
         }
-        if ((rc = LEARNED(FAM_FACES_X, 0)) || (rc = LEARNED(FAM_FACES_Y, 1))) return rc;
+        if ((rc = launch_faces_learned<NV, 0, T>(c, p, reuse)) || (rc = launch_faces_learned<NV, 1, T>(c, p, reuse))) return rc;
         if constexpr (NV == 5)
-            if ((rc = LEARNED(FAM_FACES_Z, 2))) return rc;
-#undef LEARNED
+            if ((rc = launch_faces_learned<NV, 2, T>(c, p, reuse))) return rc;
 #undef LFACES
         return FVG_OK;
     }
@@ -269,15 +298,9 @@ int enqueue_residual_nv(fvg_ctx* c, const double* Uin, int mode, bool audit, boo
     if (mode == MODE_HANCOCK)
         if ((rc = launch(c, FAM_HANCOCK, [&] { hipLaunchKernelGGL(k_hancock<NV>, dim3(grid_for(c->nc)), dim3(kBlock), 0, c->stream, p); })))
             return rc;
-#define FACES(D, M)                                                                                                                       \
-    launch(c, FAM_FACES_X + D, [&] { hipLaunchKernelGGL((k_faces<NV, D, M, T>), dim3(faces_grid(c, D)), dim3(faces_block(c, D)), 0, c->stream, p); })
-#define AXIS(D) (mode == MODE_PLAIN ? FACES(D, MODE_PLAIN) : FACES(D, MODE_FIRST_ORDER))
-    if ((rc = AXIS(0))) return rc;
-    if ((rc = AXIS(1))) return rc;
+    if ((rc = launch_faces<NV, 0, T>(c, p, mode)) || (rc = launch_faces<NV, 1, T>(c, p, mode))) return rc;
     if constexpr (NV == 5)
-        if ((rc = AXIS(2))) return rc;
-#undef AXIS
-#undef FACES
+        if ((rc = launch_faces<NV, 2, T>(c, p, mode))) return rc;
     return FVG_OK;
 }
 
@@ -285,14 +308,9 @@ int enqueue_residual_nv(fvg_ctx* c, const double* Uin, int mode, bool audit, boo
 template <int NV>
 int enqueue_hancock_faces(fvg_ctx* c, const KP& p) {
     int rc;
-#define HFACES(D)                                                                                                                         \
-    launch(c, FAM_FACES_X + D, [&] { hipLaunchKernelGGL((k_faces<NV, D, MODE_HANCOCK, double>), dim3(faces_grid(c, D)), dim3(faces_block(c, D)), 0, \
-                                                        c->stream, p); })
-    if ((rc = HFACES(0))) return rc;
-    if ((rc = HFACES(1))) return rc;
+    if ((rc = launch_faces_recon<NV, 0, MODE_HANCOCK, 0, double>(c, p)) || (rc = launch_faces_recon<NV, 1, MODE_HANCOCK, 0, double>(c, p))) return rc;
     if constexpr (NV == 5)
-        if ((rc = HFACES(2))) return rc;
-#undef HFACES
+        if ((rc = launch_faces_recon<NV, 2, MODE_HANCOCK, 0, double>(c, p))) return rc;
     return FVG_OK;
 }
 
@@ -693,6 +711,9 @@ void fill_kernel_params(const fvg_config& cfg, KP& p) {
     p.dx = cfg.Lx / cfg.nx;
     p.dy = cfg.Ly / cfg.ny;
     p.dz = cfg.Lz / cfg.nz;
+    p.inv_h[0] = 1.0 / p.dx;
+    p.inv_h[1] = 1.0 / p.dy;
+    p.inv_h[2] = 1.0 / p.dz;
     if (three) {   // Mesh::face_area / cell_volume (Core.hpp:94-99)
         p.Ax = p.dy * p.dz;
         p.Ay = p.dx * p.dz;
@@ -704,9 +725,7 @@ void fill_kernel_params(const fvg_config& cfg, KP& p) {
         p.Az = 0.0;
         p.inv_vol = 1.0 / (p.dx * p.dy);
     }
-    p.rs.eos.stiff = cfg.eos_type == FVG_EOS_STIFFENED;
-    p.rs.eos.gamma = cfg.gamma;
-    p.rs.eos.p_inf = p.rs.eos.stiff ? cfg.p_inf : 0.0;
+    p.rs.eos = make_eos(cfg.eos_type == FVG_EOS_STIFFENED, cfg.gamma, cfg.p_inf);
     p.rs.lowmach = cfg.riemann == FVG_LOWMACH_HLLC;
     p.rs.blend = cfg.shock_blend;
     for (int s = 0; s < 6; ++s) p.bp.bc[s] = cfg.bc[s];
@@ -725,6 +744,12 @@ void fill_kernel_params(const fvg_config& cfg, KP& p) {
     p.Dh = cfg.reconstruction == FVG_RECON_WENO5 ? 3 : 2;
     p.bo2 = cfg.boundary_order == 2;
     p.weno_eps = cfg.weno_epsilon;
+    // the in-range FP64 operations (fvg_device.hpp) need moderate constants as well as moderate primitives
+    auto moderate = [](double v, int e) { return std::fabs(v) >= std::ldexp(1.0, -e) && std::fabs(v) <= std::ldexp(1.0, e); };
+    auto moderate_or_zero = [&](double v) { return v == 0.0 || moderate(v, 100); };
+    p.ir = cfg.gamma > 1.0 && moderate(cfg.gamma - 1.0, 20) && p.rs.eos.p_inf >= 0.0 && moderate_or_zero(p.rs.eos.p_inf) &&
+           cfg.weno_epsilon > 0.0 && moderate(cfg.weno_epsilon, 40) && moderate_or_zero(cfg.u_in) && moderate_or_zero(cfg.v_in) &&
+           moderate_or_zero(cfg.p_out) && moderate_or_zero(cfg.rho_in) && moderate(p.dx, 100) && moderate(p.dy, 100) && moderate(p.dz, 100);
     // halos of the reconstruction (Simulation.cpp:863-905, 1109-1170)
     const int n3[3] = {cfg.nx, cfg.ny, cfg.nz};
     for (int a = 0; a < 3; ++a) {
@@ -1275,9 +1300,7 @@ int fvg_riemann_batch(const fvg_config* cfg, int device, const double* UL, const
         if (axis[k] < 0 || axis[k] > 2) return set_err(nullptr, FVG_EINVAL, "axis must be 0, 1 or 2");
     if (hipSetDevice(device) != hipSuccess) return set_err(nullptr, FVG_EHIP, "hipSetDevice failed");
     RiemannParams rs;
-    rs.eos.stiff = cfg->eos_type == FVG_EOS_STIFFENED;
-    rs.eos.gamma = cfg->gamma;
-    rs.eos.p_inf = rs.eos.stiff ? cfg->p_inf : 0.0;
+    rs.eos = make_eos(cfg->eos_type == FVG_EOS_STIFFENED, cfg->gamma, cfg->p_inf);
     rs.lowmach = cfg->riemann == FVG_LOWMACH_HLLC;
     rs.blend = cfg->shock_blend;
     double *dUL = nullptr, *dUR = nullptr, *dF = nullptr, *dS = nullptr;

@@ -13,6 +13,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 namespace fvg {
 
 constexpr double kEosEps = 1e-10;    // Core.hpp:169
@@ -34,20 +36,16 @@ __device__ __forceinline__ float dv(float a, float b) { return a * __builtin_amd
 __device__ __forceinline__ double sq(double a) { return sqrt(a); }
 __device__ __forceinline__ float sq(float a) { return __builtin_amdgcn_sqrtf(a); }
 
-// x / 6 correctly rounded in three operations, for x = 0 or 2^-960 <= |x| <= 2^905 (Markstein's correction step with
-// a = RN(1/6) = (1/6)(1 - 2^-54)): x a is within ulp(x/6)/2 of x/6, so q0 = RN(x a) is within 1 ulp, r = 6 q0 - x is
-// an integer multiple of 2 ulp(x/6) smaller than 3 of them and exact in one FMA, and q0 - r a equals
-// x/6 + (q0 - x/6) 2^-54 before its one rounding. x/6 = (M/3) 2^e for an integer significand M is either
-// representable or M/3 leaves a remainder of 1/3 or 2/3, which puts x/6 at least 1/6 ulp from every midpoint; an
-// error below 2^-54 ulp cannot cross one, so the result is the IEEE quotient. Zeros keep their sign (r = +0, and
-// -r a + q0 = q0). Below the range the quotient may be subnormal and a midpoint (x = 9 2^-1074 gives 2^-1074, the
-// division 2 2^-1074); above it, or for non-finite x, the FMA can overflow or give NaN: callers keep the IEEE
-// division there (range_fits_quot6).
+// x / 6 correctly rounded in two operations, for x = 0 or 2^-960 <= |x| <= 2^905: with 1/6 = a + b (a = RN(1/6) =
+// (1/6)(1 - 2^-54), so b = 2^-54 / 6, whose double is b to 2^-107), RN(x a + RN(x b)) rounds x/6 with an error below
+// 2^-105 |x/6|. x/6 = (M/3) 2^e for an integer significand M is either representable or M/3 leaves a remainder of 1/3
+// or 2/3, which puts x/6 at least 1/6 ulp from every midpoint, so the result is the IEEE quotient. Zeros keep their
+// sign. Below the range the quotient may be subnormal and a midpoint (x = 9 2^-1074 gives 2^-1074, the division
+// 2 2^-1074); above it, or for non-finite x, the FMA can overflow or give NaN: callers keep the IEEE division there
+// (range_fits_quot6).
 __host__ __device__ __forceinline__ double quot6(double x) {
-    constexpr double a = 1.0 / 6.0;
-    const double q0 = x * a;
-    const double r = __builtin_fma(q0, 6.0, -x);
-    return __builtin_fma(-r, a, q0);
+    constexpr double a = 1.0 / 6.0, b = 0x1p-54 / 6.0;
+    return __builtin_fma(x, a, x * b);
 }
 // v is 0 or 2^-900 <= |v| <= 2^900: the numerators of WENO5-Z's candidates (sums of 2, 7 and 11 times such values)
 // are then 0 or between 2^-952 and 2^905 in magnitude, inside the range of quot6. NaN is outside.
@@ -55,6 +53,85 @@ __host__ __device__ __forceinline__ bool range_fits_quot6(double v) {
     const double m = v < 0.0 ? -v : v;
     return (v == 0.0) | ((m >= 0x1p-900) & (m <= 0x1p+900));   // no short-circuit branches
 }
+// ---- FP64 operations whose operands are known to be in range (IR) ----
+// The IEEE division of the compiler scales its operands (two v_div_scale), ends in v_div_fmas / v_div_fixup and so
+// takes about 70 cycles of a SIMD per wavefront, the IEEE square root 85; the face kernels spend a third of their time
+// in them. When neither operand needs the scaling (denominator and its reciprocal normal, quotient normal or zero,
+// |numerator| >= 2^-969 or zero), scaling multiplies by one and the same reciprocal, Newton steps and correction
+// give the same bits without it: 57 cycles with the fixup (which keeps zeros, infinities and NaN as IEEE has them), 52
+// without it, 53 for the square root.
+// The kernels take these forms when every primitive that k_cells stored is zero or between 2^-400 and 2^100 in
+// magnitude (value_in_range; DevState::wide) and the configuration's constants are moderate (KP::ir). Then, with
+// WENO5-Z (eps at least 2^-42 of the stencil's mean square): differences are zero or at least 2^-453, the smoothness
+// indicators zero or at least 2^-908, tau zero or at least 2^-961, tau / (b + eps) at most 2^53, candidates zero or
+// at least 2^-458 and the last quotient at least 2^-570; van Leer's 2 a b is at least 2^-906. The Riemann solver
+// divides by densities and pressures of at least 1e-10 and by speed differences of at least 1e-14; its contact
+// speed, whose numerator may be any small number, keeps the IEEE division.
+__device__ __forceinline__ double rcp_refined(double b) {   // the compiler's reciprocal: two Newton steps
+    double r = __builtin_amdgcn_rcp(b);
+    r = __builtin_fma(r, __builtin_fma(-b, r, 1.0), r);
+    return __builtin_fma(r, __builtin_fma(-b, r, 1.0), r);
+}
+// a / b from r = rcp_refined(b): zeros of a keep their sign for b > 0
+__device__ __forceinline__ double quot_rcp(double a, double b, double r) {
+    const double q = a * r;
+    return __builtin_fma(-__builtin_fma(q, b, -a), r, q);
+}
+// a / b for b > 0 or a != 0, both finite
+template <bool IR> __device__ __forceinline__ double dvp(double a, double b) {
+    if constexpr (IR) return quot_rcp(a, b, rcp_refined(b));
+    else return a / b;
+}
+template <bool IR> __device__ __forceinline__ float dvp(float a, float b) { return dv(a, b); }
+// a / b, any zeros, infinities and NaN
+template <bool IR> __device__ __forceinline__ double dvx(double a, double b) {
+    if constexpr (IR) return __builtin_amdgcn_div_fixup(quot_rcp(a, b, rcp_refined(b)), b, a);
+    else return a / b;
+}
+template <bool IR> __device__ __forceinline__ float dvx(float a, float b) { return dv(a, b); }
+// the compiler's square root without its scaling of arguments below 2^-767 (zeros, infinities and NaN as IEEE has them)
+template <bool IR> __device__ __forceinline__ double sqx(double x) {
+    if constexpr (IR) {
+        const double y = __builtin_amdgcn_rsq(x);
+        double g = x * y, h = y * 0.5;
+        const double r = __builtin_fma(-h, g, 0.5);
+        g = __builtin_fma(g, r, g);
+        h = __builtin_fma(h, r, h);
+        g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+        g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+        return __builtin_amdgcn_class(x, 0x260) ? x : g;   // +-0 and +inf are their own roots
+    } else {
+        return sqrt(x);
+    }
+}
+template <bool IR> __device__ __forceinline__ float sqx(float x) { return sq(x); }
+// x / c for a constant c > 0 with inv = RN(1 / c): Markstein's correction as in quot6 (with a correctly rounded
+// reciprocal the corrected quotient is the IEEE one for every significand of c); FP32: the product
+template <bool IR> __host__ __device__ __forceinline__ double by_const(double x, double c, double inv) {
+    if constexpr (IR) {
+        const double q = x * inv;
+        return __builtin_fma(-__builtin_fma(q, c, -x), inv, q);
+    } else {
+        return x / c;
+    }
+}
+template <bool IR> __device__ __forceinline__ float by_const(float x, float c, double) { return dv(x, c); }
+// k b + c for k a power of two: the product is exact (short of overflow and underflow), so one FMA rounds as the two
+// operations do. EX<IR, T>: the operands are away from both ends (in-range FP64; FP32, whose error budget a last bit
+// of a subnormal does not touch).
+template <bool IR, typename T> constexpr bool EX = IR || std::is_same<T, float>::value;
+template <bool X> __device__ __forceinline__ double p2fma(double k, double b, double c) { return X ? __builtin_fma(k, b, c) : k * b + c; }
+template <bool X> __device__ __forceinline__ float p2fma(float k, float b, float c) { return __builtin_fmaf(k, b, c); }
+// smin / smax of finite values that are not zeros of opposite sign: one instruction instead of a compare and two selects
+template <bool IR> __device__ __forceinline__ double nmin(double a, double b) { return IR ? __builtin_fmin(a, b) : smin(a, b); }
+template <bool IR> __device__ __forceinline__ double nmax(double a, double b) { return IR ? __builtin_fmax(a, b) : smax(a, b); }
+template <bool IR> __device__ __forceinline__ float nmin(float a, float b) { return smin(a, b); }
+template <bool IR> __device__ __forceinline__ float nmax(float a, float b) { return smax(a, b); }
+__host__ __device__ __forceinline__ bool value_in_range(double v) {
+    const double m = v < 0.0 ? -v : v;
+    return (v == 0.0) | ((m >= 0x1p-400) & (m <= 0x1p+100));   // no short-circuit branches
+}
+
 // the absolute floor of the WENO regularisation: 1e-300 in FP64 (Schemes.cpp:331, 343); the smallest power of ten
 // above FLT_MIN in FP32, where 1e-300 would round to zero and 0/0 would reach the weights of an all-zero stencil
 template <typename T> __device__ __forceinline__ T weno_floor() { return T(1e-300); }
@@ -63,50 +140,51 @@ template <> __device__ __forceinline__ float weno_floor<float>() { return 1e-37f
 struct Eos {
     int stiff;
     double gamma, p_inf;
+    double inv_g1;   // 1 / (gamma - 1), correctly rounded
 };
+inline Eos make_eos(bool stiff, double gamma, double p_inf) { return Eos{stiff ? 1 : 0, gamma, stiff ? p_inf : 0.0, 1.0 / (gamma - 1.0)}; }
 
 // primitive [rho, u, v, p, w] -> conservative (Core.hpp:209-215)
-template <int NV, typename T>
+template <int NV, bool IR = false, typename T>
 __device__ __forceinline__ void p2c(const Eos& e, const T* W, T* U) {
     const T g = T(e.gamma);
     const T rho = W[0], u = W[1], v = W[2], p = W[3];
-    T ke;
+    const T en = by_const<IR>(!e.stiff ? p : p + g * T(e.p_inf), g - T(1.0), e.inv_g1);
+    T m2 = u * u + v * v;
     if constexpr (NV == 5) {
         const T w = W[4];
-        ke = T(0.5) * rho * (u * u + v * v + w * w);
+        m2 = m2 + w * w;
         U[4] = rho * w;
-    } else {
-        ke = T(0.5) * rho * (u * u + v * v);
     }
-    const T en = !e.stiff ? dv(p, g - T(1.0)) : dv(p + g * T(e.p_inf), g - T(1.0));
     U[0] = rho;
     U[1] = rho * u;
     U[2] = rho * v;
-    U[3] = en + ke;
+    if constexpr (EX<IR, T>) U[3] = p2fma<true>(T(0.5), rho * m2, en);   // en + (0.5 rho) m2
+    else U[3] = en + T(0.5) * rho * m2;
 }
 
 // conservative -> primitive with the floors of Core.hpp:219-228; *inv = 1 / rho
-template <int NV, typename T>
+template <int NV, bool IR = false, typename T>
 __device__ __forceinline__ void c2p(const Eos& e, const T* U, T* W, T* inv_out) {
     const T g = T(e.gamma);
-    const T rho = smax(U[0], T(kEosEps));
-    const T inv = dv(T(1.0), rho);
+    const T rho = nmax<IR>(U[0], T(kEosEps));
+    const T inv = dvx<IR>(T(1.0), rho);
     if (inv_out) *inv_out = inv;
     const T u = U[1] * inv, v = U[2] * inv;
-    T e_kin;
+    T m2 = u * u + v * v;
     if constexpr (NV == 5) {
         const T w = U[4] * inv;
-        e_kin = T(0.5) * rho * (u * u + v * v + w * w);
+        m2 = m2 + w * w;
         W[4] = w;
-    } else {
-        e_kin = T(0.5) * rho * (u * u + v * v);
     }
-    const T rho_e = U[3] - e_kin;
+    T rho_e;   // U[3] - (0.5 rho) m2
+    if constexpr (EX<IR, T>) rho_e = p2fma<true>(T(-0.5), rho * m2, U[3]);
+    else rho_e = U[3] - T(0.5) * rho * m2;
     const T p = !e.stiff ? (g - T(1.0)) * rho_e : (g - T(1.0)) * rho_e - g * T(e.p_inf);
     W[0] = rho;
     W[1] = u;
     W[2] = v;
-    W[3] = smax(p, T(kEosEps));
+    W[3] = nmax<IR>(p, T(kEosEps));
 }
 
 template <typename T>
@@ -114,10 +192,10 @@ __device__ __forceinline__ T sound_speed(const Eos& e, T p, T rho) {
     if (!e.stiff) return sq(dv(T(e.gamma) * smax(p, T(kEosEps)), smax(rho, T(kEosEps))));
     return sq(dv(T(e.gamma) * (p + T(e.p_inf)), smax(rho, T(kEosEps))));
 }
-template <typename T>
+template <bool IR = false, typename T>
 __device__ __forceinline__ T sound_speed_inv(const Eos& e, T p, T inv_rho) {
-    if (!e.stiff) return sq(T(e.gamma) * smax(p, T(kEosEps)) * inv_rho);
-    return sq(T(e.gamma) * (p + T(e.p_inf)) * inv_rho);
+    if (!e.stiff) return sqx<IR>(T(e.gamma) * nmax<IR>(p, T(kEosEps)) * inv_rho);
+    return sqx<IR>(T(e.gamma) * (p + T(e.p_inf)) * inv_rho);
 }
 
 template <int NV, typename T>
@@ -127,7 +205,7 @@ __device__ __forceinline__ void roundtrip(const Eos& e, T* U) {
     p2c<NV>(e, W, U);
 }
 
-template <typename T> __device__ __forceinline__ T safe_denom(T x) { return copysign(smax(fabs(x), T(kDenomEps)), x); }
+template <bool IR = false, typename T> __device__ __forceinline__ T safe_denom(T x) { return copysign(nmax<IR>(fabs(x), T(kDenomEps)), x); }
 
 struct RiemannParams {
     Eos eos;
@@ -137,67 +215,72 @@ struct RiemannParams {
 
 // HLLC with Einfeldt bounds, the contact speed of Toro (10.37) and the shock blend toward HLL
 // (Schemes.cpp:116-200). vel index a = 0, 1, 2 maps to W[1], W[2], W[4].
-template <int NV, typename T>
+// The flux of a face comes from one side of its contact: the side is picked first, by selecting its eleven or so
+// inputs, and only that side's flux, star state and two of its quotients are computed; the reference computes both
+// and picks the result. Which side its four successive conditions leave: the right one when S_R < 0 or
+// S_M < 0 <= S_R, else the left one, and zero when none of them holds (NaN speeds).
+template <int NV, bool IR = false, typename T>
 __device__ __forceinline__ void hllc_core(const RiemannParams& rs, const T* WL, const T* WR, const T* UL, const T* UR, T inv_L,
                                           T inv_R, T c_L, T c_R, int axis, T* F, T& smax_out) {
     const T rho_L = WL[0], p_L = WL[3];
     const T rho_R = WR[0], p_R = WR[3];
-    const T E_L = UL[3] * inv_L, E_R = UR[3] * inv_R;
-    const T Vn_L = WL[mom(axis)], Vn_R = WR[mom(axis)];
     const int mn = mom(axis);
-    T FL[NV], FR[NV];
-    FL[0] = rho_L * Vn_L;
-    FR[0] = rho_R * Vn_R;
-#pragma unroll
-    for (int a = 0; a < NV - 2; ++a) {
-        FL[mom(a)] = rho_L * WL[mom(a)] * Vn_L;
-        FR[mom(a)] = rho_R * WR[mom(a)] * Vn_R;
-    }
-    FL[mn] = FL[mn] + p_L;
-    FR[mn] = FR[mn] + p_R;
-    FL[3] = Vn_L * (rho_L * E_L + p_L);
-    FR[3] = Vn_R * (rho_R * E_R + p_R);
-    const T S_L = smin(Vn_L - c_L, Vn_R - c_R);
-    const T S_R = smax(Vn_L + c_L, Vn_R + c_R);
+    const T Vn_L = WL[mn], Vn_R = WR[mn];
+    const T S_L = nmin<IR>(Vn_L - c_L, Vn_R - c_R);
+    const T S_R = nmax<IR>(Vn_L + c_L, Vn_R + c_R);
     const T num = rho_R * Vn_R * (S_R - Vn_R) - rho_L * Vn_L * (S_L - Vn_L) + p_L - p_R;
     const T den = rho_R * (S_R - Vn_R) - rho_L * (S_L - Vn_L);
-    const T S_M = dv(num, safe_denom(den));
-    const T den_star_L = safe_denom(S_L - S_M);
-    const T den_star_R = safe_denom(S_R - S_M);
-    const T den_pL = safe_denom(S_L - Vn_L);
-    const T den_pR = safe_denom(S_R - Vn_R);
-    const T fL = dv(rho_L * (S_L - Vn_L), den_star_L);
-    const T fR = dv(rho_R * (S_R - Vn_R), den_star_R);
-    T UsL[NV], UsR[NV];
-    UsL[0] = fL;
-    UsR[0] = fR;
+    const T S_M = dv(num, safe_denom<IR>(den));
+    const bool right = (S_R < T(0)) | ((S_M < T(0)) & (S_R >= T(0)));
+    const bool star = right ? S_R >= T(0) : (S_L < T(0)) & (S_M >= T(0));
+    const bool none = !IR & !right & !star & !(S_L >= T(0));   // not with finite speeds
+    T W[NV], U[NV];
 #pragma unroll
-    for (int a = 0; a < NV - 2; ++a) {
-        UsL[mom(a)] = fL * (a == axis ? S_M : WL[mom(a)]);
-        UsR[mom(a)] = fR * (a == axis ? S_M : WR[mom(a)]);
+    for (int q = 0; q < NV; ++q) {
+        W[q] = right ? WR[q] : WL[q];
+        U[q] = right ? UR[q] : UL[q];
     }
-    UsL[3] = fL * (E_L + (S_M - Vn_L) * (S_M + dv(p_L, rho_L * den_pL)));
-    UsR[3] = fR * (E_R + (S_M - Vn_R) * (S_M + dv(p_R, rho_R * den_pR)));
+    const T S = right ? S_R : S_L;
+    const T rho = W[0], p = W[3], Vn = W[mn];
+    const T E = U[3] * (right ? inv_R : inv_L);
     T Fo[NV];
+    Fo[0] = rho * Vn;
 #pragma unroll
-    for (int q = 0; q < NV; ++q) Fo[q] = T(0);
-    if (S_L >= T(0))
+    for (int a = 0; a < NV - 2; ++a) Fo[mom(a)] = rho * W[mom(a)] * Vn;
+    Fo[mn] = Fo[mn] + p;
+    Fo[3] = Vn * (rho * E + p);
+    const T f = dvx<IR>(rho * (S - Vn), safe_denom<IR>(S - S_M));
+    T Us[NV];
+    Us[0] = f;
 #pragma unroll
-        for (int q = 0; q < NV; ++q) Fo[q] = FL[q];
-    if (S_L < T(0) && S_M >= T(0))
+    for (int a = 0; a < NV - 2; ++a) Us[mom(a)] = f * (a == axis ? S_M : W[mom(a)]);
+    Us[3] = f * (E + (S_M - Vn) * (S_M + dvx<IR>(p, rho * safe_denom<IR>(S - Vn))));
 #pragma unroll
-        for (int q = 0; q < NV; ++q) Fo[q] = FL[q] + S_L * (UsL[q] - UL[q]);
-    if (S_M < T(0) && S_R >= T(0))
+    for (int q = 0; q < NV; ++q) {
+        const T s = Fo[q] + S * (Us[q] - U[q]);
+        Fo[q] = star ? s : Fo[q];
+    }
+    if (none)
 #pragma unroll
-        for (int q = 0; q < NV; ++q) Fo[q] = FR[q] + S_R * (UsR[q] - UR[q]);
-    if (S_R < T(0))
-#pragma unroll
-        for (int q = 0; q < NV; ++q) Fo[q] = FR[q];
+        for (int q = 0; q < NV; ++q) Fo[q] = T(0);
     if (rs.blend > 0.0) {
         const T blend = T(rs.blend);
-        const T s = dv(fabs(p_R - p_L), smin(p_L, p_R));
+        const T s = dvx<IR>(fabs(p_R - p_L), nmin<IR>(p_L, p_R));
         if (s > blend) {
             const T phi = smin(dv(s - blend, blend), T(1.0));
+            const T E_L = UL[3] * inv_L, E_R = UR[3] * inv_R;
+            T FL[NV], FR[NV];
+            FL[0] = rho_L * Vn_L;
+            FR[0] = rho_R * Vn_R;
+#pragma unroll
+            for (int a = 0; a < NV - 2; ++a) {
+                FL[mom(a)] = rho_L * WL[mom(a)] * Vn_L;
+                FR[mom(a)] = rho_R * WR[mom(a)] * Vn_R;
+            }
+            FL[mn] = FL[mn] + p_L;
+            FR[mn] = FR[mn] + p_R;
+            FL[3] = Vn_L * (rho_L * E_L + p_L);
+            FR[3] = Vn_R * (rho_R * E_R + p_R);
             T Fh[NV];
             if (S_L >= T(0)) {
 #pragma unroll
@@ -214,102 +297,110 @@ __device__ __forceinline__ void hllc_core(const RiemannParams& rs, const T* WL, 
             for (int q = 0; q < NV; ++q) Fo[q] = (T(1.0) - phi) * Fo[q] + phi * Fh[q];
         }
     }
-    smax_out = smax(fabs(S_L), fabs(S_R));
+    smax_out = nmax<IR>(fabs(S_L), fabs(S_R));
 #pragma unroll
     for (int q = 0; q < NV; ++q) F[q] = Fo[q];
 }
 
-// RiemannSolver::face_flux (Schemes.cpp:108-113, 202-229)
-template <int NV, typename T>
-__device__ __forceinline__ void face_flux(const RiemannParams& rs, const T* UL, const T* UR, int axis, T* F, T& sm) {
-    T WL[NV], WR[NV], inv_L, inv_R;
-    c2p<NV>(rs.eos, UL, WL, &inv_L);
-    c2p<NV>(rs.eos, UR, WR, &inv_R);
-    if (!rs.lowmach) {
-        hllc_core<NV>(rs, WL, WR, UL, UR, inv_L, inv_R, sound_speed_inv(rs.eos, WL[3], inv_L), sound_speed_inv(rs.eos, WR[3], inv_R),
-                      axis, F, sm);
-        return;
-    }
-    const T c_L = sound_speed_inv(rs.eos, WL[3], inv_L);
-    const T c_R = sound_speed_inv(rs.eos, WR[3], inv_R);
-    T ML2, MR2;
-    if constexpr (NV == 5) {
-        ML2 = WL[1] * WL[1] + WL[2] * WL[2] + WL[4] * WL[4];
-        MR2 = WR[1] * WR[1] + WR[2] * WR[2] + WR[4] * WR[4];
-    } else {
-        ML2 = WL[1] * WL[1] + WL[2] * WL[2];
-        MR2 = WR[1] * WR[1] + WR[2] * WR[2];
-    }
-    const T M_L = dv(sq(ML2), c_L + T(kMachEps));
-    const T M_R = dv(sq(MR2), c_R + T(kMachEps));
-    const T z = smin(smax(smax(M_L, M_R), T(1e-4)), T(1.0));
+// RiemannSolver::face_flux (Schemes.cpp:108-113, 202-229). One hllc_core for both solvers (its code is inlined once):
+// the low-Mach variant blends the velocities first.
+template <int NV, bool IR = false, typename T>
+__device__ __forceinline__ void face_flux(const RiemannParams& rs, const T* UL0, const T* UR0, int axis, T* F, T& sm) {
+    T WL[NV], WR[NV], UL[NV], UR[NV], inv_L, inv_R;
 #pragma unroll
-    for (int a = 0; a < NV - 2; ++a) {
-        const int m = mom(a);
-        const T avg = T(0.5) * (WL[m] + WR[m]);
-        const T half = T(0.5) * (WL[m] - WR[m]);
-        WL[m] = avg + z * half;
-        WR[m] = avg - z * half;
+    for (int q = 0; q < NV; ++q) {
+        UL[q] = UL0[q];
+        UR[q] = UR0[q];
     }
-    T UsL[NV], UsR[NV];
-    p2c<NV>(rs.eos, WL, UsL);
-    p2c<NV>(rs.eos, WR, UsR);
-    hllc_core<NV>(rs, WL, WR, UsL, UsR, inv_L, inv_R, c_L, c_R, axis, F, sm);
+    c2p<NV, IR>(rs.eos, UL, WL, &inv_L);
+    c2p<NV, IR>(rs.eos, UR, WR, &inv_R);
+    const T c_L = sound_speed_inv<IR>(rs.eos, WL[3], inv_L);
+    const T c_R = sound_speed_inv<IR>(rs.eos, WR[3], inv_R);
+    if (rs.lowmach) {
+        T ML2 = WL[1] * WL[1] + WL[2] * WL[2], MR2 = WR[1] * WR[1] + WR[2] * WR[2];
+        if constexpr (NV == 5) {
+            ML2 = ML2 + WL[4] * WL[4];
+            MR2 = MR2 + WR[4] * WR[4];
+        }
+        const T M_L = dvx<IR>(sq(ML2), c_L + T(kMachEps));
+        const T M_R = dvx<IR>(sq(MR2), c_R + T(kMachEps));
+        const T z = smin(smax(smax(M_L, M_R), T(1e-4)), T(1.0));
+#pragma unroll
+        for (int a = 0; a < NV - 2; ++a) {
+            const int m = mom(a);
+            const T avg = T(0.5) * (WL[m] + WR[m]);
+            const T half = T(0.5) * (WL[m] - WR[m]);
+            WL[m] = avg + z * half;
+            WR[m] = avg - z * half;
+        }
+        p2c<NV, IR>(rs.eos, WL, UL);
+        p2c<NV, IR>(rs.eos, WR, UR);
+    }
+    hllc_core<NV, IR>(rs, WL, WR, UL, UR, inv_L, inv_R, c_L, c_R, axis, F, sm);
 }
 
 // ---- limiters (Schemes.hpp:90-117) and WENO-Z (Schemes.cpp:323-353) ----
 template <typename T> __device__ __forceinline__ T sgn(T x) { return (x > T(0)) ? T(1) : ((x < T(0)) ? T(-1) : T(0)); }
 
-template <typename T>
+template <bool IR = false, typename T>
 __device__ __forceinline__ T limiter(int l, T a, T b) {
     switch (l) {
     case 0: return T(0.5) * (sgn(a) + sgn(b)) * smin(fabs(a), fabs(b));
     case 1: {
         const T ab = a * b;
-        return (ab > T(0)) ? dv(T(2.0) * ab, a + b) : T(0.0);
+        return (ab > T(0)) ? dvp<IR>(T(2.0) * ab, a + b) : T(0.0);
     }
     case 2:
         if (!(a * b > T(0))) return T(0.0);
         return smin(smin(T(2.0) * fabs(a), T(0.5) * fabs(a + b)), T(2.0) * fabs(b)) * sgn(a);
     default:
         if (!(a * b > T(0))) return T(0.0);
-        return fmin(fmin(T(2.0) * fabs(a), dv(fabs(T(2.0) * a + b), T(3.0))), T(2.0) * fabs(b)) * sgn(a);
+        return fmin(fmin(T(2.0) * fabs(a), by_const<IR>(fabs(T(2.0) * a + b), T(3.0), 1.0 / 3.0)), T(2.0) * fabs(b)) * sgn(a);
     }
 }
 
-template <typename T>
+template <typename T, bool IR = false>
 __device__ __forceinline__ T weno3z(T c0, T c1, T c2, T eps_rel) {
     const T eps = eps_rel * (c0 * c0 + c1 * c1 + c2 * c2) * T(1.0 / 3.0) + weno_floor<T>();
     const T v0 = T(-0.5) * c0 + T(1.5) * c1, v1 = T(0.5) * c1 + T(0.5) * c2;
     const T b0 = (c1 - c0) * (c1 - c0), b1 = (c2 - c1) * (c2 - c1);
     const T tau = fabs(b0 - b1);
-    const T a0 = T(1.0 / 3.0) * (T(1.0) + dv(tau, b0 + eps)), a1 = T(2.0 / 3.0) * (T(1.0) + dv(tau, b1 + eps));
-    return dv(a0 * v0 + a1 * v1, a0 + a1);
+    const T a0 = T(1.0 / 3.0) * (T(1.0) + dvp<IR>(tau, b0 + eps)), a1 = T(2.0 / 3.0) * (T(1.0) + dvp<IR>(tau, b1 + eps));
+    return dvp<IR>(a0 * v0 + a1 * v1, a0 + a1);
 }
 
-// the candidates' quotients by 6: the IEEE division, or quot6 (the same bits) when every stencil value is known to be
-// in range_fits_quot6 (Q6)
-template <bool Q6, typename T> __device__ __forceinline__ T by6(T x) {
-    if constexpr (Q6 && std::is_same<T, double>::value) return quot6(x);
+// the candidates' quotients by 6: the IEEE division, or quot6 (the same bits) in range
+template <bool IR, typename T> __device__ __forceinline__ T by6(T x) {
+    if constexpr (IR && std::is_same<T, double>::value) return quot6(x);
     else return dv(x, T(6.0));
 }
 
-template <typename T, bool Q6 = false>
+// Products by 2, 4 and 1/4 are exact, so they share an FMA with the sum they enter (p2fma: the same bits): 188
+// operations and 8 reciprocals for the two values of a face and variable.
+template <typename T, bool IR = false>
 __device__ __forceinline__ T weno5z(T c0, T c1, T c2, T c3, T c4, T eps_rel) {
+    constexpr bool X = EX<IR, T>;
     const T eps = eps_rel * (c0 * c0 + c1 * c1 + c2 * c2 + c3 * c3 + c4 * c4) * T(0.2) + weno_floor<T>();
-    const T p0 = by6<Q6>(T(2.0) * c0 - T(7.0) * c1 + T(11.0) * c2);
-    const T p1 = by6<Q6>(-c1 + T(5.0) * c2 + T(2.0) * c3);
-    const T p2 = by6<Q6>(T(2.0) * c2 + T(5.0) * c3 - c4);
-    const T s0 = c0 - T(2.0) * c1 + c2, t0 = c0 - T(4.0) * c1 + T(3.0) * c2;
-    const T s1 = c1 - T(2.0) * c2 + c3, t1 = c1 - c3;
-    const T s2 = c2 - T(2.0) * c3 + c4, t2 = T(3.0) * c2 - T(4.0) * c3 + c4;
-    const T b0 = T(13.0 / 12.0) * s0 * s0 + T(0.25) * t0 * t0;
-    const T b1 = T(13.0 / 12.0) * s1 * s1 + T(0.25) * t1 * t1;
-    const T b2 = T(13.0 / 12.0) * s2 * s2 + T(0.25) * t2 * t2;
+    const T p0 = by6<IR>(p2fma<X>(T(2.0), c0, -(T(7.0) * c1)) + T(11.0) * c2);
+    const T p1 = by6<IR>(p2fma<X>(T(2.0), c3, T(5.0) * c2 - c1));
+    const T p2 = by6<IR>(p2fma<X>(T(2.0), c2, T(5.0) * c3) - c4);
+    const T s0 = p2fma<X>(T(-2.0), c1, c0) + c2, t0 = p2fma<X>(T(-4.0), c1, c0) + T(3.0) * c2;
+    const T s1 = p2fma<X>(T(-2.0), c2, c1) + c3, t1 = c1 - c3;
+    const T s2 = p2fma<X>(T(-2.0), c3, c2) + c4, t2 = p2fma<X>(T(-4.0), c3, T(3.0) * c2) + c4;
+    T b0, b1, b2;
+    if constexpr (X) {
+        b0 = p2fma<X>(T(0.25), t0 * t0, T(13.0 / 12.0) * s0 * s0);
+        b1 = p2fma<X>(T(0.25), t1 * t1, T(13.0 / 12.0) * s1 * s1);
+        b2 = p2fma<X>(T(0.25), t2 * t2, T(13.0 / 12.0) * s2 * s2);
+    } else {
+        b0 = T(13.0 / 12.0) * s0 * s0 + T(0.25) * t0 * t0;
+        b1 = T(13.0 / 12.0) * s1 * s1 + T(0.25) * t1 * t1;
+        b2 = T(13.0 / 12.0) * s2 * s2 + T(0.25) * t2 * t2;
+    }
     const T tau = fabs(b0 - b2);
-    const T a0 = T(0.1) * (T(1.0) + dv(tau, b0 + eps)), a1 = T(0.6) * (T(1.0) + dv(tau, b1 + eps)),
-            a2 = T(0.3) * (T(1.0) + dv(tau, b2 + eps));
-    return dv(a0 * p0 + a1 * p1 + a2 * p2, a0 + a1 + a2);
+    const T a0 = T(0.1) * (T(1.0) + dvp<IR>(tau, b0 + eps)), a1 = T(0.6) * (T(1.0) + dvp<IR>(tau, b1 + eps)),
+            a2 = T(0.3) * (T(1.0) + dvp<IR>(tau, b2 + eps));
+    return dvp<IR>(a0 * p0 + a1 * p1 + a2 * p2, a0 + a1 + a2);
 }
 
 // ---- convective ghost state (Boundaries.cpp:106-153) ----

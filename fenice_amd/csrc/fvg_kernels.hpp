@@ -23,11 +23,11 @@ struct DevState {
     long long reverted;
     int done, diverged, steps, max_steps;
     double ut[6];   // mass-flow inlet velocity per side of the current residual (k_massflow)
-    // nonzero: a value k_cells stored for the residual's WENO5-Z stencils (a primitive of the FP64 planes or, with
-    // the fourth-order quadrature, a value of the padded conservative planes) is outside range_fits_quot6, so the
-    // kernels take the IEEE division for WENO5-Z's quotients by 6. k_cells only sets it; k_update (the end of every
-    // residual of the separate passes) and k_control (after a residual's faces or between steps) clear it, never
-    // between a k_cells and the kernels that read its planes.
+    // nonzero: a value k_cells stored for the residual's stencils (a primitive of the FP64 planes or, with the
+    // fourth-order quadrature, a value of the padded conservative planes) is outside value_in_range, so the kernels
+    // take the IEEE divisions and roots. k_cells only sets it; k_update (the end of every residual of the separate
+    // passes) and k_control (after a residual's faces or between steps) clear it, never between a k_cells and the
+    // kernels that read its planes.
     int wide;
 };
 
@@ -43,6 +43,8 @@ struct KP {
     int nx, ny, nz, is3d;
     long long nc;
     double dx, dy, dz;
+    double inv_h[3];              // 1 / dx, 1 / dy, 1 / dz, correctly rounded
+    int ir;                       // the configuration's constants allow the in-range operations (fvg_device.hpp)
     double Ax, Ay, Az, inv_vol;   // face areas and 1 / volume (2-D: dy, dx, -, 1 / (dx dy))
     // numerics
     RiemannParams rs;

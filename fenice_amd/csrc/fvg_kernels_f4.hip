@@ -32,8 +32,8 @@ template <int NV> __device__ __forceinline__ double q4_m2(const double* u) {
 template <int NV> __device__ __forceinline__ bool q4_positive(double g1, double gp, const double* u) {
     return u[0] > 0.0 && g1 * (u[3] * u[0] - 0.5 * q4_m2<NV>(u)) > gp * u[0];
 }
-template <int NV> __device__ __forceinline__ double q4_pressure(double g1, double gp, const double* u) {
-    return g1 * (u[3] - 0.5 * q4_m2<NV>(u) / u[0]) - gp;
+template <int NV, bool IR = false> __device__ __forceinline__ double q4_pressure(double g1, double gp, const double* u) {
+    return g1 * (u[3] - dvx<IR>(0.5 * q4_m2<NV>(u), u[0])) - gp;
 }
 
 // the face one lattice step s (-1, +1) from face f along transverse axis t, -1 when there is none
@@ -65,8 +65,8 @@ __device__ __forceinline__ void q4_load(const double* planes, long long n, long 
 }   // namespace
 
 // R: the reconstruction, 2 WENO3-Z (four cells t-2 .. t+1), 3 WENO5-Z (six cells t-3 .. t+2)
-// Q6: WENO5-Z's quotients by 6 in three operations (quot6; every value of Wc in range_fits_quot6, the same bits)
-template <int NV, int D, int R, bool Q6>
+// IR: the operands are in range (every value of Wc in value_in_range)
+template <int NV, int D, int R, bool IR>
 __device__ __forceinline__ void k4_states_face(const KP& p, long long f) {
     int i, j, k, t;
     face_coords<NV, D>(p, f, i, j, k, t);
@@ -88,14 +88,14 @@ __device__ __forceinline__ void k4_states_face(const KP& p, long long f) {
         if constexpr (R == 3) {
 #pragma unroll
             for (int q = 0; q < NV; ++q) {
-                ul[q] = weno5z<double, Q6>(c[0][q], c[1][q], c[2][q], c[3][q], c[4][q], we);
-                ur[q] = weno5z<double, Q6>(c[5][q], c[4][q], c[3][q], c[2][q], c[1][q], we);
+                ul[q] = weno5z<double, IR>(c[0][q], c[1][q], c[2][q], c[3][q], c[4][q], we);
+                ur[q] = weno5z<double, IR>(c[5][q], c[4][q], c[3][q], c[2][q], c[1][q], we);
             }
         } else {
 #pragma unroll
             for (int q = 0; q < NV; ++q) {
-                ul[q] = weno3z(c[0][q], c[1][q], c[2][q], we);
-                ur[q] = weno3z(c[3][q], c[2][q], c[1][q], we);
+                ul[q] = weno3z<double, IR>(c[0][q], c[1][q], c[2][q], we);
+                ur[q] = weno3z<double, IR>(c[3][q], c[2][q], c[1][q], we);
             }
         }
         // admissible: positive, and the density and pressure inside the range of the stencil cells widened by the
@@ -105,7 +105,7 @@ __device__ __forceinline__ void k4_states_face(const KP& p, long long f) {
             double rlo = 1e300, rhi = -1e300, plo = 1e300, phi = -1e300;
 #pragma unroll
             for (int s = 0; s < NS; ++s) {
-                const double pc = q4_pressure<NV>(g1, gp, c[s]);
+                const double pc = q4_pressure<NV, IR>(g1, gp, c[s]);
                 rlo = smin(rlo, c[s][0]);
                 rhi = smax(rhi, c[s][0]);
                 plo = smin(plo, pc);
@@ -116,7 +116,7 @@ __device__ __forceinline__ void k4_states_face(const KP& p, long long f) {
             rhi += rw;
             plo -= pw;
             phi += pw;
-            const double pl = q4_pressure<NV>(g1, gp, ul), pr = q4_pressure<NV>(g1, gp, ur);
+            const double pl = q4_pressure<NV, IR>(g1, gp, ul), pr = q4_pressure<NV, IR>(g1, gp, ur);
             ok = ul[0] >= rlo && ul[0] <= rhi && pl >= plo && pl <= phi;
             ok = ok && ur[0] >= rlo && ur[0] <= rhi && pr >= plo && pr <= phi;
         }
@@ -137,7 +137,7 @@ __device__ __forceinline__ void k4_states_face(const KP& p, long long f) {
     // good: a full stencil, positive states, the shock sensor quiet (Schemes.cpp:1987-2005)
     bool good = upgrade && q4_positive<NV>(g1, gp, ul) && q4_positive<NV>(g1, gp, ur);
     if (good && p.rs.blend > 0.0) {
-        const double pL = q4_pressure<NV>(g1, gp, ul), pR = q4_pressure<NV>(g1, gp, ur);
+        const double pL = q4_pressure<NV, IR>(g1, gp, ul), pR = q4_pressure<NV, IR>(g1, gp, ur);
         if (fabs(pR - pL) > p.rs.blend * smin(pL, pR)) good = false;
     }
 #pragma unroll
@@ -152,12 +152,8 @@ template <int NV, int D, int R>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k4_states(KP p) {
     const long long f = xcd_block() * blockDim.x + threadIdx.x;
     if (f >= p.nfa[D] || p.st->done) return;
-    if constexpr (R == 3) {   // uniform over the launch: quot6 unless a value of Wc is outside its range
-        if (__builtin_amdgcn_readfirstlane(p.st->wide) == 0) k4_states_face<NV, D, R, true>(p, f);
-        else k4_states_face<NV, D, R, false>(p, f);
-    } else {
-        k4_states_face<NV, D, R, false>(p, f);
-    }
+    if (in_range(p)) k4_states_face<NV, D, R, true>(p, f);
+    else k4_states_face<NV, D, R, false>(p, f);
 }
 
 template <int NV, int D>

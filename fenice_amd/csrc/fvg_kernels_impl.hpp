@@ -36,6 +36,11 @@ __device__ __forceinline__ int halo_of(const KP& p, int s) {
 __device__ __forceinline__ int vper_of(const KP& p, int a) { return a == 0 ? p.vper[0] : (a == 1 ? p.vper[1] : p.vper[2]); }
 __device__ __forceinline__ int wrap_of(const KP& p, int a) { return a == 0 ? p.wrap[0] : (a == 1 ? p.wrap[1] : p.wrap[2]); }
 
+__device__ __forceinline__ double inv_hstep(const KP& p, int d) { return d == 0 ? p.inv_h[0] : (d == 1 ? p.inv_h[1] : p.inv_h[2]); }
+// whether the residual's FP64 operands are in range (fvg_device.hpp): uniform over the launch, since k_cells finished
+// before it and nothing else sets the flag
+__device__ __forceinline__ bool in_range(const KP& p) { return p.ir != 0 && __builtin_amdgcn_readfirstlane(p.st->wide) == 0; }
+
 template <int NV> __device__ __forceinline__ void load_cons(const KP& p, long long c, double* u) {
 #pragma unroll
     for (int q = 0; q < NV; ++q) u[q] = p.U[q * p.nc + c];
@@ -241,8 +246,10 @@ __device__ __forceinline__ void outside_first_order(const KP& p, int d, int side
 }
 
 // MUSCL face values of one variable (Schemes.cpp:627-635): wl from (c0, c1, c2), wr from (c1, c2, c3)
-__device__ __forceinline__ double muscl_wl(int lim, double c0, double c1, double c2) { return c1 + 0.5 * limiter(lim, c1 - c0, c2 - c1); }
-__device__ __forceinline__ double muscl_wr(int lim, double c1, double c2, double c3) { return c2 - 0.5 * limiter(lim, c3 - c2, c2 - c1); }
+template <bool IR = false>
+__device__ __forceinline__ double muscl_wl(int lim, double c0, double c1, double c2) { return p2fma<IR>(0.5, limiter<IR>(lim, c1 - c0, c2 - c1), c1); }
+template <bool IR = false>
+__device__ __forceinline__ double muscl_wr(int lim, double c1, double c2, double c3) { return p2fma<IR>(-0.5, limiter<IR>(lim, c3 - c2, c2 - c1), c2); }
 
 // ------------------------------------------------------------------------------------------------------------
 // Viscous padded state (Boundaries.cpp:379-700): cell coordinates may lie one cell outside the domain.
@@ -415,7 +422,7 @@ __device__ __forceinline__ double cell_gradients_f32(const KP& p, long long c, i
 // beyond the other side; with a ghost slab (boundary_order = 2) it writes the primitives of its ghost state at its
 // mirror position; a side with neither has its halo layers copy the edge cell. u: the cell's state, w: its
 // primitives as stored. CONS: the planes Wo hold the conservative state (w = u, and a ghost is stored as it is).
-// wide: set when a ghost value stored is outside range_fits_quot6 (the copies of w are the caller's to check).
+// wide: set when a ghost value stored is outside value_in_range (the copies of w are the caller's to check).
 template <int NV, typename T, bool CONS = false>
 __device__ __forceinline__ void push_halo(const KP& p, T* Wo, int i, int j, int k, const double* u, const T* w, bool& wide) {
     auto put = [&](int d, int t, const T* v) {
@@ -435,7 +442,7 @@ __device__ __forceinline__ void push_halo(const KP& p, T* Wo, int i, int j, int 
         }
         if constexpr (std::is_same<T, double>::value) {   // FP64 primitives, or the conservative ghosts
 #pragma unroll
-            for (int q = 0; q < NV; ++q) wide |= !range_fits_quot6(v[q]);
+            for (int q = 0; q < NV; ++q) wide |= !value_in_range(v[q]);
         }
         put(d, t, v);
     };
@@ -467,7 +474,7 @@ __global__ __launch_bounds__(256) void k_cells(KP p) {
     const int i = rb.i, j = rb.j, k = rb.k;
     const long long c = ((long long)k * p.ny + j) * p.nx + i;
     double local = 0.0;
-    bool wide = false;   // a primitive stored in the FP64 planes is outside range_fits_quot6
+    bool wide = false;   // a primitive stored in the FP64 planes is outside value_in_range
     if (i < p.nx && !p.st->done) {
         const long long pc = pidx(p, i, j, k);
         if constexpr (std::is_same<T, float>::value) {
@@ -492,7 +499,7 @@ __global__ __launch_bounds__(256) void k_cells(KP p) {
 #pragma unroll
                 for (int q = 0; q < NV; ++q) {
                     p.Wc[q * p.npad + pc] = u[q];
-                    wide |= !range_fits_quot6(u[q]);
+                    wide |= !value_in_range(u[q]);
                 }
                 push_halo<NV, double, true>(p, p.Wc, i, j, k, u, u, wide);
             }
@@ -501,7 +508,7 @@ __global__ __launch_bounds__(256) void k_cells(KP p) {
 #pragma unroll
                 for (int q = 0; q < NV; ++q) {
                     Wo[q * p.npad + pc] = w[q];
-                    wide |= !range_fits_quot6(w[q]);
+                    wide |= !value_in_range(w[q]);
                 }
                 push_halo<NV, double>(p, Wo, i, j, k, u, w, wide);
             }
@@ -543,10 +550,10 @@ __global__ __launch_bounds__(256) void k_nrbc(KP p) {
 // k_hancock: the limited states of every cell advanced by half a step with the cell's own flux difference;
 // an inadmissible state stays as it was (Schemes.cpp:2135-2199, 2907-2933, 2989-3016).
 // ------------------------------------------------------------------------------------------------------------
-template <int NV>
+template <int NV, bool IR>
 __device__ __forceinline__ void euler_flux_axis(const Eos& e, const double* U, int a, double* F) {
     double W[NV];
-    c2p<NV>(e, U, W, (double*)nullptr);
+    c2p<NV, IR>(e, U, W, (double*)nullptr);
     const double un = W[mom(a)], pr = W[3];
     F[0] = U[0] * un;
     F[1] = U[1] * un + (a == 0 ? pr : 0.0);
@@ -555,12 +562,11 @@ __device__ __forceinline__ void euler_flux_axis(const Eos& e, const double* U, i
     if constexpr (NV == 5) F[4] = U[4] * un + (a == 2 ? pr : 0.0);
 }
 
-template <int NV>
-__global__ __launch_bounds__(256) void k_hancock(KP p) {
+template <int NV, bool IR>
+__device__ __forceinline__ unsigned long long hancock_cell(const KP& p, long long c) {
     constexpr int ND = NV - 2, NS = 2 * ND;
-    const long long c = xcd_block() * blockDim.x + threadIdx.x;
     unsigned long long reverted = 0;
-    if (c < p.nc && !p.st->done) {
+    {
         const int i = (int)(c % p.nx);
         const long long r = c / p.nx;
         const int j = (int)(r % p.ny), k = (int)(r / p.ny);
@@ -578,14 +584,14 @@ __global__ __launch_bounds__(256) void k_hancock(KP p) {
             double lo[NV], hi[NV], uc[NV];
 #pragma unroll
             for (int q = 0; q < NV; ++q) {
-                lo[q] = muscl_wr(p.lim, wm[q], w0[q], wp[q]);
-                hi[q] = muscl_wl(p.lim, wm[q], w0[q], wp[q]);
+                lo[q] = muscl_wr<IR>(p.lim, wm[q], w0[q], wp[q]);
+                hi[q] = muscl_wl<IR>(p.lim, wm[q], w0[q], wp[q]);
             }
             load_cons<NV>(p, c, uc);
             roundtrip<NV>(p.rs.eos, uc);   // the first-order state of a side face without a halo
             double a0[NV], a1[NV];
-            p2c<NV>(p.rs.eos, lo, a0);
-            p2c<NV>(p.rs.eos, hi, a1);
+            p2c<NV, IR>(p.rs.eos, lo, a0);
+            p2c<NV, IR>(p.rs.eos, hi, a1);
 #pragma unroll
             for (int q = 0; q < NV; ++q) {
                 st[2 * d][q] = up_lo ? a0[q] : uc[q];
@@ -596,7 +602,7 @@ __global__ __launch_bounds__(256) void k_hancock(KP p) {
         const double hx = half_dt / p.dx, hy = half_dt / p.dy;
         double f[NS][NV];
 #pragma unroll
-        for (int s = 0; s < NS; ++s) euler_flux_axis<NV>(p.rs.eos, st[s], s / 2, f[s]);
+        for (int s = 0; s < NS; ++s) euler_flux_axis<NV, IR>(p.rs.eos, st[s], s / 2, f[s]);
         double dd[NV];
 #pragma unroll
         for (int q = 0; q < NV; ++q) {
@@ -620,6 +626,13 @@ __global__ __launch_bounds__(256) void k_hancock(KP p) {
             for (int q = 0; q < NV; ++q) p.HS[((long long)s * NV + q) * p.nc + c] = ok ? nw[q] : st[s][q];
         }
     }
+    return reverted;
+}
+template <int NV>
+__global__ __launch_bounds__(256) void k_hancock(KP p) {
+    const long long c = xcd_block() * blockDim.x + threadIdx.x;
+    if (c >= p.nc || p.st->done) return;
+    const unsigned long long reverted = in_range(p) ? hancock_cell<NV, true>(p, c) : hancock_cell<NV, false>(p, c);
     if (reverted) atomicAdd((unsigned long long*)&p.st->reverted, reverted);
 }
 
@@ -653,7 +666,8 @@ __device__ __forceinline__ T cross_term(const KP& p, bool phys, int i, int j, in
     return T(0.5) * (Gp[xL] + Gp[xR]);
 }
 
-template <int NV, int D, typename T>
+// PER: both sides of the axis are periodic and its halo wraps, so the padded primitives hold both cells of every face.
+template <int NV, int D, typename T, bool IR, bool PER>
 __device__ __forceinline__ void viscous_face(const KP& p, int i, int j, int k, int t, int n, T* out) {
     constexpr int ND = NV - 2;
     const bool lo = t == 0, hi = t == n;
@@ -661,7 +675,7 @@ __device__ __forceinline__ void viscous_face(const KP& p, int i, int j, int k, i
     T vL[ND], vR[ND], TL, TR;
     {
         T w[NV];
-        if (lo) {
+        if (!PER && lo) {
             double wd[NV];
             visc_pad_prim<NV>(p, D == 0 ? -1 : i, D == 1 ? -1 : j, D == 2 ? -1 : k, wd);
 #pragma unroll
@@ -671,8 +685,8 @@ __device__ __forceinline__ void viscous_face(const KP& p, int i, int j, int k, i
         }
 #pragma unroll
         for (int a = 0; a < ND; ++a) vL[a] = w[mom(a)];
-        TL = dv(w[3], w[0]);
-        if (hi) {
+        TL = dvp<IR>(w[3], w[0]);
+        if (!PER && hi) {
             double wd[NV];
             visc_pad_prim<NV>(p, D == 0 ? n : i, D == 1 ? n : j, D == 2 ? n : k, wd);
 #pragma unroll
@@ -682,19 +696,20 @@ __device__ __forceinline__ void viscous_face(const KP& p, int i, int j, int k, i
         }
 #pragma unroll
         for (int a = 0; a < ND; ++a) vR[a] = w[mom(a)];
-        TR = dv(w[3], w[0]);
+        TR = dvp<IR>(w[3], w[0]);
     }
-    const long long xL = (lo && vper_of(p, D)) ? cidx_d(p, D, i, j, k, n - 1) : cL;
-    const long long xR = (hi && vper_of(p, D)) ? cidx_d(p, D, i, j, k, 0) : cR;
-    const bool phys = p.bo2 && !vper_of(p, D) && (lo || hi);
+    const long long xL = (lo && (PER || vper_of(p, D))) ? cidx_d(p, D, i, j, k, n - 1) : cL;
+    const long long xR = (hi && (PER || vper_of(p, D))) ? cidx_d(p, D, i, j, k, 0) : cR;
+    const bool phys = !PER && p.bo2 && !vper_of(p, D) && (lo || hi);
     const T h = T(hstep(p, D));
+    const double inv_h = inv_hstep(p, D);
     const int tg = lo ? -1 : n, tc = lo ? 0 : n - 1;   // the ghost and the cell layer of a boundary face
 #define CROSS(a, b) cross_term<NV, D, T>(p, phys, i, j, k, tg, tc, xL, xR, a, b)
     const T mu = T(p.mu), kc = T(p.k_cond), MD = T(MU_DIAG), MO = T(MU_OFF), half = T(0.5);
     if constexpr (ND == 2) {
         const T u_f = half * (vL[0] + vR[0]), v_f = half * (vL[1] + vR[1]);
         if constexpr (D == 0) {
-            const T du_dx = dv(vR[0] - vL[0], h), dv_dx = dv(vR[1] - vL[1], h), dT_dx = dv(TR - TL, h);
+            const T du_dx = by_const<IR>(vR[0] - vL[0], h, inv_h), dv_dx = by_const<IR>(vR[1] - vL[1], h, inv_h), dT_dx = by_const<IR>(TR - TL, h, inv_h);
             const T du_dy = CROSS(0, 1), dv_dy = CROSS(1, 1);
             const T tau_xx = mu * (MD * du_dx - MO * dv_dy);
             const T tau_xy = mu * (du_dy + dv_dx);
@@ -704,7 +719,7 @@ __device__ __forceinline__ void viscous_face(const KP& p, int i, int j, int k, i
             out[1] = tau_xy * ar;
             out[2] = (u_f * tau_xx + v_f * tau_xy - q_x) * ar;
         } else {
-            const T dv_dy = dv(vR[1] - vL[1], h), du_dy = dv(vR[0] - vL[0], h), dT_dy = dv(TR - TL, h);
+            const T dv_dy = by_const<IR>(vR[1] - vL[1], h, inv_h), du_dy = by_const<IR>(vR[0] - vL[0], h, inv_h), dT_dy = by_const<IR>(TR - TL, h, inv_h);
             const T du_dx = CROSS(0, 0), dv_dx = CROSS(1, 0);
             const T tau_yy = mu * (MD * dv_dy - MO * du_dx);
             const T tau_yx = mu * (du_dy + dv_dx);
@@ -718,10 +733,10 @@ __device__ __forceinline__ void viscous_face(const KP& p, int i, int j, int k, i
         T Gn[3], vf[3];
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
-            Gn[a] = dv(vR[a] - vL[a], h);
+            Gn[a] = by_const<IR>(vR[a] - vL[a], h, inv_h);
             vf[a] = half * (vL[a] + vR[a]);
         }
-        const T dT = dv(TR - TL, h);
+        const T dT = by_const<IR>(TR - TL, h, inv_h);
         T tau[3];
         if constexpr (D == 0) {
             const T g01 = CROSS(0, 1), g11 = CROSS(1, 1), g22 = CROSS(2, 2), g02 = CROSS(0, 2);
@@ -783,7 +798,7 @@ __device__ __forceinline__ double area_of(const KP& p, int d) { return d == 0 ? 
 // The fluxes of face f normal to D. FP64: the convective flux and (with viscosity) the viscous flux in their own
 // planes, combined by k_update in the reference's order. FP32 fluxes: one combined plane set, convective flux
 // times the face area minus the viscous flux, so the update reads each face once.
-template <int NV, int D, typename T>
+template <int NV, int D, typename T, bool IR = false, bool PER = false>
 __device__ __forceinline__ void store_face(const KP& p, long long f, int i, int j, int k, int t, int n, const T* F) {
     T* Fc = (T*)p.Fc[D];
     const long long ps = p.nfa[D];
@@ -794,7 +809,7 @@ __device__ __forceinline__ void store_face(const KP& p, long long f, int i, int 
         for (int q = 0; q < NV; ++q) G[q] = F[q] * A;
         if (p.viscous) {
             float v[NV - 1];
-            viscous_face<NV, D, float>(p, i, j, k, t, n, v);
+            viscous_face<NV, D, float, IR, PER>(p, i, j, k, t, n, v);
 #pragma unroll
             for (int q = 1; q < NV; ++q) G[q] -= v[q - 1];
         }
@@ -805,7 +820,7 @@ __device__ __forceinline__ void store_face(const KP& p, long long f, int i, int 
         for (int q = 0; q < NV; ++q) Fc[q * ps + f] = F[q];
         if (p.viscous) {
             T v[NV - 1];
-            viscous_face<NV, D, T>(p, i, j, k, t, n, v);
+            viscous_face<NV, D, T, IR, PER>(p, i, j, k, t, n, v);
             T* Fv = (T*)p.Fv[D];
 #pragma unroll
             for (int q = 0; q < NV - 1; ++q) Fv[q * ps + f] = v[q];
@@ -815,9 +830,9 @@ __device__ __forceinline__ void store_face(const KP& p, long long f, int i, int 
 
 // The two states of face (i, j, k) normal to D (t its coordinate along D, n the cells along D) that the Riemann
 // solver takes: reconstructed from the padded primitives, first-order at a side without a halo, or the
-// MUSCL-Hancock predicted states (Schemes.cpp:389-749, 2934-2988). Q6: WENO5-Z divides by 6 with quot6 (every
-// stencil value in range_fits_quot6; the same bits).
-template <int NV, int D, int MODE, typename T, bool Q6 = false>
+// MUSCL-Hancock predicted states (Schemes.cpp:389-749, 2934-2988). IR: the operands are in range (in_range). RECON: the
+// reconstruction (enum fvg_recon; 0: KP::recon). PER: the axis has a periodic halo, so every face is reconstructed.
+template <int NV, int D, int MODE, typename T, bool IR = false, int RECON = 0, bool PER = false>
 __device__ __forceinline__ void face_states(const KP& p, int i, int j, int k, int t, int n, T* UL, T* UR) {
     const bool lo = t == 0, hi = t == n;
     // the cells left and right of the face (their coordinate along D is t - 1 and t)
@@ -831,39 +846,40 @@ __device__ __forceinline__ void face_states(const KP& p, int i, int j, int k, in
         to_t<NV>(ul, UL);
         to_t<NV>(ur, UR);
     } else if constexpr (MODE == MODE_PLAIN) {
-        const bool upgrade = (t > 0 && t < n) || (lo && halo_of(p, 2 * D)) || (hi && halo_of(p, 2 * D + 1));
+        const int recon = RECON ? RECON : p.recon;
+        const bool upgrade = PER || (t > 0 && t < n) || (lo && halo_of(p, 2 * D)) || (hi && halo_of(p, 2 * D + 1));
         if (upgrade) {
             T wl[NV], wr[NV];
             const T we = T(p.weno_eps);
-            if (p.recon == 3) {   // WENO5-Z on six cells t-3 .. t+2
+            if (recon == 3) {   // WENO5-Z on six cells t-3 .. t+2
                 T c[6][NV];
 #pragma unroll
                 for (int s = 0; s < 6; ++s) stencil_prim<NV, T>(p, D, i, j, k, t - 3 + s, c[s]);
 #pragma unroll
                 for (int q = 0; q < NV; ++q) {
-                    wl[q] = weno5z<T, Q6>(c[0][q], c[1][q], c[2][q], c[3][q], c[4][q], we);
-                    wr[q] = weno5z<T, Q6>(c[5][q], c[4][q], c[3][q], c[2][q], c[1][q], we);
+                    wl[q] = weno5z<T, IR>(c[0][q], c[1][q], c[2][q], c[3][q], c[4][q], we);
+                    wr[q] = weno5z<T, IR>(c[5][q], c[4][q], c[3][q], c[2][q], c[1][q], we);
                 }
             } else {   // four cells t-2 .. t+1
                 T c[4][NV];
 #pragma unroll
                 for (int s = 0; s < 4; ++s) stencil_prim<NV, T>(p, D, i, j, k, t - 2 + s, c[s]);
-                if (p.recon == 2) {
+                if (recon == 2) {
 #pragma unroll
                     for (int q = 0; q < NV; ++q) {
-                        wl[q] = weno3z(c[0][q], c[1][q], c[2][q], we);
-                        wr[q] = weno3z(c[3][q], c[2][q], c[1][q], we);
+                        wl[q] = weno3z<T, IR>(c[0][q], c[1][q], c[2][q], we);
+                        wr[q] = weno3z<T, IR>(c[3][q], c[2][q], c[1][q], we);
                     }
                 } else {
 #pragma unroll
                     for (int q = 0; q < NV; ++q) {
-                        wl[q] = muscl_wl(p.lim, c[0][q], c[1][q], c[2][q]);
-                        wr[q] = muscl_wr(p.lim, c[1][q], c[2][q], c[3][q]);
+                        wl[q] = muscl_wl<IR>(p.lim, c[0][q], c[1][q], c[2][q]);
+                        wr[q] = muscl_wr<IR>(p.lim, c[1][q], c[2][q], c[3][q]);
                     }
                 }
             }
-            p2c<NV>(p.rs.eos, wl, UL);
-            p2c<NV>(p.rs.eos, wr, UR);
+            p2c<NV, IR>(p.rs.eos, wl, UL);
+            p2c<NV, IR>(p.rs.eos, wr, UR);
         } else {
             double ul[NV], ur[NV];
             if (!lo) load_cons<NV>(p, cidx(p, il, jl, kl), ul);
@@ -874,6 +890,13 @@ __device__ __forceinline__ void face_states(const KP& p, int i, int j, int k, in
             roundtrip<NV>(p.rs.eos, ur);
             to_t<NV>(ul, UL);
             to_t<NV>(ur, UR);
+        }
+    } else if constexpr (PER) {   // MUSCL-Hancock, periodic axis: the seam faces take the cells of both ends
+        const long long cl = cidx_d(p, D, i, j, k, lo ? n - 1 : t - 1), cr = cidx_d(p, D, i, j, k, hi ? 0 : t);
+#pragma unroll
+        for (int q = 0; q < NV; ++q) {
+            UL[q] = p.HS[((long long)(2 * D + 1) * NV + q) * p.nc + cl];
+            UR[q] = p.HS[((long long)(2 * D) * NV + q) * p.nc + cr];
         }
     } else {   // MUSCL-Hancock: the predicted states of the cells on both sides (Schemes.cpp:2934-2988)
         if (!lo) {
@@ -902,7 +925,20 @@ __device__ __forceinline__ void face_coords(const KP& p, long long f, int& i, in
     t = coord(D, i, j, k);
 }
 
-template <int NV, int D, int MODE, typename T = double>
+// The flux of face f normal to D, stored; its wave speed
+template <int NV, int D, int MODE, typename T, bool IR, int RECON, bool PER>
+__device__ __forceinline__ double face_body(const KP& p, long long f, int i, int j, int k, int t, int n) {
+    T UL[NV], UR[NV], F[NV], sm;
+    face_states<NV, D, MODE, T, IR, RECON, PER>(p, i, j, k, t, n, UL, UR);
+    face_flux<NV, IR>(p.rs, UL, UR, D, F, sm);
+    store_face<NV, D, T, IR, PER>(p, f, i, j, k, t, n, F);
+    return double(sm);
+}
+
+// RECON and PER as in face_states (the host launches the variant of the configuration's reconstruction and of the
+// axis' sides): one reconstruction's code, and no boundary code on a periodic axis, leaves a face kernel a tenth of
+// the instructions of one that carries them all, without spills.
+template <int NV, int D, int MODE, int RECON, bool PER, typename T = double>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_faces(KP p) {
     const int ni = p.nx + (D == 0), nj = p.ny + (D == 1), nk = p.nz + (D == 2);
     const long long nf = (long long)ni * nj * nk;
@@ -914,18 +950,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
         int i = rb.i, j = rb.j, k = rb.k, t = rb.k;
         if (D != 2) face_coords<NV, D>(p, f, i, j, k, t);
         const int n = ncell(p, D);
-        T UL[NV], UR[NV];
-        if constexpr (MODE == MODE_PLAIN && std::is_same<T, double>::value) {
-            // uniform over the launch: quot6 unless k_cells stored a primitive outside its range
-            if (__builtin_amdgcn_readfirstlane(p.st->wide) == 0) face_states<NV, D, MODE, T, true>(p, i, j, k, t, n, UL, UR);
-            else face_states<NV, D, MODE, T, false>(p, i, j, k, t, n, UL, UR);
-        } else {
-            face_states<NV, D, MODE, T>(p, i, j, k, t, n, UL, UR);
-        }
-        T F[NV], sm;
-        face_flux<NV>(p.rs, UL, UR, D, F, sm);
-        if (double(sm) > local) local = double(sm);
-        store_face<NV, D, T>(p, f, i, j, k, t, n, F);
+        double sm;
+        if (std::is_same<T, double>::value && in_range(p))
+            sm = face_body<NV, D, MODE, T, std::is_same<T, double>::value, RECON, PER>(p, f, i, j, k, t, n);
+        else
+            sm = face_body<NV, D, MODE, T, false, RECON, PER>(p, f, i, j, k, t, n);
+        if (sm > local) local = sm;
     }
     block_max_slot(p, local, SPD_CONV);
 }
@@ -949,11 +979,11 @@ __device__ __forceinline__ bool face_upgrade(const KP& p, int t) {
 template <int NV, int D> __device__ __forceinline__ unsigned char* kept_of(const KP& p) {
     return D == 0 ? p.ind_kept[0] : (D == 1 ? p.ind_kept[1] : p.ind_kept[2]);
 }
-// Q6: the troubled faces' WENO5-Z divides by 6 with quot6 (every stencil value in range_fits_quot6; the same bits)
-template <int NV, int D, int USE, typename T, bool Q6 = false>
+// IR: the operands are in range (in_range)
+template <int NV, int D, int USE, typename T, bool IR = false, bool PER = false>
 __device__ __forceinline__ void learned_face(const KP& p, bool active, long long f, int i, int j, int k, int t, int n, T* F,
                                              T& sm) {
-    const bool upgrade = active && face_upgrade<NV, D>(p, t);
+    const bool upgrade = active && (PER || face_upgrade<NV, D>(p, t));
     // once the audit has switched the indicator off every face takes WENO5-Z and the network is not run (the switch
     // changes only between steps; read once per wavefront, so the branch is uniform)
     const bool off = __builtin_amdgcn_readfirstlane(p.ind->off) != 0;
@@ -1005,12 +1035,12 @@ __device__ __forceinline__ void learned_face(const KP& p, bool active, long long
         } else {
 #pragma unroll
             for (int q = 0; q < NV; ++q) {
-                wl[q] = weno5z<T, Q6>(c[0][q], c[1][q], c[2][q], c[3][q], c[4][q], we);
-                wr[q] = weno5z<T, Q6>(c[5][q], c[4][q], c[3][q], c[2][q], c[1][q], we);
+                wl[q] = weno5z<T, IR>(c[0][q], c[1][q], c[2][q], c[3][q], c[4][q], we);
+                wr[q] = weno5z<T, IR>(c[5][q], c[4][q], c[3][q], c[2][q], c[1][q], we);
             }
         }
-        p2c<NV>(p.rs.eos, wl, UL);
-        p2c<NV>(p.rs.eos, wr, UR);
+        p2c<NV, IR>(p.rs.eos, wl, UL);
+        p2c<NV, IR>(p.rs.eos, wr, UR);
     } else {
         double ul[NV], ur[NV];
         if (!lo) load_cons<NV>(p, cidx(p, il, jl, kl), ul);
@@ -1022,10 +1052,19 @@ __device__ __forceinline__ void learned_face(const KP& p, bool active, long long
         to_t<NV>(ul, UL);
         to_t<NV>(ur, UR);
     }
-    face_flux<NV>(p.rs, UL, UR, D, F, sm);
+    face_flux<NV, IR>(p.rs, UL, UR, D, F, sm);
 }
 
-template <int NV, int D, int USE, typename T>
+template <int NV, int D, int USE, typename T, bool IR, bool PER>
+__device__ __forceinline__ double learned_body(const KP& p, bool active, long long f, int i, int j, int k, int t, int n) {
+    T F[NV], sm = T(0);
+    learned_face<NV, D, USE, T, IR, PER>(p, active, f, i, j, k, t, n, F, sm);
+    if (!active) return 0.0;
+    store_face<NV, D, T, IR, PER>(p, f, i, j, k, t, n, F);
+    return double(sm);
+}
+
+template <int NV, int D, int USE, bool PER, typename T>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_faces_learned(KP p) {
     if (p.st->done) return;   // uniform: the whole grid leaves
     const int ni = p.nx + (D == 0), nj = p.ny + (D == 1), nk = p.nz + (D == 2);
@@ -1043,17 +1082,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
         face_coords<NV, D>(p, f, i, j, k, t);
     }
     const int n = ncell(p, D);
-    T F[NV], sm = T(0);
-    // uniform over the launch: quot6 for FP64 unless k_cells stored a primitive outside its range
-    if (std::is_same<T, double>::value && __builtin_amdgcn_readfirstlane(p.st->wide) == 0)
-        learned_face<NV, D, USE, T, std::is_same<T, double>::value>(p, active, f, i, j, k, t, n, F, sm);
-    else
-        learned_face<NV, D, USE, T>(p, active, f, i, j, k, t, n, F, sm);
     double local = 0.0;
-    if (active) {
-        if (double(sm) > local) local = double(sm);
-        store_face<NV, D, T>(p, f, i, j, k, t, n, F);
-    }
+    double sm;
+    if (std::is_same<T, double>::value && in_range(p))
+        sm = learned_body<NV, D, USE, T, std::is_same<T, double>::value, PER>(p, active, f, i, j, k, t, n);
+    else
+        sm = learned_body<NV, D, USE, T, false, PER>(p, active, f, i, j, k, t, n);
+    if (sm > local) local = sm;
     block_max_slot(p, local, SPD_CONV);
 }
 
@@ -1241,17 +1276,18 @@ __device__ __forceinline__ void face_all(const KP& p, bool active, long long f, 
     } else {
         if (!active) return;
         T UL[NV], UR[NV];
-        if constexpr (MODE == MODE_PLAIN && std::is_same<T, double>::value) {
-            if (__builtin_amdgcn_readfirstlane(p.st->wide) == 0) face_states<NV, D, MODE, T, true>(p, i, j, k, t, n, UL, UR);
-            else face_states<NV, D, MODE, T, false>(p, i, j, k, t, n, UL, UR);
+        if (std::is_same<T, double>::value && in_range(p)) {
+            constexpr bool IR = std::is_same<T, double>::value;
+            face_states<NV, D, MODE, T, IR>(p, i, j, k, t, n, UL, UR);
+            face_flux<NV, IR>(p.rs, UL, UR, D, Fc, sm);
         } else {
             face_states<NV, D, MODE, T>(p, i, j, k, t, n, UL, UR);
+            face_flux<NV>(p.rs, UL, UR, D, Fc, sm);
         }
-        face_flux<NV>(p.rs, UL, UR, D, Fc, sm);
     }
     if (!active) return;
     if (double(sm) > local) local = double(sm);
-    if (p.viscous) viscous_face<NV, D, T>(p, i, j, k, t, n, Fv);
+    if (p.viscous) viscous_face<NV, D, T, false, false>(p, i, j, k, t, n, Fv);
     if constexpr (std::is_same<T, float>::value) {   // the combined flux of store_face
         const float A = float(area_of(p, D));
 #pragma unroll
