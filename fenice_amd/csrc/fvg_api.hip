@@ -17,6 +17,7 @@
 
 #include "../../include/fvg.h"
 #include "fvg_host.hpp"
+#include "fvg_transfer.hpp"
 
 namespace fvg {
 template <int NV, typename T> __global__ void k_cells(KP);
@@ -76,6 +77,7 @@ struct fvg_ctx {
     DevState* st = nullptr;
     unsigned long long* spd = nullptr;   // wave-speed slots (KP::spd)
     DevState* st_host = nullptr;   // pinned mirror for the read-back
+    HostCopy copy;                 // pinned staging of uploads and downloads
     KP base{};
     bool lagged_positive = false;
     std::string err;
@@ -613,6 +615,7 @@ void free_ctx(fvg_ctx* c) {
         if (b) hipFree(b);
     if (c->st) hipFree(c->st);
     if (c->st_host) hipHostFree(c->st_host);
+    c->copy.release();
     for (auto& r : c->recs) {
         hipEventDestroy(r.a);
         hipEventDestroy(r.b);
@@ -970,28 +973,23 @@ int fvg_destroy(fvg_ctx* c) {
     return FVG_OK;
 }
 
+// the planes of a Field's components (rho*w of a 2-D field has none: it is +0)
+static unsigned field_map(const fvg_ctx* c) { return c->NV == 5 ? plane_map(0, 1, 2, 3, 4) : plane_map(0, 1, 2, 3); }
+
 int fvg_upload(fvg_ctx* c, const double* U, size_t ncells, int ncomp) {
     if (!c || !U) return set_err(c, FVG_EINVAL, "null argument");
     if ((long long)ncells != c->nc) return set_err(c, FVG_EINVAL, "ncells does not match the mesh");
     if (ncomp != 5 && !(ncomp == 4 && c->NV == 4)) return set_err(c, FVG_EINVAL, "ncomp must be 5 (or 4 on a 2-D mesh)");
     HIPCHK(c, hipSetDevice(c->device));
-    std::vector<double> soa((size_t)c->NV * c->nc);
-    for (long long x = 0; x < c->nc; ++x)
-        for (int q = 0; q < c->NV; ++q) soa[(size_t)q * c->nc + x] = U[(size_t)x * ncomp + q];
-    HIPCHK(c, hipMemcpyAsync(c->U, soa.data(), soa.size() * sizeof(double), hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    return FVG_OK;
+    std::string what;
+    const hipError_t e = c->copy.to_device(c->device, c->stream, U, c->nc, ncomp, c->U, c->nc, field_map(c), what);
+    return e == hipSuccess ? FVG_OK : set_err(c, FVG_EHIP, what + ": " + hipGetErrorString(e));
 }
 
 static int download_planes(fvg_ctx* c, const double* src, double* U, int ncomp) {
-    std::vector<double> soa((size_t)c->NV * c->nc);
-    HIPCHK(c, hipMemcpyAsync(soa.data(), src, soa.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    for (long long x = 0; x < c->nc; ++x) {
-        for (int q = 0; q < c->NV; ++q) U[(size_t)x * ncomp + q] = soa[(size_t)q * c->nc + x];
-        if (c->NV == 4 && ncomp == 5) U[(size_t)x * 5 + 4] = 0.0;   // rho*w of a 2-D field
-    }
-    return FVG_OK;
+    std::string what;
+    const hipError_t e = c->copy.to_host(c->device, c->stream, src, c->nc, U, c->nc, ncomp, field_map(c), what);
+    return e == hipSuccess ? FVG_OK : set_err(c, FVG_EHIP, what + ": " + hipGetErrorString(e));
 }
 
 int fvg_download(fvg_ctx* c, double* U, size_t ncells, int ncomp) {

@@ -25,6 +25,7 @@
 #include <vector>
 
 #include "fvg_host.hpp"
+#include "fvg_transfer.hpp"
 
 namespace fvg {
 
@@ -811,6 +812,26 @@ __device__ void run_instance2(const BP2& b, int id, int r, int m, TeamSync* ts, 
     __syncthreads();
 }
 
+// The largest initial wave speed |v| + c of each instance (one workgroup each; the estimate that orders the launch).
+// NP planes: (rho, rho u, E) or (rho, rho u, rho v, E); the cells of instance i from inst[i].c0 to the next one's.
+template <int NP, typename I>
+__global__ __launch_bounds__(256) void k_initial_speed(const double* __restrict__ U, long long nc, const I* __restrict__ inst, int ninst, double g,
+                                                       double pinf, double* __restrict__ speed) {
+    __shared__ double red[4];
+    const int i = blockIdx.x;
+    const long long c1 = i + 1 < ninst ? inst[i + 1].c0 : nc;
+    double s = 0.0;
+    for (long long c = inst[i].c0 + threadIdx.x; c < c1; c += 256) {
+        const double rho = smax(U[c], kEosEps), u = U[nc + c] / rho, v = NP == 4 ? U[(NP - 2) * nc + c] / rho : 0.0;
+        const double p = (g - 1.0) * (U[(NP - 1) * nc + c] - 0.5 * rho * (u * u + v * v)) - (pinf != 0.0 ? g * pinf : 0.0);
+        const double c2 = g * (smax(p, kEosEps) + pinf) / rho;
+        const double a = sqrt(u * u + v * v) + sqrt(smax(c2, 0.0));
+        if (isfinite(a) && a > s) s = a;
+    }
+    s = bmax_all<256>(s, red);
+    if (threadIdx.x == 0) speed[i] = s;
+}
+
 // as k_ensemble: workgroups [0, team_wgs) run the teams' instances, then every workgroup takes queued instances;
 // without a queue, workgroup k runs instance order[k] alone
 template <int BS, int RECON>
@@ -875,6 +896,8 @@ struct fvg_batch {
     int* d_order = nullptr;
     BOut* d_out = nullptr;
     double *U = nullptr, *Ut = nullptr, *W = nullptr, *F = nullptr, *Usave = nullptr;
+    double* d_speed = nullptr;   // largest initial wave speed per instance
+    HostCopy copy;               // pinned staging of uploads and downloads
     BP base{};
     int block = 256;
     bool uploaded = false;
@@ -913,6 +936,8 @@ void free_batch(fvg_batch* b) {
     hipFree(b->d_inst2);
     hipFree(b->d_order);
     hipFree(b->d_out);
+    hipFree(b->d_speed);
+    b->copy.release();
     hipFree(b->U);
     hipFree(b->Ut);
     hipFree(b->W);
@@ -1290,7 +1315,7 @@ int fvg_batch_create(const fvg_config* cfg_in, int ninst, const int* ncells, int
     if (hipMalloc(&b->U, cb) != hipSuccess || hipMalloc(&b->Ut, cb) != hipSuccess || hipMalloc(&b->W, cb) != hipSuccess ||
         hipMalloc(&b->Usave, cb) != hipSuccess || hipMalloc(&b->F, fb) != hipSuccess ||
         hipMalloc(&b->d_inst, sizeof(BInst) * ninst) != hipSuccess || hipMalloc(&b->d_order, sizeof(int) * ninst) != hipSuccess ||
-        hipMalloc(&b->d_out, sizeof(BOut) * ninst) != hipSuccess || hipMalloc(&b->d_teams, sizeof(BTeam) * ninst) != hipSuccess ||
+        hipMalloc(&b->d_speed, sizeof(double) * ninst) != hipSuccess || hipMalloc(&b->d_out, sizeof(BOut) * ninst) != hipSuccess || hipMalloc(&b->d_teams, sizeof(BTeam) * ninst) != hipSuccess ||
         hipMalloc(&b->d_queue, sizeof(int) * ninst) != hipSuccess || hipMalloc(&b->d_qnext, sizeof(unsigned)) != hipSuccess ||
         hipMalloc(&b->d_sync, sizeof(TeamSync) * ninst) != hipSuccess)
         return fail(FVG_ENOMEM, "hipMalloc of the ensemble buffers");
@@ -1401,7 +1426,7 @@ int fvg_batch_create_2d(const fvg_config* cfg_in, int ninst, const int* nx, cons
     if (hipMalloc(&b->U, cb) != hipSuccess || hipMalloc(&b->Ut, cb) != hipSuccess || hipMalloc(&b->W, cb) != hipSuccess ||
         hipMalloc(&b->Usave, cb) != hipSuccess || hipMalloc(&b->F, fb) != hipSuccess ||
         hipMalloc(&b->d_inst2, sizeof(BInst2) * ninst) != hipSuccess || hipMalloc(&b->d_order, sizeof(int) * ninst) != hipSuccess ||
-        hipMalloc(&b->d_out, sizeof(BOut) * ninst) != hipSuccess || hipMalloc(&b->d_teams, sizeof(BTeam) * ninst) != hipSuccess ||
+        hipMalloc(&b->d_speed, sizeof(double) * ninst) != hipSuccess || hipMalloc(&b->d_out, sizeof(BOut) * ninst) != hipSuccess || hipMalloc(&b->d_teams, sizeof(BTeam) * ninst) != hipSuccess ||
         hipMalloc(&b->d_queue, sizeof(int) * ninst) != hipSuccess || hipMalloc(&b->d_qnext, sizeof(unsigned)) != hipSuccess ||
         hipMalloc(&b->d_sync, sizeof(TeamSync) * ninst) != hipSuccess)
         return fail(FVG_ENOMEM, "hipMalloc of the ensemble buffers");
@@ -1437,42 +1462,37 @@ int fvg_batch_create_2d(const fvg_config* cfg_in, int ninst, const int* nx, cons
     return FVG_OK;
 }
 
+// the planes of the host components: (rho, rho u, E), with rho v = +0 from the fourth component on, or
+// (rho, rho u, rho v, E) of 2-D instances
+static unsigned batch_map(const fvg_batch* b, int ncomp) {
+    if (b->dim == 2) return plane_map(0, 1, 2, 3);
+    return ncomp == 3 ? plane_map(0, 1, 2) : plane_map(0, 1, kNoPlane, 2);
+}
+
 int fvg_batch_upload(fvg_batch* b, const double* U, long long ncells, int ncomp) {
     if (!b || !U) return bset(b, FVG_EINVAL, "null argument");
     if (ncells != b->nc) return bset(b, FVG_EINVAL, "cell count differs from the ensemble's total");
     if (b->dim == 2 ? (ncomp != 4 && ncomp != 5) : (ncomp != 3 && ncomp != 4 && ncomp != 5))
         return bset(b, FVG_EINVAL, b->dim == 2 ? "ncomp must be 4 or 5" : "ncomp must be 3, 4 or 5");
-    // the planes ((rho, rho u, E), or (rho, rho u, rho v, E) for 2-D instances); the estimated cost of each instance
-    // (cells x the cells along its longer axis x the largest initial wave speed) orders the workgroups, longest first
-    const int np = b->nplanes, e = ncomp == 3 ? 2 : 3;
-    std::vector<double> h((size_t)np * b->nc);
+    BCHK(b, hipSetDevice(b->device));
+    std::string what;
+    hipError_t e = b->copy.to_device(b->device, b->stream, U, b->nc, ncomp, b->U, b->nc, batch_map(b, ncomp), what);
+    if (e != hipSuccess) return bset(b, FVG_EHIP, what + ": " + hipGetErrorString(e));
+    // the estimated cost of each instance (cells x the cells along its longer axis x the largest initial wave speed)
+    // orders the workgroups, longest first
     const double g = b->cfg.gamma, pinf = b->cfg.eos_type == FVG_EOS_STIFFENED ? b->cfg.p_inf : 0.0;
+    if (b->dim == 2) hipLaunchKernelGGL((k_initial_speed<4, BInst2>), dim3(b->ninst), dim3(256), 0, b->stream, b->U, b->nc, b->d_inst2, b->ninst, g, pinf, b->d_speed);
+    else hipLaunchKernelGGL((k_initial_speed<3, BInst>), dim3(b->ninst), dim3(256), 0, b->stream, b->U, b->nc, b->d_inst, b->ninst, g, pinf, b->d_speed);
+    BCHK(b, hipGetLastError());
     std::vector<double> cost(b->ninst);
-    for (int i = 0; i < b->ninst; ++i) {
-        const long long c0 = b->dim == 2 ? b->inst2[i].c0 : b->inst[i].c0;
-        const int nc_i = b->n[i];
-        const int lmax = b->dim == 2 ? std::max(b->inst2[i].nx, b->inst2[i].ny) : nc_i;
-        double smax0 = 0.0;
-        for (int k = 0; k < nc_i; ++k) {
-            const long long c = c0 + k;
-            const double* s = U + (size_t)ncomp * c;
-            h[c] = s[0];
-            h[b->nc + c] = s[1];
-            if (np == 4) h[2 * b->nc + c] = s[2];
-            h[(np - 1) * b->nc + c] = s[e];
-            const double rho = std::max(s[0], 1e-10), u = s[1] / rho, v = np == 4 ? s[2] / rho : 0.0;
-            const double p = (g - 1.0) * (s[e] - 0.5 * rho * (u * u + v * v)) - (pinf != 0.0 ? g * pinf : 0.0);
-            const double c2 = g * (std::max(p, 1e-10) + pinf) / rho;
-            const double sp = std::sqrt(u * u + v * v) + std::sqrt(std::max(c2, 0.0));
-            if (std::isfinite(sp) && sp > smax0) smax0 = sp;
-        }
-        cost[i] = (double)nc_i * lmax * (smax0 + 1e-3);
-    }
+    BCHK(b, hipMemcpyAsync(cost.data(), b->d_speed, sizeof(double) * b->ninst, hipMemcpyDeviceToHost, b->stream));
+    BCHK(b, hipStreamSynchronize(b->stream));
+    for (int i = 0; i < b->ninst; ++i)
+        cost[i] = (double)b->n[i] * (b->dim == 2 ? std::max(b->inst2[i].nx, b->inst2[i].ny) : b->n[i]) * (cost[i] + 1e-3);
     std::stable_sort(b->order.begin(), b->order.end(), [&](int a, int c) { return cost[a] > cost[c]; });
     b->cost = cost;
-    BCHK(b, hipSetDevice(b->device));
-    BCHK(b, hipMemcpy(b->U, h.data(), sizeof(double) * h.size(), hipMemcpyHostToDevice));
-    BCHK(b, hipMemcpy(b->d_order, b->order.data(), sizeof(int) * b->ninst, hipMemcpyHostToDevice));
+    BCHK(b, hipMemcpyAsync(b->d_order, b->order.data(), sizeof(int) * b->ninst, hipMemcpyHostToDevice, b->stream));
+    BCHK(b, hipStreamSynchronize(b->stream));
     b->uploaded = true;
     return FVG_OK;
 }
@@ -1482,26 +1502,10 @@ int fvg_batch_download(fvg_batch* b, double* U, long long ncells, int ncomp) {
     if (ncells != b->nc) return bset(b, FVG_EINVAL, "cell count differs from the ensemble's total");
     if (b->dim == 2 ? (ncomp != 4 && ncomp != 5) : (ncomp != 3 && ncomp != 4 && ncomp != 5))
         return bset(b, FVG_EINVAL, b->dim == 2 ? "ncomp must be 4 or 5" : "ncomp must be 3, 4 or 5");
-    std::vector<double> h((size_t)b->nplanes * b->nc);
     BCHK(b, hipSetDevice(b->device));
-    BCHK(b, hipMemcpy(h.data(), b->U, sizeof(double) * h.size(), hipMemcpyDeviceToHost));
-    for (long long c = 0; c < b->nc; ++c) {
-        double* s = U + (size_t)ncomp * c;
-        s[0] = h[c];
-        s[1] = h[b->nc + c];
-        if (b->nplanes == 4) {
-            s[2] = h[2 * b->nc + c];
-            s[3] = h[3 * b->nc + c];
-            if (ncomp == 5) s[4] = 0.0;
-        } else if (ncomp == 3) {
-            s[2] = h[2 * b->nc + c];
-        } else {
-            s[2] = 0.0;
-            s[3] = h[2 * b->nc + c];
-            if (ncomp == 5) s[4] = 0.0;
-        }
-    }
-    return FVG_OK;
+    std::string what;
+    const hipError_t e = b->copy.to_host(b->device, b->stream, b->U, b->nc, U, b->nc, ncomp, batch_map(b, ncomp), what);
+    return e == hipSuccess ? FVG_OK : bset(b, FVG_EHIP, what + ": " + hipGetErrorString(e));
 }
 
 int fvg_batch_run(fvg_batch* b, double t_end, double dt_max, int max_steps, double* t, int* steps, int* diverged, double* s_last,
