@@ -20,7 +20,8 @@
 #include "fvg_transfer.hpp"
 
 namespace fvg {
-template <int NV, typename T> __global__ void k_cells(KP);
+template <int NV, bool PER, typename T> __global__ void k_cells(KP);
+template <typename T> __global__ void k_cells_march(KP);
 template <int NV> __global__ void k_hancock(KP);
 template <int NV, int D, int MODE, int RECON, bool PER, typename T> __global__ void k_faces(KP);
 template <int NV, int UPD, typename T> __global__ void k_update(KP, const double*, const double*, double*);
@@ -215,6 +216,16 @@ int enqueue_massflow(fvg_ctx* c, const KP& p) {
     return rc;
 }
 
+// the primitives and gradients, in the variant of the mesh's sides
+template <int NV, typename T>
+int launch_cells(fvg_ctx* c, const KP& p) {
+    const bool per = p.wrap[0] && p.wrap[1] && (NV == 4 || p.wrap[2]);
+    return launch(c, FAM_CELLS, [&] {
+        if (p.kseg > 1) hipLaunchKernelGGL((k_cells_march<T>), dim3(row_grid(c, (p.nz + p.kseg - 1) / p.kseg)), dim3(cells_block(c)), 0, c->stream, p);
+        else if (per) hipLaunchKernelGGL((k_cells<NV, true, T>), dim3(cells_grid(c)), dim3(cells_block(c)), 0, c->stream, p);
+        else hipLaunchKernelGGL((k_cells<NV, false, T>), dim3(cells_grid(c)), dim3(cells_block(c)), 0, c->stream, p);
+    });
+}
 // the faces normal to D in the variant of the configuration: the reconstruction, and whether the axis has a periodic halo
 template <int NV, int D, int MODE, int RECON, typename T>
 int launch_faces_recon(fvg_ctx* c, const KP& p) {
@@ -257,8 +268,7 @@ int enqueue_residual_nv(fvg_ctx* c, const double* Uin, int mode, bool audit, boo
     const KP p = make_kp(c, Uin);
     int rc;
     if ((rc = enqueue_massflow(c, p))) return rc;
-    if ((rc = launch(c, FAM_CELLS, [&] { hipLaunchKernelGGL((k_cells<NV, T>), dim3(cells_grid(c)), dim3(cells_block(c)), 0, c->stream, p); })))
-        return rc;
+    if ((rc = launch_cells<NV, T>(c, p))) return rc;
     if (mode == MODE_LEARNED) {
 #define LFACES(KERNEL, FAM, D, GRID, BLOCK) \
     launch(c, FAM, [&] { hipLaunchKernelGGL((KERNEL<NV, D, T>), dim3(GRID), dim3(BLOCK), 0, c->stream, p); })
@@ -321,8 +331,7 @@ int enqueue_hancock_residual(fvg_ctx* c, const double* Uin) {
     const KP p = make_kp(c, Uin);
     int rc;
     if ((rc = enqueue_massflow(c, p))) return rc;
-    if ((rc = launch(c, FAM_CELLS, [&] { hipLaunchKernelGGL((k_cells<NV, double>), dim3(cells_grid(c)), dim3(cells_block(c)), 0, c->stream, p); })))
-        return rc;
+    if ((rc = launch_cells<NV, double>(c, p))) return rc;
     if ((rc = launch(c, FAM_HANCOCK, [&] { hipLaunchKernelGGL(k_hancock<NV>, dim3(grid_for(c->nc)), dim3(kBlock), 0, c->stream, p); })))
         return rc;
     return enqueue_hancock_faces<NV>(c, p);
@@ -421,8 +430,7 @@ int enqueue_fused_nv(fvg_ctx* c, const double* Uin, int mode, bool audit, bool r
     const KP p = make_kp(c, Uin);
     int rc;
     if ((rc = enqueue_massflow(c, p))) return rc;
-    if ((rc = launch(c, FAM_CELLS, [&] { hipLaunchKernelGGL((k_cells<NV, T>), dim3(cells_grid(c)), dim3(cells_block(c)), 0, c->stream, p); })))
-        return rc;
+    if ((rc = launch_cells<NV, T>(c, p))) return rc;
     if constexpr (std::is_same<T, double>::value) {
         if (mode == MODE_HANCOCK) {
             if ((rc = launch(c, FAM_HANCOCK, [&] { hipLaunchKernelGGL(k_hancock<NV>, dim3(grid_for(c->nc)), dim3(kBlock), 0, c->stream, p); })))
@@ -787,6 +795,14 @@ void fill_kernel_params(const fvg_config& cfg, KP& p) {
         p.mg_fj[d] = magic_for((unsigned)(cfg.ny + (d == 1)));
     }
     p.npad = (long long)p.px * p.py * (cfg.nz + 2 * p.phz);
+    // k_cells_march: 16 planes per thread where that leaves at least 16 blocks per CU (4,096), else fewer; below four
+    // planes the two extra planes it loads cost what it saves (256^3 FP64: 2 planes 0.86 ms, 4 0.77, 8 0.75, 16 0.745,
+    // 32 0.745; 128^3: 0.093 at 2 to 4, 0.096 for k_cells)
+    p.kseg = 1;
+    if (three && visc && p.wrap[0] && p.wrap[1] && p.wrap[2]) {
+        const int planes = (int)std::min<long long>(16, (long long)cfg.nz * cfg.ny * p.nchunk / 4096);
+        if (planes >= 4) p.kseg = planes;
+    }
     // line segments of the fused passes along y and z: 4m - 1 cells (4m faces: whole steps of the block's 4
     // wavefronts), the longest of 127, 63, .., 3 that still gives the last axis' pass 1536 blocks (two rounds of
     // three blocks per CU); a segment of m cells computes m + 1 faces. FVG_LINE_SEGMENT overrides it (tuning).
@@ -1224,12 +1240,12 @@ int fvg_indicator_samples(fvg_ctx* c, int axis, float* X, float* dep, long long 
     auto samples = [&](auto tag) {   // the primitives in the context's flux precision, then the axis' samples
         using T = decltype(tag);
         if (c->NV == 5) {
-            hipLaunchKernelGGL((k_cells<5, T>), gc, bc, 0, c->stream, p);
+            hipLaunchKernelGGL((k_cells<5, false, T>), gc, bc, 0, c->stream, p);
             if (axis == 0) hipLaunchKernelGGL((k_samples<5, 0, T>), gf, b, 0, c->stream, p, dX, dd);
             else if (axis == 1) hipLaunchKernelGGL((k_samples<5, 1, T>), gf, b, 0, c->stream, p, dX, dd);
             else hipLaunchKernelGGL((k_samples<5, 2, T>), gf, b, 0, c->stream, p, dX, dd);
         } else {
-            hipLaunchKernelGGL((k_cells<4, T>), gc, bc, 0, c->stream, p);
+            hipLaunchKernelGGL((k_cells<4, false, T>), gc, bc, 0, c->stream, p);
             if (axis == 0) hipLaunchKernelGGL((k_samples<4, 0, T>), gf, b, 0, c->stream, p, dX, dd);
             else hipLaunchKernelGGL((k_samples<4, 1, T>), gf, b, 0, c->stream, p, dX, dd);
         }

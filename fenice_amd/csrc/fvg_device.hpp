@@ -105,6 +105,13 @@ template <bool IR> __device__ __forceinline__ double sqx(double x) {
     }
 }
 template <bool IR> __device__ __forceinline__ float sqx(float x) { return sq(x); }
+// 1 / rho for a density above the floor of c2p (or NaN): only beyond 2^1000 does the division scale
+__device__ __forceinline__ double recip_rho(double rho) {
+    double r = dvx<true>(1.0, rho);
+    if (rho > 0x1p+1000) r = 1.0 / rho;
+    return r;
+}
+__device__ __forceinline__ float recip_rho(float rho) { return dv(1.0f, rho); }
 // x / c for a constant c > 0 with inv = RN(1 / c): Markstein's correction as in quot6 (with a correctly rounded
 // reciprocal the corrected quotient is the IEEE one for every significand of c); FP32: the product
 template <bool IR> __host__ __device__ __forceinline__ double by_const(double x, double c, double inv) {
@@ -168,7 +175,7 @@ template <int NV, bool IR = false, typename T>
 __device__ __forceinline__ void c2p(const Eos& e, const T* U, T* W, T* inv_out) {
     const T g = T(e.gamma);
     const T rho = nmax<IR>(U[0], T(kEosEps));
-    const T inv = dvx<IR>(T(1.0), rho);
+    const T inv = IR ? dvx<IR>(T(1.0), rho) : recip_rho(rho);
     if (inv_out) *inv_out = inv;
     const T u = U[1] * inv, v = U[2] * inv;
     T m2 = u * u + v * v;

@@ -70,6 +70,7 @@ struct KP {
     // XCD slab (ny / 8), rows per plane (ny)
     int rbt, nchunk, slabs;   // slabs: 1 when ny divides by 8 (each XCD takes a y-slab), else 0 (rows in mesh order)
     Magic mg_chunk, mg_slab, mg_ny;
+    int kseg;   // planes per thread of k_cells_march (1: k_cells)
     Magic mg_fi[3], mg_fj[3];   // faces per row and rows per plane of the faces normal to each axis
     // fused residual passes (k_xacc, k_lacc): accumulator planes A of the partial sums of the divergence (FP64: NV
     // convective, then NV - 1 viscous with FP64 fluxes and viscosity), and the line segments of the passes along y

@@ -5,7 +5,8 @@ namespace fvg {
 
 #define FVG_UPDATE(NV, UPD) template __global__ void k_update<NV, UPD, float>(KP, const double*, const double*, double*);
 #define FVG_INST(NV)                     \
-    template __global__ void k_cells<NV, float>(KP); \
+    template __global__ void k_cells<NV, true, float>(KP);  \
+    template __global__ void k_cells<NV, false, float>(KP); \
     FVG_UPDATE(NV, UPD_RESIDUAL)         \
     FVG_UPDATE(NV, UPD_AXPY)             \
     FVG_UPDATE(NV, UPD_RK2_2)            \
@@ -13,6 +14,7 @@ namespace fvg {
     FVG_UPDATE(NV, UPD_RK3_3)
 FVG_INST(4)
 FVG_INST(5)
+template __global__ void k_cells_march<float>(KP);
 #define FVG_FACES(NV, D, PER)                                            \
     template __global__ void k_faces<NV, D, MODE_PLAIN, 1, PER, float>(KP); \
     template __global__ void k_faces<NV, D, MODE_PLAIN, 2, PER, float>(KP); \

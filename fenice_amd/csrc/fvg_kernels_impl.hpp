@@ -350,56 +350,100 @@ __device__ __forceinline__ void visc_pad_prim(const KP& p, int i, int j, int k, 
 // k_cells: primitives; with viscosity the cell velocity gradients and the viscous speed bound
 // (Physics.cpp:44-76 2-D, 520-555 and 733-741 3-D; ViscousBound.hpp:16-24)
 // ------------------------------------------------------------------------------------------------------------
+// The conservative padded state one cell from (i, j, k) along axis b (hi: beyond it, else before it). PER: every axis
+// is periodic, so it is a cell of the mesh.
+template <int NV, bool PER>
+__device__ __forceinline__ void pad_neighbour(const KP& p, int i, int j, int k, int b, bool hi, double* u) {
+    if constexpr (PER) {
+        const int n = ncell(p, b), t = coord(b, i, j, k);
+        load_cons<NV>(p, cidx_d(p, b, i, j, k, hi ? (t + 1 == n ? 0 : t + 1) : (t == 0 ? n - 1 : t - 1)), u);
+    } else {
+        const int o = hi ? 1 : -1;
+        visc_pad_cons<NV>(p, i + (b == 0 ? o : 0), j + (b == 1 ? o : 0), k + (b == 2 ? o : 0), u);
+    }
+}
+// The differences of the conservative padded state across the cell along each axis: slots 0 (rho) and the momenta
+// 1..ND. Loaded before k_cells stores anything: its stores may alias the state for all the compiler knows, so a load
+// behind them waits for nothing but still starts late (256^3: one memory latency instead of two per cell).
+template <int NV, bool PER, typename T, int AXES = NV - 2>
+__device__ __forceinline__ void cell_differences(const KP& p, int i, int j, int k, T (*d)[NV - 1]) {
+#pragma unroll
+    for (int b = 0; b < AXES; ++b) {
+        double lo[NV], hi[NV];
+        pad_neighbour<NV, PER>(p, i, j, k, b, false, lo);
+        pad_neighbour<NV, PER>(p, i, j, k, b, true, hi);
+        d[b][0] = T(hi[0] - lo[0]);
+#pragma unroll
+        for (int a = 0; a < NV - 2; ++a) d[b][a + 1] = T(hi[mom(a)] - lo[mom(a)]);
+    }
+}
+// Quotients of one cell without operand scaling: n / rho for several n from one reciprocal, n / h from 1 / h
+// (fvg_device.hpp). k_cells sees any state, so each numerator is checked; bad: one of them is out of range (or NaN) and
+// the cell is done again with the IEEE divisions.
+struct CellQuot {
+    double rho, r;
+    bool bad;
+    __device__ __forceinline__ explicit CellQuot(double rho_) : rho(rho_), r(rcp_refined(rho_)), bad(!(rho_ <= 0x1p+200)) {}
+    __device__ __forceinline__ void check(double n) { bad |= !(fabs(n) <= 0x1p+200) | ((fabs(n) < 0x1p-500) & (n != 0.0)); }
+    __device__ __forceinline__ double by_rho(double n) {
+        check(n);
+        return quot_rcp(n, rho, r);
+    }
+    __device__ __forceinline__ double by_h2(double n, double h2, double inv) {
+        check(n);
+        return by_const<true>(n, h2, inv);
+    }
+};
 // Viscous cell gradients G (velocity gradients from central differences of the conservative padded state) and the
 // cell's viscous speed bound (Physics.cpp:44-76 2-D, 520-555 and 733-741 3-D; ViscousBound.hpp:16-24), FP64 in the
-// reference's operation order.
-template <int NV>
-__device__ __forceinline__ double cell_gradients_f64(const KP& p, long long c, int i, int j, int k, const double* w) {
-    const double rho = w[0];
+// reference's operation order. FAST: the quotients of CellQuot; returns false when one was out of range.
+template <int NV, bool FAST>
+__device__ __forceinline__ bool cell_gradients_f64(const KP& p, const double (*d)[NV - 1], const double* w, double (*G)[NV - 2], double& speed) {
     constexpr int ND = NV - 2;
-    double grad[ND][ND + 1];   // grad[b][slot]: slots 0 (rho) and the momenta 1..ND
+    const double rho = w[0];
+    CellQuot q(rho);
+    double grad[ND][ND + 1];   // grad[b][slot]
 #pragma unroll
     for (int b = 0; b < ND; ++b) {
-        double lo[NV], hi[NV];
-        const int o0[3] = {b == 0 ? -1 : 0, b == 1 ? -1 : 0, b == 2 ? -1 : 0};
-        visc_pad_cons<NV>(p, i + o0[0], j + o0[1], k + o0[2], lo);
-        visc_pad_cons<NV>(p, i - o0[0], j - o0[1], k - o0[2], hi);
-        const double h2 = 2.0 * hstep(p, b);
-        grad[b][0] = (hi[0] - lo[0]) / h2;
+        const double h2 = 2.0 * hstep(p, b), inv = 0.5 * inv_hstep(p, b);
 #pragma unroll
-        for (int a = 0; a < ND; ++a) grad[b][a + 1] = (hi[mom(a)] - lo[mom(a)]) / h2;
+        for (int a = 0; a <= ND; ++a) grad[b][a] = FAST ? q.by_h2(d[b][a], h2, inv) : d[b][a] / h2;
     }
 #pragma unroll
-    for (int a = 0; a < ND; ++a) {
-        const double ua = w[mom(a)];
+    for (int a = 0; a < ND; ++a)
 #pragma unroll
-        for (int b = 0; b < ND; ++b) ((double*)p.G)[(a * ND + b) * p.nc + c] = (grad[b][a + 1] - ua * grad[b][0]) / rho;
-    }
-    const double g = p.rs.eos.gamma;
-    const double nu = smax((4.0 / 3.0) * (p.mu / rho), (p.k_cond * (g - 1.0)) / rho) + 1e-12;
+        for (int b = 0; b < ND; ++b) {
+            const double n = grad[b][a + 1] - w[mom(a)] * grad[b][0];
+            G[a][b] = FAST ? q.by_rho(n) : n / rho;
+        }
+    const double g = p.rs.eos.gamma, kg = p.k_cond * (g - 1.0);
     double mv = fabs(w[1]);
     if (mv < fabs(w[2])) mv = fabs(w[2]);
     if constexpr (NV == 5)
         if (mv < fabs(w[4])) mv = fabs(w[4]);
-    return mv + sound_speed(p.rs.eos, w[3], rho) + 2.0 * p.Ldt * p.inv_h2 * nu;
+    double nu, cs;
+    if constexpr (FAST) {   // rho and p are above their floors
+        nu = smax((4.0 / 3.0) * q.by_rho(p.mu), q.by_rho(kg)) + 1e-12;
+        cs = sqx<true>(q.by_rho(p.rs.eos.stiff ? g * (w[3] + p.rs.eos.p_inf) : g * w[3]));
+    } else {
+        nu = smax((4.0 / 3.0) * (p.mu / rho), kg / rho) + 1e-12;
+        cs = sound_speed(p.rs.eos, w[3], rho);
+    }
+    speed = mv + cs + 2.0 * p.Ldt * p.inv_h2 * nu;
+    return !FAST || !q.bad;
 }
 
 // The same in float for the FP32-flux mode: products with the reciprocals of 2h and rho in place of divisions.
 template <int NV>
-__device__ __forceinline__ double cell_gradients_f32(const KP& p, long long c, int i, int j, int k, const float* w) {
+__device__ __forceinline__ double cell_gradients_f32(const KP& p, long long c, const float (*d)[NV - 1], const float* w) {
     const float rho = w[0], inv_rho = __builtin_amdgcn_rcpf(rho);
     constexpr int ND = NV - 2;
     float grad[ND][ND + 1];
 #pragma unroll
     for (int b = 0; b < ND; ++b) {
-        double lo[NV], hi[NV];
-        const int o0[3] = {b == 0 ? -1 : 0, b == 1 ? -1 : 0, b == 2 ? -1 : 0};
-        visc_pad_cons<NV>(p, i + o0[0], j + o0[1], k + o0[2], lo);
-        visc_pad_cons<NV>(p, i - o0[0], j - o0[1], k - o0[2], hi);
         const float inv2h = float(0.5 / hstep(p, b));
-        grad[b][0] = float(hi[0] - lo[0]) * inv2h;
 #pragma unroll
-        for (int a = 0; a < ND; ++a) grad[b][a + 1] = float(hi[mom(a)] - lo[mom(a)]) * inv2h;
+        for (int a = 0; a <= ND; ++a) grad[b][a] = d[b][a] * inv2h;
     }
 #pragma unroll
     for (int a = 0; a < ND; ++a) {
@@ -423,7 +467,7 @@ __device__ __forceinline__ double cell_gradients_f32(const KP& p, long long c, i
 // mirror position; a side with neither has its halo layers copy the edge cell. u: the cell's state, w: its
 // primitives as stored. CONS: the planes Wo hold the conservative state (w = u, and a ghost is stored as it is).
 // wide: set when a ghost value stored is outside value_in_range (the copies of w are the caller's to check).
-template <int NV, typename T, bool CONS = false>
+template <int NV, typename T, bool PER, bool CONS = false>
 __device__ __forceinline__ void push_halo(const KP& p, T* Wo, int i, int j, int k, const double* u, const T* w, bool& wide) {
     auto put = [&](int d, int t, const T* v) {
         const long long pc = pidx_d(p, d, i, j, k, t);
@@ -450,7 +494,7 @@ __device__ __forceinline__ void push_halo(const KP& p, T* Wo, int i, int j, int 
     for (int d = 0; d < NV - 2; ++d) {
         const int t = coord(d, i, j, k), n = ncell(p, d);
         if (t >= PH && t < n - PH) continue;   // no halo value comes from this cell along d
-        const int hl = halo_of(p, 2 * d), hh = halo_of(p, 2 * d + 1);
+        const int hl = PER ? 1 : halo_of(p, 2 * d), hh = PER ? 1 : halo_of(p, 2 * d + 1);
         if (hl == 1) {   // periodic: both sides wrap
             if (t >= n - PH) put(d, t - n, w);
             if (t < PH) put(d, t + n, w);
@@ -468,55 +512,111 @@ __device__ __forceinline__ void push_halo(const KP& p, T* Wo, int i, int j, int 
         }
     }
 }
-template <int NV, typename T = double>
+// What k_cells stores of cell (i, j, k) with state u and differences d (viscous): primitives, halo values, gradients; the
+// viscous speed bound goes into local, wide is set when a value of the FP64 planes is outside value_in_range.
+template <int NV, bool PER, typename T>
+__device__ __forceinline__ void store_cell(const KP& p, long long c, int i, int j, int k, const double* u, const T (*d)[NV - 1], bool& wide,
+                                           double& local) {
+    constexpr int ND = NV - 2;
+    const long long pc = pidx(p, i, j, k);
+    double wd[NV];
+    c2p<NV>(p.rs.eos, u, wd, (double*)nullptr);
+    if constexpr (std::is_same<T, float>::value) {
+        // FP32 fluxes: the primitives are the FP64 ones rounded to float (the viscous ghosts of a periodic side
+        // round the same FP64 primitives, so the two faces of a periodic seam stay identical); the viscous cell
+        // gradients are computed in float
+        float w[NV];
+        to_t<NV>(wd, w);
+        float* Wo = (float*)p.W;
+#pragma unroll
+        for (int q = 0; q < NV; ++q) Wo[q * p.npad + pc] = w[q];
+        push_halo<NV, float, PER>(p, Wo, i, j, k, u, w, wide);
+        if (p.viscous) local = smax(local, cell_gradients_f32<NV>(p, c, d, w));
+    } else {
+        const double* w = wd;
+        if (p.quad4) {   // fourth-order fluxes: the padded conservative state; the primitives only for the viscous term
+#pragma unroll
+            for (int q = 0; q < NV; ++q) {
+                p.Wc[q * p.npad + pc] = u[q];
+                wide |= !value_in_range(u[q]);
+            }
+            push_halo<NV, double, PER, true>(p, p.Wc, i, j, k, u, u, wide);
+        }
+        if (!p.quad4 || p.viscous) {
+            double* Wo = (double*)p.W;
+#pragma unroll
+            for (int q = 0; q < NV; ++q) {
+                Wo[q * p.npad + pc] = w[q];
+                wide |= !value_in_range(w[q]);
+            }
+            push_halo<NV, double, PER>(p, Wo, i, j, k, u, w, wide);
+        }
+        if (p.viscous) {
+            double G[ND][ND], sp;
+            if (!p.ir || !cell_gradients_f64<NV, true>(p, d, w, G, sp)) cell_gradients_f64<NV, false>(p, d, w, G, sp);
+#pragma unroll
+            for (int a = 0; a < ND; ++a)
+#pragma unroll
+                for (int b = 0; b < ND; ++b) ((double*)p.G)[(a * ND + b) * p.nc + c] = G[a][b];
+            local = smax(local, sp);
+        }
+    }
+}
+// PER: every axis is periodic with a wrapped halo, so there is no boundary code.
+template <int NV, bool PER, typename T = double>
 __global__ __launch_bounds__(256) void k_cells(KP p) {
     const RowBlock rb = row_block(p);
-    const int i = rb.i, j = rb.j, k = rb.k;
-    const long long c = ((long long)k * p.ny + j) * p.nx + i;
     double local = 0.0;
     bool wide = false;   // a primitive stored in the FP64 planes is outside value_in_range
-    if (i < p.nx && !p.st->done) {
-        const long long pc = pidx(p, i, j, k);
-        if constexpr (std::is_same<T, float>::value) {
-            // FP32 fluxes: the primitives are the FP64 ones rounded to float (the viscous ghosts of a periodic side
-            // round the same FP64 primitives, so the two faces of a periodic seam stay identical); the viscous cell
-            // gradients are computed in float
-            double u[NV], wd[NV];
-            float w[NV];
-            load_cons<NV>(p, c, u);
-            c2p<NV>(p.rs.eos, u, wd, (double*)nullptr);
-            to_t<NV>(wd, w);
-            float* Wo = (float*)p.W;
-#pragma unroll
-            for (int q = 0; q < NV; ++q) Wo[q * p.npad + pc] = w[q];
-            push_halo<NV, float>(p, Wo, i, j, k, u, w, wide);
-            if (p.viscous) local = smax(local, cell_gradients_f32<NV>(p, c, i, j, k, w));
-        } else {
-            double u[NV], w[NV];
-            load_cons<NV>(p, c, u);
-            c2p<NV>(p.rs.eos, u, w, (double*)nullptr);
-            if (p.quad4) {   // fourth-order fluxes: the padded conservative state; the primitives only for the viscous term
-#pragma unroll
-                for (int q = 0; q < NV; ++q) {
-                    p.Wc[q * p.npad + pc] = u[q];
-                    wide |= !value_in_range(u[q]);
-                }
-                push_halo<NV, double, true>(p, p.Wc, i, j, k, u, u, wide);
-            }
-            if (!p.quad4 || p.viscous) {
-                double* Wo = (double*)p.W;
-#pragma unroll
-                for (int q = 0; q < NV; ++q) {
-                    Wo[q * p.npad + pc] = w[q];
-                    wide |= !value_in_range(w[q]);
-                }
-                push_halo<NV, double>(p, Wo, i, j, k, u, w, wide);
-            }
-            if (p.viscous) local = smax(local, cell_gradients_f64<NV>(p, c, i, j, k, w));
-        }
+    if (rb.i < p.nx) {
+        T d[NV - 2][NV - 1];
+        double u[NV];
+        const long long c = cidx(p, rb.i, rb.j, rb.k);
+        load_cons<NV>(p, c, u);
+        if (p.viscous) cell_differences<NV, PER, T>(p, rb.i, rb.j, rb.k, d);
+        if (!p.st->done)   // read behind the loads, which it need not hold up
+            store_cell<NV, PER, T>(p, c, rb.i, rb.j, rb.k, u, d, wide, local);
     }
     if (wide) p.st->wide = 1;   // a plain store of the same value from every lane that found one
     if (p.viscous) block_max_slot(p, local, SPD_VISC);
+}
+// The same on a periodic viscous 3-D mesh, each thread going up kseg planes with the states below and above in
+// registers: the loads of the planes above and below a cell cost 0.2 of 0.74 ms at 256^3 in a kernel of nothing but
+// these loads and stores, whatever the order of the blocks or the distance of the planes, although the cache holds
+// them. Measured per launch: FP64 256^3 0.80 -> 0.75 ms, FP32 192^3 0.229 -> 0.204 ms. The loop holds its addresses in
+// registers (185 / 135 VGPRs); capped at 128 for four wavefronts per SIMD it spills and takes 1.32 ms in FP64.
+template <typename T>
+__global__ __launch_bounds__(256) void k_cells_march(KP p) {
+    constexpr int NV = 5, ND = 3;
+    const RowBlock rb = row_block(p);
+    const int i = rb.i, j = rb.j;
+    double local = 0.0;
+    bool wide = false;
+    if (i < p.nx) {
+        const int k0 = rb.k * p.kseg, k1 = min(k0 + p.kseg, p.nz);
+        double below[NV], u[NV], above[NV];
+        load_cons<NV>(p, cidx(p, i, j, k0 == 0 ? p.nz - 1 : k0 - 1), below);
+        load_cons<NV>(p, cidx(p, i, j, k0), u);
+        if (!p.st->done) {
+#pragma unroll 1
+            for (int k = k0; k < k1; ++k) {
+                T d[ND][ND + 1];
+                load_cons<NV>(p, cidx(p, i, j, k + 1 == p.nz ? 0 : k + 1), above);
+                cell_differences<NV, true, T, 2>(p, i, j, k, d);
+                d[2][0] = T(above[0] - below[0]);
+#pragma unroll
+                for (int a = 0; a < ND; ++a) d[2][a + 1] = T(above[mom(a)] - below[mom(a)]);
+                store_cell<NV, true, T>(p, cidx(p, i, j, k), i, j, k, u, d, wide, local);
+#pragma unroll
+                for (int q = 0; q < NV; ++q) {
+                    below[q] = u[q];
+                    u[q] = above[q];
+                }
+            }
+        }
+    }
+    if (wide) p.st->wide = 1;
+    block_max_slot(p, local, SPD_VISC);
 }
 
 // k_nrbc: the non-reflecting ghosts of side SIDE's boundary cells (thread per cell, in the side's boundary order),
