@@ -39,6 +39,7 @@ __global__ void k_indicator_control(KP, int);
 __global__ void k_totals_final(const double*, int, long long, int, double*);
 __global__ void k_control(KP, int, int);
 __global__ void k_massflow(KP);
+__global__ void k_hancock_step2d(KP, const double*, double*);
 template <int NV, int SIDE> __global__ void k_nrbc(KP);
 __global__ void k_riemann_batch(RiemannParams, const double*, const double*, const int*, long long, double*, double*);
 }   // namespace fvg
@@ -50,6 +51,7 @@ namespace {
 constexpr int kBlock = 256;
 static_assert(kBlock >= kRowBlock, "block sizes of the kernels' launch bounds");
 constexpr int kGraphSteps = 4;   // steps per captured graph of fvg_advance
+static_assert(kGraphSteps % 2 == 0, "a graph leaves the state in the plane set it started from");
 thread_local std::string g_create_error;
 
 enum Family { FAM_CELLS, FAM_HANCOCK, FAM_FACES_X, FAM_FACES_Y, FAM_FACES_Z, FAM_UPDATE, FAM_CONTROL, FAM_AXPY, FAM_AUDIT,
@@ -99,7 +101,10 @@ struct fvg_ctx {
     bool fused = false;                // fused residual passes (k_xacc, k_lacc; no face fluxes in HBM, opt-in), or
                                        // separate face and update passes (k_faces, k_update; the default)
     double* A = nullptr;               // KP::A
-    hipGraphExec_t graph = nullptr;    // kGraphSteps steps of the scheme
+    // kGraphSteps steps of the scheme, from either of the two state plane sets: a step that goes from one to the other
+    // (k_hancock_step2d) leaves a run in U or Ut, and a graph holds the pointers it was captured with
+    hipGraphExec_t graph[2] = {nullptr, nullptr};
+    int parity = 0;                    // swaps of U and Ut so far, mod 2
     bool quad4 = false;                // flux_quadrature = fourth
     bool massflow = false;             // a mass-flow inlet side: k_massflow runs before every k_cells
     int nrbc_sides = 0;                // bit s: side s is non-reflecting (k_nrbc runs for it before every k_cells)
@@ -487,6 +492,21 @@ int plain_mode(const fvg_ctx* c) {
     return c->cfg.reconstruction == FVG_RECON_NONE ? MODE_FIRST_ORDER : MODE_PLAIN;
 }
 
+// MUSCL-Hancock steps of a periodic, inviscid 2-D mesh in one launch (k_hancock_step2d)
+bool hancock_tiles(const fvg_ctx* c) {
+    return c->NV == 4 && c->cfg.time_scheme == FVG_TS_HANCOCK && c->cfg.reconstruction == FVG_RECON_MUSCL && !c->cfg.use_viscous &&
+           c->base.wrap[0] && c->base.wrap[1] && !c->fused && c->cfg.ny / kHancockTile < 65535;   // the grid's y extent
+}
+int enqueue_hancock_tiles(fvg_ctx* c) {
+    const KP p = make_kp(c, c->U);
+    const dim3 g((c->cfg.nx + kHancockTile - 1) / kHancockTile, (c->cfg.ny + kHancockTile - 1) / kHancockTile);
+    const int rc = launch(c, FAM_HANCOCK, [&] { hipLaunchKernelGGL(k_hancock_step2d, g, dim3(512), 0, c->stream, p, c->U, c->Ut); });
+    if (rc) return rc;
+    std::swap(c->U, c->Ut);
+    c->parity ^= 1;
+    return FVG_OK;
+}
+
 // One step of the configured scheme, enqueued (TimeScheme.cpp:110-319).
 // link (MUSCL-Hancock with a lagged speed only, for steps enqueued back to back): LINK_AFTER, the previous step's end
 // was left to this step's first control launch; LINK_BEFORE, leave this step's end to the next step's.
@@ -506,7 +526,9 @@ int enqueue_step(fvg_ctx* c, int link = 0) {
         } else if ((rc = enqueue_control(c, (link & LINK_AFTER) ? CTL_END_BEGIN_HANCOCK : CTL_BEGIN_HANCOCK, ts))) {
             return rc;
         }
-        if (fused) {   // the residual into Rb, then U += dt Rb (the faces read U, so the update waits for them)
+        if (hancock_tiles(c)) {
+            if ((rc = enqueue_hancock_tiles(c))) return rc;
+        } else if (fused) {   // the residual into Rb, then U += dt Rb (the faces read U, so the update waits for them)
             if ((rc = residual_into(c, c->U, mode, false, c->Rb)) || (rc = enqueue_axpy(c, c->U, c->Rb, c->U))) return rc;
         } else {
             if ((rc = enqueue_residual(c, c->U, mode))) return rc;
@@ -565,7 +587,9 @@ int enqueue_step(fvg_ctx* c, int link = 0) {
 // no-ops. The MUSCL-Hancock seed residual is never in the graph (the first step after a reset of the lagged speed
 // runs eagerly).
 int ensure_graph(fvg_ctx* c) {
-    if (c->graph) return FVG_OK;
+    const int parity = c->parity;
+    hipGraphExec_t& graph = c->graph[parity];
+    if (graph) return FVG_OK;
     hipGraph_t g = nullptr;
     HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
     int rc = FVG_OK;
@@ -575,13 +599,17 @@ int ensure_graph(fvg_ctx* c) {
         rc = enqueue_step(c, hancock ? (k > 0 ? LINK_AFTER : 0) | (k + 1 < kGraphSteps ? LINK_BEFORE : 0) : 0);
     const hipError_t e = hipStreamEndCapture(c->stream, &g);
     if (rc || e != hipSuccess) {
+        if (c->parity != parity) {   // a failed capture ran nothing: the state is where it was
+            std::swap(c->U, c->Ut);
+            c->parity = parity;
+        }
         if (g) hipGraphDestroy(g);
         return rc ? rc : set_err(c, FVG_EHIP, std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
     }
-    const hipError_t e2 = hipGraphInstantiate(&c->graph, g, nullptr, nullptr, 0);
+    const hipError_t e2 = hipGraphInstantiate(&graph, g, nullptr, nullptr, 0);
     hipGraphDestroy(g);
     if (e2 != hipSuccess) {
-        c->graph = nullptr;
+        graph = nullptr;
         return set_err(c, FVG_EHIP, std::string("hipGraphInstantiate: ") + hipGetErrorString(e2));
     }
     return FVG_OK;
@@ -609,11 +637,18 @@ DevState fresh_state(const fvg_ctx* c) {
     return s;
 }
 
+void drop_graphs(fvg_ctx* c) {
+    for (hipGraphExec_t& g : c->graph) {
+        if (g) hipGraphExecDestroy(g);
+        g = nullptr;
+    }
+}
+
 void free_ctx(fvg_ctx* c) {
     if (!c) return;
     hipSetDevice(c->device);
     if (c->stream) hipStreamSynchronize(c->stream);
-    if (c->graph) hipGraphExecDestroy(c->graph);
+    drop_graphs(c);
     hipFree(c->mlp);
     hipFree(c->ind);
     void* bufs[] = {c->U,     c->Ut,    c->Rb,    c->W,        c->G,         c->HS,  c->Fc[0], c->Fc[1], c->Fc[2], c->A,
@@ -1090,7 +1125,7 @@ int fvg_advance(fvg_ctx* c, int max_steps, double* t, double t_end, double dt_ma
         }
         if (graphed) {
             if ((rc = ensure_graph(c))) return rc;
-            for (int k = 0; k < n; k += kGraphSteps) HIPCHK(c, hipGraphLaunch(c->graph, c->stream));
+            for (int k = 0; k < n; k += kGraphSteps) HIPCHK(c, hipGraphLaunch(c->graph[c->parity], c->stream));
         } else {
             for (int k = 0; k < n; ++k)
                 if ((rc = enqueue_step(c))) return rc;
@@ -1271,10 +1306,7 @@ int fvg_set_fused(fvg_ctx* c, int on) {
         c->base.A = c->A;
     }
     c->fused = on != 0;
-    if (c->graph) {   // the captured graph holds the old kernel sequence
-        hipGraphExecDestroy(c->graph);
-        c->graph = nullptr;
-    }
+    drop_graphs(c);   // the captured graphs hold the old kernel sequence
     return FVG_OK;
 }
 

@@ -662,6 +662,12 @@ __device__ __forceinline__ void euler_flux_axis(const Eos& e, const double* U, i
     if constexpr (NV == 5) F[4] = U[4] * un + (a == 2 ? pr : 0.0);
 }
 
+// admissible_state (Schemes.cpp:2145-2148)
+template <int NV>
+__device__ __forceinline__ bool admissible(const KP& p, const double* u) {
+    const double u4 = NV == 5 ? u[NV - 1] : 0.0;
+    return (u[0] > kEosEps) && (0.5 * (u[1] * u[1] + u[2] * u[2] + u4 * u4) < u[0] * (u[3] - p.rs.eos.p_inf));
+}
 template <int NV, bool IR>
 __device__ __forceinline__ unsigned long long hancock_cell(const KP& p, long long c) {
     constexpr int ND = NV - 2, NS = 2 * ND;
@@ -718,9 +724,7 @@ __device__ __forceinline__ unsigned long long hancock_cell(const KP& p, long lon
             double nw[NV];
 #pragma unroll
             for (int q = 0; q < NV; ++q) nw[q] = st[s][q] - dd[q];
-            const double u4 = NV == 5 ? nw[NV - 1] : 0.0;
-            // admissible_state (Schemes.cpp:2145-2148)
-            const bool ok = (nw[0] > kEosEps) && (0.5 * (nw[1] * nw[1] + nw[2] * nw[2] + u4 * u4) < nw[0] * (nw[3] - p.rs.eos.p_inf));
+            const bool ok = admissible<NV>(p, nw);
             reverted += ok ? 0 : 1;
 #pragma unroll
             for (int q = 0; q < NV; ++q) p.HS[((long long)s * NV + q) * p.nc + c] = ok ? nw[q] : st[s][q];
