@@ -40,6 +40,7 @@ __global__ void k_totals_final(const double*, int, long long, int, double*);
 __global__ void k_control(KP, int, int);
 __global__ void k_massflow(KP);
 __global__ void k_hancock_step2d(KP, const double*, double*);
+template <int RECON, bool VISC, bool PER> __global__ void k_stage2d(KP, int, const double*, const double*, double*);
 template <int NV, int SIDE> __global__ void k_nrbc(KP);
 __global__ void k_riemann_batch(RiemannParams, const double*, const double*, const int*, long long, double*, double*);
 }   // namespace fvg
@@ -55,9 +56,9 @@ static_assert(kGraphSteps % 2 == 0, "a graph leaves the state in the plane set i
 thread_local std::string g_create_error;
 
 enum Family { FAM_CELLS, FAM_HANCOCK, FAM_FACES_X, FAM_FACES_Y, FAM_FACES_Z, FAM_UPDATE, FAM_CONTROL, FAM_AXPY, FAM_AUDIT,
-              FAM_Q4_STATES, FAM_Q4_POINTS, FAM_Q4_FLUXES, FAM_N };
+              FAM_Q4_STATES, FAM_Q4_POINTS, FAM_Q4_FLUXES, FAM_STAGE2D, FAM_N };
 const char* kFamilyNames[FAM_N] = {"k_cells", "k_hancock", "k_faces_x", "k_faces_y", "k_faces_z", "k_update", "k_control", "k_axpy",
-                                   "k_audit", "k4_states", "k4_points", "k4_fluxes"};
+                                   "k_audit", "k4_states", "k4_points", "k4_fluxes", "k_stage2d"};
 
 struct Err {
     int code;
@@ -479,8 +480,32 @@ int enqueue_axpy(fvg_ctx* c, const double* U0, const double* R, double* out) {
 // whether the residuals of this context take the fused passes (the fourth-order quadrature keeps its own passes)
 bool fused_path(const fvg_ctx* c) { return c->fused && !c->quad4; }
 
-// The residual of Uin stored into R (Rb for fvg_residual): fused passes, or separate face and update passes
+// whether the Runge-Kutta stages of this context run as one launch each (k_stage2d): 2-D, FP64 fluxes, reconstructed
+// faces. Faster than the separate passes at every size measured (see the kernel).
+bool stage_tiles(const fvg_ctx* c) {
+    return c->NV == 4 && !c->fp32 && !c->learned && !c->quad4 && !c->fused && c->cfg.reconstruction != FVG_RECON_NONE &&
+           c->cfg.ny / kStageTile < 65535;   // the grid's y extent
+}
+// One stage of the 2-D residual of Uin: stored into out (UPD_RESIDUAL), or combined into the stage output; out is not Uin
+int enqueue_stage_tiles(fvg_ctx* c, const double* Uin, int upd, const double* U0, const double* Ut, double* out) {
+    const KP p = make_kp(c, Uin);
+    int rc;
+    if ((rc = enqueue_massflow(c, p))) return rc;
+    const dim3 g((c->cfg.nx + kStageTile - 1) / kStageTile, (c->cfg.ny + kStageTile - 1) / kStageTile);
+    auto go = [&](auto kernel) { return launch(c, FAM_STAGE2D, [&] { hipLaunchKernelGGL(kernel, g, dim3(512), 0, c->stream, p, upd, U0, Ut, out); }); };
+    const bool per = p.wrap[0] && p.wrap[1], visc = p.viscous != 0;
+#define STAGE(R) (visc ? (per ? go(k_stage2d<R, true, true>) : go(k_stage2d<R, true, false>)) : (per ? go(k_stage2d<R, false, true>) : go(k_stage2d<R, false, false>)))
+    switch (p.recon) {
+    case FVG_RECON_MUSCL: return STAGE(FVG_RECON_MUSCL);
+    case FVG_RECON_WENO3: return STAGE(FVG_RECON_WENO3);
+    default: return STAGE(FVG_RECON_WENO5);
+    }
+#undef STAGE
+}
+
+// The residual of Uin stored into R (Rb for fvg_residual): fused passes, one 2-D stage, or separate face and update passes
 int residual_into(fvg_ctx* c, const double* Uin, int mode, bool audit, double* R) {
+    if (mode == MODE_PLAIN && stage_tiles(c)) return enqueue_stage_tiles(c, Uin, UPD_RESIDUAL, nullptr, nullptr, R);
     if (fused_path(c)) return enqueue_fused(c, Uin, mode, audit, false, UPD_RESIDUAL, nullptr, nullptr, R);
     int rc = enqueue_residual(c, Uin, mode, audit);
     return rc ? rc : enqueue_update(c, UPD_RESIDUAL, nullptr, nullptr, R);
@@ -541,19 +566,22 @@ int enqueue_step(fvg_ctx* c, int link = 0) {
     if ((rc = enqueue_control(c, CTL_BEGIN_STEP, ts))) return rc;
     const int mode = plain_mode(c);
     if (c->learned && (rc = enqueue_indicator(c, CTL_AUDIT_BEGIN))) return rc;
-    if (fused) {
+    if (fused || stage_tiles(c)) {
         // stage 1: R into Rb, dt from its wave speed, then the first update; stages 2-3 finish their combination in
         // the last face pass (the SSP-RK3 stage-2 output goes to Rb, which stage 1's R no longer needs)
+        auto stage = [&](const double* Uin, int upd, const double* Ut, double* out) {
+            return fused ? enqueue_fused(c, Uin, mode, false, c->learned, upd, c->U, Ut, out) : enqueue_stage_tiles(c, Uin, upd, c->U, Ut, out);
+        };
         if ((rc = residual_into(c, c->U, mode, c->learned, c->Rb))) return rc;
         if ((rc = enqueue_control(c, CTL_STAGE1_DT, ts))) return rc;
         if ((rc = enqueue_axpy(c, c->U, c->Rb, ts == FVG_TS_EULER ? c->U : c->Ut))) return rc;
         if (ts == FVG_TS_SSPRK2) {
-            if ((rc = enqueue_fused(c, c->Ut, mode, false, c->learned, UPD_RK2_2, c->U, c->Ut, c->U))) return rc;
+            if ((rc = stage(c->Ut, UPD_RK2_2, c->Ut, c->U))) return rc;
             if ((rc = enqueue_control(c, CTL_STAGE_S, 2))) return rc;
         } else if (ts == FVG_TS_SSPRK3) {
-            if ((rc = enqueue_fused(c, c->Ut, mode, false, c->learned, UPD_RK3_2, c->U, c->Ut, c->Rb))) return rc;
+            if ((rc = stage(c->Ut, UPD_RK3_2, c->Ut, c->Rb))) return rc;
             if ((rc = enqueue_control(c, CTL_STAGE_S, 2))) return rc;
-            if ((rc = enqueue_fused(c, c->Rb, mode, false, c->learned, UPD_RK3_3, c->U, c->Rb, c->U))) return rc;
+            if ((rc = stage(c->Rb, UPD_RK3_3, c->Rb, c->U))) return rc;
             if ((rc = enqueue_control(c, CTL_STAGE_S, 3))) return rc;
         }
         if ((rc = enqueue_control(c, CTL_END_RK, ts))) return rc;

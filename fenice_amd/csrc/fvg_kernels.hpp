@@ -118,6 +118,7 @@ struct KP {
 constexpr int kSpeedSlots = 64, kSlotStride = 32;   // 64 slots per quantity, 256 B apart
 constexpr int SPD_CONV = 0, SPD_VISC = 1;
 constexpr int kHancockTile = 14;   // cells per side of a tile of k_hancock_step2d
+constexpr int kStageTile = 15;     // cells per side of a tile of k_stage2d
 constexpr int kRowBlock = 256;   // most threads of a row block
 constexpr int PH = 3;     // halo layers of the padded primitive planes (the WENO5-Z stencil reaches 3 cells out)
 constexpr int PXA = 32;   // row alignment of the padded planes in elements (128 B in FP32, 256 B in FP64)

@@ -1271,8 +1271,7 @@ __global__ __launch_bounds__(256) void k_samples(KP p, float* __restrict__ X, fl
 // ------------------------------------------------------------------------------------------------------------
 // The stage combination of the time scheme (TimeScheme.cpp:27-59, 150-156, 213-219) for cell c.
 template <int NV, int UPD>
-__device__ __forceinline__ void combine(const KP& p, long long c, const double* R, const double* __restrict__ U0,
-                                        const double* __restrict__ Ut, double* __restrict__ out) {
+__device__ __forceinline__ void combine(const KP& p, long long c, const double* R, const double* U0, const double* Ut, double* out) {
     const double dt = p.st->dt;
 #pragma unroll
     for (int q = 0; q < NV; ++q) {
