@@ -38,6 +38,8 @@ template <int NV, int D> __global__ void k4_fluxes(KP);
 __global__ void k_indicator_control(KP, int);
 __global__ void k_totals_final(const double*, int, long long, int, double*);
 __global__ void k_control(KP, int, int);
+__global__ void k_set_state(DevState*, DevState);
+__global__ void k_publish_state(const DevState*, DevState*);
 __global__ void k_massflow(KP);
 __global__ void k_hancock_step2d(KP, const double*, double*);
 template <int RECON, bool VISC, bool PER> __global__ void k_stage2d(KP, int, const double*, const double*, double*);
@@ -79,7 +81,8 @@ struct fvg_ctx {
     bool fp32 = false;
     double *tot_part = nullptr, *tot_out = nullptr;
     DevState* st = nullptr;
-    unsigned long long* spd = nullptr;   // wave-speed slots (KP::spd)
+    unsigned long long* spd = nullptr;   // wave-speed slots (KP::spd), a set per Runge-Kutta stage
+    int stage = 0;                       // the stage whose kernels are being enqueued (its slot set)
     DevState* st_host = nullptr;   // pinned mirror for the read-back
     HostCopy copy;                 // pinned staging of uploads and downloads
     KP base{};
@@ -186,6 +189,7 @@ int harvest_timing(fvg_ctx* c) {
 KP make_kp(fvg_ctx* c, const double* Uin) {
     KP p = c->base;
     p.U = Uin;
+    p.spd = c->spd + (size_t)c->stage * kSlotSet;
     return p;
 }
 
@@ -563,26 +567,28 @@ int enqueue_step(fvg_ctx* c, int link = 0) {
         c->lagged_positive = true;
         return FVG_OK;
     }
-    if ((rc = enqueue_control(c, CTL_BEGIN_STEP, ts))) return rc;
+    // Runge-Kutta: the start of a step (loop condition) is the end of the previous one's control launch, or the host's
+    // for a run's first step; the speeds of the later stages wait in their own slot sets for that launch
+    c->stage = 0;
     const int mode = plain_mode(c);
     if (c->learned && (rc = enqueue_indicator(c, CTL_AUDIT_BEGIN))) return rc;
     if (fused || stage_tiles(c)) {
         // stage 1: R into Rb, dt from its wave speed, then the first update; stages 2-3 finish their combination in
         // the last face pass (the SSP-RK3 stage-2 output goes to Rb, which stage 1's R no longer needs)
-        auto stage = [&](const double* Uin, int upd, const double* Ut, double* out) {
-            return fused ? enqueue_fused(c, Uin, mode, false, c->learned, upd, c->U, Ut, out) : enqueue_stage_tiles(c, Uin, upd, c->U, Ut, out);
+        auto stage = [&](int k, const double* Uin, int upd, double* out) {
+            c->stage = k;
+            const int r = fused ? enqueue_fused(c, Uin, mode, false, c->learned, upd, c->U, Uin, out) : enqueue_stage_tiles(c, Uin, upd, c->U, Uin, out);
+            c->stage = 0;
+            return r;
         };
         if ((rc = residual_into(c, c->U, mode, c->learned, c->Rb))) return rc;
         if ((rc = enqueue_control(c, CTL_STAGE1_DT, ts))) return rc;
         if ((rc = enqueue_axpy(c, c->U, c->Rb, ts == FVG_TS_EULER ? c->U : c->Ut))) return rc;
         if (ts == FVG_TS_SSPRK2) {
-            if ((rc = stage(c->Ut, UPD_RK2_2, c->Ut, c->U))) return rc;
-            if ((rc = enqueue_control(c, CTL_STAGE_S, 2))) return rc;
+            if ((rc = stage(1, c->Ut, UPD_RK2_2, c->U))) return rc;
         } else if (ts == FVG_TS_SSPRK3) {
-            if ((rc = stage(c->Ut, UPD_RK3_2, c->Ut, c->Rb))) return rc;
-            if ((rc = enqueue_control(c, CTL_STAGE_S, 2))) return rc;
-            if ((rc = stage(c->Rb, UPD_RK3_3, c->Rb, c->U))) return rc;
-            if ((rc = enqueue_control(c, CTL_STAGE_S, 3))) return rc;
+            if ((rc = stage(1, c->Ut, UPD_RK3_2, c->Rb))) return rc;
+            if ((rc = stage(2, c->Rb, UPD_RK3_3, c->U))) return rc;
         }
         if ((rc = enqueue_control(c, CTL_END_RK, ts))) return rc;
         return c->learned ? enqueue_indicator(c, CTL_AUDIT_END) : FVG_OK;
@@ -595,16 +601,20 @@ int enqueue_step(fvg_ctx* c, int link = 0) {
         return c->learned ? enqueue_indicator(c, CTL_AUDIT_END) : FVG_OK;
     }
     if ((rc = enqueue_update(c, UPD_AXPY, c->U, nullptr, c->Ut))) return rc;
-    if ((rc = enqueue_residual(c, c->Ut, mode, false, c->learned))) return rc;
-    if ((rc = enqueue_control(c, CTL_STAGE_S, 2))) return rc;
+    auto residual = [&](int k) {
+        c->stage = k;
+        const int r = enqueue_residual(c, c->Ut, mode, false, c->learned);
+        c->stage = 0;
+        return r;
+    };
+    if ((rc = residual(1))) return rc;
     if (ts == FVG_TS_SSPRK2) {
         if ((rc = enqueue_update(c, UPD_RK2_2, c->U, c->Ut, c->U))) return rc;
         if ((rc = enqueue_control(c, CTL_END_RK, ts))) return rc;
         return c->learned ? enqueue_indicator(c, CTL_AUDIT_END) : FVG_OK;
     }
     if ((rc = enqueue_update(c, UPD_RK3_2, c->U, c->Ut, c->Ut))) return rc;
-    if ((rc = enqueue_residual(c, c->Ut, mode, false, c->learned))) return rc;
-    if ((rc = enqueue_control(c, CTL_STAGE_S, 3))) return rc;
+    if ((rc = residual(2))) return rc;
     if ((rc = enqueue_update(c, UPD_RK3_3, c->U, c->Ut, c->U))) return rc;
     if ((rc = enqueue_control(c, CTL_END_RK, ts))) return rc;
     return c->learned ? enqueue_indicator(c, CTL_AUDIT_END) : FVG_OK;
@@ -643,17 +653,26 @@ int ensure_graph(fvg_ctx* c) {
     return FVG_OK;
 }
 
+// The device state set from and published to the host by one-wavefront kernels: two small copies and the wait took 14 us
+// of a step() call, these 8.
 int write_state(fvg_ctx* c, const DevState& s) {
     *c->st_host = s;
-    HIPCHK(c, hipMemcpyAsync(c->st, c->st_host, sizeof(DevState), hipMemcpyHostToDevice, c->stream));
+    hipLaunchKernelGGL(k_set_state, dim3(1), dim3(64), 0, c->stream, c->st, s);
+    HIPCHK(c, hipGetLastError());
     return FVG_OK;
 }
 int read_state(fvg_ctx* c, DevState& s) {
-    HIPCHK(c, hipMemcpyAsync(c->st_host, c->st, sizeof(DevState), hipMemcpyDeviceToHost, c->stream));
+    hipLaunchKernelGGL(k_publish_state, dim3(1), dim3(64), 0, c->stream, c->st, c->st_host);
+    HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipStreamSynchronize(c->stream));
     s = *c->st_host;
     harvest_timing(c);
     return FVG_OK;
+}
+// the start of a run's first step: the loop condition of SimulationRun.cpp:167 and the time its steps may not pass
+void begin_run(DevState& s) {
+    s.done = !(s.t < s.t_end);
+    s.t_max = s.t_end < s.t_max ? s.t_end : s.t_max;
 }
 
 DevState fresh_state(const fvg_ctx* c) {
@@ -991,7 +1010,7 @@ int fvg_create(const fvg_config* cfg_in, int device, fvg_ctx** out) {
     }
     if (!rc && (hipMalloc(&c->st, sizeof(DevState)) != hipSuccess || hipMemset(c->st, 0, sizeof(DevState)) != hipSuccess))
         rc = set_err(c, FVG_ENOMEM, "hipMalloc of the device state");
-    const size_t spd_bytes = sizeof(unsigned long long) * 2 * kSpeedSlots * kSlotStride;
+    const size_t spd_bytes = sizeof(unsigned long long) * 3 * kSlotSet;
     if (!rc && (hipMalloc(&c->spd, spd_bytes) != hipSuccess || hipMemset(c->spd, 0, spd_bytes) != hipSuccess))
         rc = set_err(c, FVG_ENOMEM, "hipMalloc of the wave-speed slots");
     if (!rc && hipHostMalloc(&c->st_host, sizeof(DevState)) != hipSuccess) rc = set_err(c, FVG_ENOMEM, "hipHostMalloc of the state mirror");
@@ -1114,6 +1133,7 @@ int fvg_step(fvg_ctx* c, double t, double t_max, double dt_max, double* dt, doub
     s.t_max = t_max;
     s.dt_max = dt_max;
     s.max_steps = 1;
+    begin_run(s);
     if ((rc = write_state(c, s))) return rc;
     if ((rc = enqueue_step(c))) return rc;
     DevState o;
@@ -1138,6 +1158,7 @@ int fvg_advance(fvg_ctx* c, int max_steps, double* t, double t_end, double dt_ma
     s.t_max = t_end;
     s.dt_max = dt_max;
     s.max_steps = max_steps > 0 ? max_steps : 0;
+    begin_run(s);
     if ((rc = write_state(c, s))) return rc;
     DevState o{};
     long long enqueued = 0;

@@ -84,30 +84,54 @@ __global__ __launch_bounds__(kMassflowThreads) void k_massflow(KP p) {
     }
 }
 
-// op: the CTL_* step; arg: the time scheme (CTL_STAGE1_DT, CTL_END_RK) or the stage number (CTL_STAGE_S).
-// Launched with kSpeedSlots threads: each takes one slot of each speed maximum, clears it, and the wavefront's
-// maxima become s_conv / s_visc; the rest runs on one thread.
+// The maximum over the 64 slots of one quantity (bit patterns of non-negative doubles order as integers); clears them.
+// Every lane of the wavefront calls it and gets the maximum.
+__device__ __forceinline__ unsigned long long take_slots(unsigned long long* set, int quantity) {
+    unsigned long long* a = set + (size_t)(quantity * kSpeedSlots + (threadIdx.x & 63)) * kSlotStride;
+    unsigned long long c = *a;
+    *a = 0;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        const unsigned long long other = __shfl_xor(c, o, 64);
+        c = other > c ? other : c;
+    }
+    return c;
+}
+// the speed of a stage from its two maxima
+__device__ __forceinline__ double slot_speed(unsigned long long conv, unsigned long long visc, int viscous) {
+    const double sc = __longlong_as_double((long long)conv);
+    return viscous ? smax(sc, __longlong_as_double((long long)visc)) : sc;
+}
+
+// The device state from a kernel argument and into pinned host memory (one wavefront, a word per lane)
+static_assert(sizeof(DevState) % 8 == 0, "DevState is copied in words of 8 bytes");
+__global__ void k_set_state(DevState* st, DevState s) {
+    if (threadIdx.x == 0) *st = s;
+}
+__global__ void k_publish_state(const DevState* st, DevState* host) {
+    constexpr int n = sizeof(DevState) / 8;
+    for (int k = threadIdx.x; k < n; k += blockDim.x) ((unsigned long long*)host)[k] = ((const unsigned long long*)st)[k];
+}
+
+// op: the CTL_* step; arg: the time scheme (CTL_STAGE1_DT, CTL_END_RK).
+// Launched with kSpeedSlots threads (one wavefront): they reduce and clear the slots of the speed maxima; the rest runs on
+// one thread. A Runge-Kutta step has two control launches: CTL_STAGE1_DT (the first stage's speed gives dt) and
+// CTL_END_RK, which takes the later stages' speeds from their own slot sets, ends the step and decides whether another
+// one follows.
 __global__ void k_control(KP p, int op, int arg) {
     const int scheme = arg;
     DevState* s = p.st;
     // every control launch comes after a residual's face kernels or between steps, never between a k_cells and its
-    // faces: clear the quotient range flag for the next k_cells (the fused passes have no k_update to clear it)
+    // faces: clear the range flag for the next k_cells (the fused passes have no k_update to clear it)
     if (threadIdx.x == 0) s->wide = 0;
+    double later[2] = {0.0, 0.0};
     if (!s->done) {
-        const int l = threadIdx.x;
-        unsigned long long* cs = p.spd + (size_t)(SPD_CONV * kSpeedSlots + l) * kSlotStride;
-        unsigned long long* vs = p.spd + (size_t)(SPD_VISC * kSpeedSlots + l) * kSlotStride;
-        unsigned long long c = *cs, v = *vs;
-        *cs = 0;
-        *vs = 0;
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {   // bit patterns of non-negative doubles order as integers
-            const unsigned long long oc = __shfl_xor(c, o, 64), ov = __shfl_xor(v, o, 64);
-            c = oc > c ? oc : c;
-            v = ov > v ? ov : v;
-        }
+        const unsigned long long c = take_slots(p.spd, SPD_CONV), v = take_slots(p.spd, SPD_VISC);
+        if (op == CTL_END_RK)
+            for (int k = 1; k <= scheme; ++k)   // uniform: SSP-RK2 has one more stage, SSP-RK3 two
+                later[k - 1] = slot_speed(take_slots(p.spd + k * kSlotSet, SPD_CONV), take_slots(p.spd + k * kSlotSet, SPD_VISC), p.viscous);
         __syncthreads();   // every lane has read s->done before thread 0 may set it
-        if (l == 0) {
+        if (threadIdx.x == 0) {
             s->s_conv = c;
             s->s_visc = v;
         }
@@ -162,14 +186,14 @@ __global__ void k_control(KP p, int op, int arg) {
             s->s_step = S;
         }
         break;
-    case CTL_STAGE_S:
-        if (arg == 2) s->s2 = S;
-        else s->s3 = S;
-        break;
     case CTL_END_RK:
+        s->s2 = later[0];
+        s->s3 = later[1];
         if (scheme == 1) s->s_step = smax(s->s1, s->s2);
         else if (scheme == 2) s->s_step = smax(s->s1, smax(s->s2, s->s3));
         end_step(s);
+        // the start of the next step
+        if (!(s->t < s->t_end) || (s->max_steps > 0 && s->steps >= s->max_steps)) s->done = 1;
         break;
     case CTL_SEED: s->lagged = S; break;
     case CTL_HANCOCK_DT:

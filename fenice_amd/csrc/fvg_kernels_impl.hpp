@@ -746,27 +746,31 @@ __global__ __launch_bounds__(256) void k_hancock(KP p) {
 // Schemes.cpp:389-700 (states), 842-911 (fused line), 231-240 (Riemann); Physics.cpp:100-176 (2-D),
 // 567-707 (3-D) for the viscous flux.
 // ------------------------------------------------------------------------------------------------------------
-// Cross derivative d u_a / d x_b on a face normal to D: the average of the cell gradients of the two cells xL, xR
-// (the opposite cell across a periodic seam), or on a physical boundary face with boundary_order = 2 the
-// tangential difference of the face values, ghost and cell layer averaged (Physics.cpp:614-628).
-template <int NV, int D, typename T>
-__device__ __forceinline__ T cross_term(const KP& p, bool phys, int i, int j, int k, int tg, int tc, long long xL, long long xR, int a,
-                                             int b) {
+// Cross derivatives d u_a / d x_b of every velocity component a on a physical boundary face with boundary_order = 2: the
+// tangential difference of the face values, ghost and cell layer averaged (Physics.cpp:614-628). tg, tc: the ghost and
+// the cell layer's coordinate along D. The four padded states are made once for all components.
+template <int NV, int D>
+__device__ __forceinline__ void boundary_cross(const KP& p, int i, int j, int k, int tg, int tc, int b, double* du) {
     constexpr int ND = NV - 2;
-    if (phys) {
-        double f[2];
+    double f[2][ND];
 #pragma unroll
-        for (int s = 0; s < 2; ++s) {
-            const int off = s == 0 ? 1 : -1;
-            const int oi = b == 0 ? off : 0, oj = b == 1 ? off : 0, ok = b == 2 ? off : 0;
-            double wg[NV], wc[NV];
-            visc_pad_prim<NV>(p, (D == 0 ? tg : i) + oi, (D == 1 ? tg : j) + oj, (D == 2 ? tg : k) + ok, wg);
-            visc_pad_prim<NV>(p, (D == 0 ? tc : i) + oi, (D == 1 ? tc : j) + oj, (D == 2 ? tc : k) + ok, wc);
-            f[s] = 0.5 * (wg[mom(a)] + wc[mom(a)]);
-        }
-        return T((f[0] - f[1]) / (2.0 * hstep(p, b)));
+    for (int s = 0; s < 2; ++s) {
+        const int off = s == 0 ? 1 : -1;
+        const int oi = b == 0 ? off : 0, oj = b == 1 ? off : 0, ok = b == 2 ? off : 0;
+        double wg[NV], wc[NV];
+        visc_pad_prim<NV>(p, (D == 0 ? tg : i) + oi, (D == 1 ? tg : j) + oj, (D == 2 ? tg : k) + ok, wg);
+        visc_pad_prim<NV>(p, (D == 0 ? tc : i) + oi, (D == 1 ? tc : j) + oj, (D == 2 ? tc : k) + ok, wc);
+#pragma unroll
+        for (int a = 0; a < ND; ++a) f[s][a] = 0.5 * (wg[mom(a)] + wc[mom(a)]);
     }
-    const T* Gp = (const T*)p.G + (long long)(a * ND + b) * p.nc;
+#pragma unroll
+    for (int a = 0; a < ND; ++a) du[a] = (f[0][a] - f[1][a]) / (2.0 * hstep(p, b));
+}
+// Cross derivative d u_a / d x_b on the other faces: the average of the cell gradients of the two cells xL, xR (the
+// opposite cell across a periodic seam).
+template <int NV, typename T>
+__device__ __forceinline__ T cell_cross(const KP& p, long long xL, long long xR, int a, int b) {
+    const T* Gp = (const T*)p.G + (long long)(a * (NV - 2) + b) * p.nc;
     return T(0.5) * (Gp[xL] + Gp[xR]);
 }
 
@@ -808,13 +812,33 @@ __device__ __forceinline__ void viscous_face(const KP& p, int i, int j, int k, i
     const T h = T(hstep(p, D));
     const double inv_h = inv_hstep(p, D);
     const int tg = lo ? -1 : n, tc = lo ? 0 : n - 1;   // the ghost and the cell layer of a boundary face
-#define CROSS(a, b) cross_term<NV, D, T>(p, phys, i, j, k, tg, tc, xL, xR, a, b)
+    // the tangential axes of the face and the cross derivatives it takes: of the component along D and of its own
+    constexpr int B1 = D == 0 ? 1 : 0, B2 = D == 2 ? 1 : 2;
+    T own1, own2 = T(0), nor1, nor2 = T(0);   // d u_B / d x_B and d u_D / d x_B for B1, B2
+    if (phys) {
+        double du[ND];
+        boundary_cross<NV, D>(p, i, j, k, tg, tc, B1, du);
+        own1 = T(du[B1]);
+        nor1 = T(du[D]);
+        if constexpr (ND == 3) {
+            boundary_cross<NV, D>(p, i, j, k, tg, tc, B2, du);
+            own2 = T(du[B2]);
+            nor2 = T(du[D]);
+        }
+    } else {
+        own1 = cell_cross<NV, T>(p, xL, xR, B1, B1);
+        nor1 = cell_cross<NV, T>(p, xL, xR, D, B1);
+        if constexpr (ND == 3) {
+            own2 = cell_cross<NV, T>(p, xL, xR, B2, B2);
+            nor2 = cell_cross<NV, T>(p, xL, xR, D, B2);
+        }
+    }
     const T mu = T(p.mu), kc = T(p.k_cond), MD = T(MU_DIAG), MO = T(MU_OFF), half = T(0.5);
     if constexpr (ND == 2) {
         const T u_f = half * (vL[0] + vR[0]), v_f = half * (vL[1] + vR[1]);
         if constexpr (D == 0) {
             const T du_dx = by_const<IR>(vR[0] - vL[0], h, inv_h), dv_dx = by_const<IR>(vR[1] - vL[1], h, inv_h), dT_dx = by_const<IR>(TR - TL, h, inv_h);
-            const T du_dy = CROSS(0, 1), dv_dy = CROSS(1, 1);
+            const T du_dy = nor1, dv_dy = own1;
             const T tau_xx = mu * (MD * du_dx - MO * dv_dy);
             const T tau_xy = mu * (du_dy + dv_dx);
             const T q_x = -kc * dT_dx;
@@ -824,7 +848,7 @@ __device__ __forceinline__ void viscous_face(const KP& p, int i, int j, int k, i
             out[2] = (u_f * tau_xx + v_f * tau_xy - q_x) * ar;
         } else {
             const T dv_dy = by_const<IR>(vR[1] - vL[1], h, inv_h), du_dy = by_const<IR>(vR[0] - vL[0], h, inv_h), dT_dy = by_const<IR>(TR - TL, h, inv_h);
-            const T du_dx = CROSS(0, 0), dv_dx = CROSS(1, 0);
+            const T du_dx = own1, dv_dx = nor1;
             const T tau_yy = mu * (MD * dv_dy - MO * du_dx);
             const T tau_yx = mu * (du_dy + dv_dx);
             const T q_y = -kc * dT_dy;
@@ -842,22 +866,9 @@ __device__ __forceinline__ void viscous_face(const KP& p, int i, int j, int k, i
         }
         const T dT = by_const<IR>(TR - TL, h, inv_h);
         T tau[3];
-        if constexpr (D == 0) {
-            const T g01 = CROSS(0, 1), g11 = CROSS(1, 1), g22 = CROSS(2, 2), g02 = CROSS(0, 2);
-            tau[0] = mu * (MD * Gn[0] - MO * ((T(0.0) + g11) + g22));
-            tau[1] = mu * (Gn[1] + g01);
-            tau[2] = mu * (Gn[2] + g02);
-        } else if constexpr (D == 1) {
-            const T g00 = CROSS(0, 0), g10 = CROSS(1, 0), g22 = CROSS(2, 2), g12 = CROSS(1, 2);
-            tau[0] = mu * (Gn[0] + g10);
-            tau[1] = mu * (MD * Gn[1] - MO * ((T(0.0) + g00) + g22));
-            tau[2] = mu * (Gn[2] + g12);
-        } else {
-            const T g00 = CROSS(0, 0), g11 = CROSS(1, 1), g20 = CROSS(2, 0), g21 = CROSS(2, 1);
-            tau[0] = mu * (Gn[0] + g20);
-            tau[1] = mu * (Gn[1] + g21);
-            tau[2] = mu * (MD * Gn[2] - MO * ((T(0.0) + g00) + g11));
-        }
+        tau[D] = mu * (MD * Gn[D] - MO * ((T(0.0) + own1) + own2));
+        tau[B1] = mu * (Gn[B1] + nor1);
+        tau[B2] = mu * (Gn[B2] + nor2);
         const T q_d = -kc * dT;
         const T area = T(D == 0 ? p.Ax : (D == 1 ? p.Ay : p.Az));
         out[0] = tau[0] * area;
@@ -866,8 +877,6 @@ __device__ __forceinline__ void viscous_face(const KP& p, int i, int j, int k, i
         out[3] = tau[2] * area;
     }
 }
-
-#undef CROSS
 
 // The MUSCL-Hancock state outside a boundary face (side `side`, boundary cell (i, j, k) whose predicted state
 // on the face is `in`): the seam copy of the cell across a periodic wrap, the reconstructed state of the ghost

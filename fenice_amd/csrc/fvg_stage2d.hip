@@ -78,22 +78,29 @@ __device__ __forceinline__ void tile_viscous(const KP& p, const StageTile<true>&
     TR = dvp<IR>(w[3], w[0]);
     const bool phys = !PER && p.bo2 && !vper_of(p, D) && (lo || hi);
     const int tg = lo ? -1 : n, tc = lo ? 0 : n - 1;
-    auto cross = [&](int a, int b) {
-        if (phys) return cross_term<4, D, double>(p, true, i, j, 0, tg, tc, 0, 0, a, b);
-        const int g = a * 2 + b;   // the cells on both sides of the face
-        return 0.5 * (s.G[g][fj + (D == 0)][fi + (D == 1)] + s.G[g][fj + 1][fi + 1]);
-    };
+    constexpr int B = 1 - D;   // the tangential axis; d u_B / d x_B and d u_D / d x_B
+    double own, nor;
+    if (phys) {
+        double d[2];
+        boundary_cross<4, D>(p, i, j, 0, tg, tc, B, d);
+        own = d[B];
+        nor = d[D];
+    } else {   // the gradients of the cells on both sides of the face
+        const int xl = fi + (D == 1), yl = fj + (D == 0);
+        own = 0.5 * (s.G[B * 2 + B][yl][xl] + s.G[B * 2 + B][fj + 1][fi + 1]);
+        nor = 0.5 * (s.G[D * 2 + B][yl][xl] + s.G[D * 2 + B][fj + 1][fi + 1]);
+    }
     const double h = hstep(p, D), inv_h = inv_hstep(p, D), mu = p.mu, kc = p.k_cond;
     const double u_f = 0.5 * (vL[0] + vR[0]), v_f = 0.5 * (vL[1] + vR[1]);
     const double du = by_const<IR>(vR[0] - vL[0], h, inv_h), dvel = by_const<IR>(vR[1] - vL[1], h, inv_h), dT = by_const<IR>(TR - TL, h, inv_h);
     if constexpr (D == 0) {
-        const double du_dy = cross(0, 1), dv_dy = cross(1, 1);
+        const double du_dy = nor, dv_dy = own;
         const double tau_xx = mu * (MU_DIAG * du - MU_OFF * dv_dy), tau_xy = mu * (du_dy + dvel), q_x = -kc * dT, ar = p.dy;
         out[0] = tau_xx * ar;
         out[1] = tau_xy * ar;
         out[2] = (u_f * tau_xx + v_f * tau_xy - q_x) * ar;
     } else {
-        const double du_dx = cross(0, 0), dv_dx = cross(1, 0);
+        const double du_dx = own, dv_dx = nor;
         const double tau_yy = mu * (MU_DIAG * dvel - MU_OFF * du_dx), tau_yx = mu * (du + dv_dx), q_y = -kc * dT, ar = p.dx;
         out[0] = tau_yx * ar;
         out[1] = tau_yy * ar;
