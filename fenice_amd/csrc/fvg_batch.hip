@@ -58,6 +58,14 @@ struct TeamSync {
     double halo[16][2][KH * 3];  // per rank, low and high end of its chunk: (rho, u, p) of its KH end cells
 };
 constexpr int kMaxTeam = 16;
+// The exchange of a team of k_ensemble_lds: a double is two words, each half of its bits below the number of the stage
+// it belongs to, so that a word says by itself whether it has arrived (no counter, no order between words). Two
+// buffers by the parity of the stage: a rank writes stage k + 2 only when every reader of its stage k is past it.
+struct TeamXch {
+    int broken, pad;
+    unsigned long long smax[2][kMaxTeam][2];
+    unsigned long long halo[2][kMaxTeam][2][KH * 3][2];   // [low, high end of the rank's chunk][cell, (rho, u, p)]
+};
 
 struct BP {
     RiemannParams rs;
@@ -79,6 +87,9 @@ struct BP {
     int nqueue, pad;
     unsigned* qnext;          // next queue entry (zeroed before the launch)
     TeamSync* sync;           // one per team (zeroed before the launch)
+    // k_ensemble_lds
+    TeamXch* xch;             // one per team (zeroed before the launch)
+    int cap, ir;              // cells that a workgroup's LDS holds; KP::ir
 };
 
 // the state of cell i of the instance as the 2-D path holds it: (rho, rho u, rho v = +0, E)
@@ -460,6 +471,402 @@ __device__ void run_instance(const BP& b, int id, int r, int m, TeamSync* ts, do
     __syncthreads();
 }
 
+// ------------------------------------------------------------------------------------------------------------
+// The run of an instance whose chunks fit in LDS (RECON 1 .. 3; see lds_cells for the rule). What bounds a run is the
+// longest instance's chain of stages: each is a few thousand cycles of dependent FP64 work and what the workgroup
+// waits between its passes. So the primitives and fluxes stay in LDS, a stage is two passes and two workgroup
+// barriers (the faces with the y faces' speeds, then the balance, stage combination and next primitives of the
+// thread's own cells, whose state is loaded while the wave speeds are reduced), the faces take the in-range
+// operations where the chunk's primitives allow them, and the ranks of a team wait for each other's words themselves
+// (TeamXch) instead of at counted barriers: for the end cells once per stage, and for the wave speed only in the
+// stage that sets dt; the others' maxima arrive with the next end cells.
+// Measured (MUSCL MC, SSP-RK2, 768 threads; microseconds per stage of one instance): 2,048 cells on one workgroup 22
+// by run_instance, 11.6 here, 4.6 by 16 workgroups; up to 256 cells 3.6, of which about 1.2 are the faces, 0.7 the
+// next primitives, 0.3 the reduction; a team adds 0.9. 512 instances of 128 .. 2,048 cells to t = 0.02: 203 -> 73 ms,
+// with the longest one's 13,604 stages the bound. The in-range operations alone, with run_instance's passes, changed
+// nothing (215 ms)).
+// ------------------------------------------------------------------------------------------------------------
+struct Lds {
+    double *W, *F;   // 3 rows each: primitives of cells lo - KH .. hi + KH - 1, fluxes of faces lo .. hi
+    int ws, fs;      // row lengths
+    double* ub;      // [2][3]: the conservative state of the instance's end cells, for sides without a halo
+};
+
+// the first-order state beyond x side `side` (boutside)
+__device__ __forceinline__ void loutside(const BP& b, const Lds& l, int side, double* ug) {
+    const int from = bc_of(b.bp, side) == 7 ? 1 - side : side;
+    double ui[4] = {l.ub[from * 3], l.ub[from * 3 + 1], 0.0, l.ub[from * 3 + 2]};
+    if (from != side) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) ug[q] = ui[q];
+        return;
+    }
+    ghost_state<4>(b.rs.eos, b.bp, side, ui, ug);
+}
+
+// the reconstruction of (rho, u, p) at the face whose left cell's primitives are at w[0] (w points into row rho of Lds::W)
+template <int RECON, int LIM, bool IR>
+__device__ __forceinline__ void lrecon(const BP& b, const Lds& l, const double* w, double* wl, double* wr) {
+    const double we = b.weno_eps;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        if (q == 2) {   // v: see bface
+            wl[q] = 0.0;
+            wr[q] = 0.0;
+            continue;
+        }
+        const double* c = w + (q == 3 ? 2 : q) * l.ws;
+        if constexpr (RECON == 3) {
+            wl[q] = weno5z<double, IR>(c[-2], c[-1], c[0], c[1], c[2], we);
+            wr[q] = weno5z<double, IR>(c[3], c[2], c[1], c[0], c[-1], we);
+        } else if constexpr (RECON == 2) {
+            wl[q] = weno3z<double, IR>(c[-1], c[0], c[1], we);
+            wr[q] = weno3z<double, IR>(c[2], c[1], c[0], we);
+        } else {
+            wl[q] = p2fma<IR>(0.5, limiter<IR>(LIM, c[0] - c[-1], c[1] - c[0]), c[0]);
+            wr[q] = p2fma<IR>(-0.5, limiter<IR>(LIM, c[2] - c[1], c[1] - c[0]), c[1]);
+        }
+    }
+}
+
+// the face whose left cell's primitives are at w[0]: bface
+template <int RECON, bool IR>
+__device__ __forceinline__ void lface(const BP& b, const Lds& l, const double* w, bool lo_end, bool hi_end, double* F, double& sm) {
+    double UL[4], UR[4];
+    if (!lo_end && !hi_end) {
+        double wl[4], wr[4];
+        if constexpr (RECON == 1) {   // one branch for the six limited slopes
+            switch (b.lim) {
+            case 0: lrecon<RECON, 0, IR>(b, l, w, wl, wr); break;
+            case 1: lrecon<RECON, 1, IR>(b, l, w, wl, wr); break;
+            case 2: lrecon<RECON, 2, IR>(b, l, w, wl, wr); break;
+            default: lrecon<RECON, 3, IR>(b, l, w, wl, wr); break;
+            }
+        } else {
+            lrecon<RECON, 0, IR>(b, l, w, wl, wr);
+        }
+        p2c<4, IR>(b.rs.eos, wl, UL);
+        p2c<4, IR>(b.rs.eos, wr, UR);
+    } else {   // end of the instance without a halo (one cell: both ends)
+        const int e = lo_end ? 0 : 1;
+        double in[4] = {l.ub[e * 3], l.ub[e * 3 + 1], 0.0, l.ub[e * 3 + 2]}, out[4];
+        loutside(b, l, e, out);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            UL[q] = lo_end ? out[q] : in[q];
+            UR[q] = lo_end ? in[q] : out[q];
+        }
+        roundtrip<4>(b.rs.eos, UL);
+        roundtrip<4>(b.rs.eos, UR);
+    }
+    face_flux<4, IR>(b.rs, UL, UR, 0, F, sm);
+}
+// by_speed of a reconstructed scheme
+template <bool IR>
+__device__ __forceinline__ double ly_speed(const BP& b, const double* w, int ws) {
+    const double wc[4] = {w[0], w[ws], 0.0, w[2 * ws]};
+    double u2[4], w2[4], inv2;
+    p2c<4, IR>(b.rs.eos, wc, u2);
+    c2p<4, IR>(b.rs.eos, u2, w2, &inv2);
+    return sound_speed_inv<IR>(b.rs.eos, w2[3], inv2);
+}
+
+__device__ __forceinline__ void word_put(unsigned long long* p, double v, unsigned tag) {
+    const unsigned long long u = (unsigned long long)__double_as_longlong(v), h = (unsigned long long)tag << 32;
+    __hip_atomic_store(p, h | (u & 0xffffffffull), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(p + 1, h | (u >> 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ unsigned long long word_get(const unsigned long long* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// the double of an even lane's low and its odd neighbour's high half, in both lanes
+__device__ __forceinline__ double word_join(unsigned long long v) {
+    const unsigned mine = (unsigned)v, other = __shfl_xor(mine, 1, 64);
+    const bool odd = threadIdx.x & 1;
+    return __longlong_as_double((long long)(((unsigned long long)(odd ? mine : other) << 32) | (odd ? other : mine)));
+}
+// One wavefront waits until word h (of stage hk) and word s (of stage sk) of each lane have arrived (null: nothing to
+// wait for). Bounded as team_barrier's wait; false when this or another member gave up.
+__device__ __forceinline__ bool words_wait(TeamXch* tx, const unsigned long long* h, unsigned hk, const unsigned long long* s, unsigned sk,
+                                           unsigned long long& hv, unsigned long long& sv) {
+    hv = 0;
+    sv = 0;
+    for (unsigned spins = 0;; ++spins) {
+        if (h) hv = word_get(h);
+        if (s) sv = word_get(s);
+        const bool here = (!h || (unsigned)(hv >> 32) == hk) && (!s || (unsigned)(sv >> 32) == sk);
+        if (__all(here)) return true;
+        if (spins >= kTeamSpin || ((spins & 255) == 255 && __hip_atomic_load(&tx->broken, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
+            __hip_atomic_store(&tx->broken, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            return false;
+        }
+    }
+}
+// the largest of a wavefront's non-negative doubles, in lane 63 (moves between neighbouring rows of lanes, about a
+// quarter of the time of six shuffles through LDS)
+template <int CTRL>
+__device__ __forceinline__ double dpp_max(double v) {
+    const long long u = __double_as_longlong(v);
+    const int lo = (int)u, hi = (int)(u >> 32);
+    const unsigned a = (unsigned)__builtin_amdgcn_update_dpp(lo, lo, CTRL, 0xf, 0xf, false);
+    const unsigned c = (unsigned)__builtin_amdgcn_update_dpp(hi, hi, CTRL, 0xf, 0xf, false);
+    return fmax(v, __longlong_as_double((long long)(((unsigned long long)c << 32) | a)));
+}
+__device__ __forceinline__ double wave_max(double v) {
+    v = dpp_max<0x111>(v);   // row_shr 1, 2, 4, 8: the largest of each row of 16 in its last lane
+    v = dpp_max<0x112>(v);
+    v = dpp_max<0x114>(v);
+    v = dpp_max<0x118>(v);
+    v = dpp_max<0x142>(v);   // row_bcast 15 and 31: on to the next row, and to the upper half
+    return dpp_max<0x143>(v);
+}
+
+// the workgroup's barrier for LDS alone: a thread's global memory is its own (the state), or words that say themselves
+// whether they have arrived, so no load or store in flight has to be waited for
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+struct LdsShared {
+    double red[16], ub[6], sx[2];
+    int wide[2], ok[2];
+};
+
+// run_instance with the chunk in LDS: the same values, times and step counts. k numbers the stages of the run from 1.
+template <int BS, int RECON>
+__device__ void run_instance_lds(const BP& b, int id, int r, int m, TeamXch* tx, double* mem, LdsShared& sh) {
+    const BInst in = b.inst[id];
+    const int n = in.n, nst = b.scheme + 1;
+    const bool team = m > 1, per = in.halo_lo == 1;
+    const int lo = (int)((long long)n * r / m), hi = (int)((long long)n * (r + 1) / m);
+    const bool from_lo = team && (r > 0 || per), from_hi = team && (r < m - 1 || per);   // halos that other ranks hold
+    Lds l;
+    l.ws = b.cap + 2 * KH;
+    l.fs = b.cap + 1;
+    l.W = mem;
+    l.F = mem + 3 * l.ws;
+    l.ub = sh.ub;
+    const int tid = threadIdx.x;
+    if (tid < 2) {
+        sh.wide[tid] = 0;
+        sh.ok[tid] = 1;
+    }
+    lds_barrier();
+
+    // the primitives of cell c of an end of the chunk, to the neighbour rank
+    auto give = [&](int side, int c, const double* w, unsigned k) {
+        unsigned long long(*y)[2] = tx->halo[k & 1][r][side] + c * 3;
+        word_put(y[0], w[0], k);
+        word_put(y[1], w[1], k);
+        word_put(y[2], w[3], k);
+    };
+    // the primitives of cell i of the next stage's input u, and the padded or exchanged cells that they are
+    auto publish = [&](int i, const double* u3, unsigned k) {
+        const double u[4] = {u3[0], u3[1], 0.0, u3[2]};
+        double w[4];
+        c2p<4>(b.rs.eos, u, w, (double*)nullptr);
+        if (from_lo && i < lo + KH) give(0, i - lo, w, k);
+        if (from_hi && i >= hi - KH) give(1, i - hi + KH, w, k);
+        double* W = l.W + (i - lo + KH);
+        auto put = [&](int t, const double* v) {   // the primitives at x index t
+            double* y = l.W + (t - lo + KH);
+            y[0] = v[0];
+            y[l.ws] = v[1];
+            y[2 * l.ws] = v[3];
+        };
+        bool out = !(value_in_range(w[0]) & value_in_range(w[1]) & value_in_range(w[3]));
+        W[0] = w[0];
+        W[l.ws] = w[1];
+        W[2 * l.ws] = w[3];
+        if ((!from_lo && i < lo + KH) || (!from_hi && i >= hi - KH)) {   // at an end of the instance
+#pragma unroll 1
+            for (int side = 0; side < 2; ++side) {
+                const int d = side ? hi - 1 - i : i - lo;   // cells from that end of the chunk
+                if (d >= KH || (side ? from_hi : from_lo)) continue;
+                if (d == 0) {
+                    sh.ub[side * 3] = u3[0];
+                    sh.ub[side * 3 + 1] = u3[1];
+                    sh.ub[side * 3 + 2] = u3[2];
+                }
+                const int h = side ? in.halo_hi : in.halo_lo;
+                if (h == 1) {   // the cell as the other end's halo
+                    put(side ? i - n : i + n, w);
+                } else if (h == 2 && bc_of(b.bp, side) == 6) {   // a transmissive side's ghost is the mirrored cell
+                    put(side ? n + d : -1 - d, w);
+                } else if (h == 2) {   // the ghost of the mirrored cell
+                    double ug[4], wg[4];
+                    ghost_state<4>(b.rs.eos, b.bp, side, u, ug);
+                    c2p<4>(b.rs.eos, ug, wg, (double*)nullptr);
+                    out |= !(value_in_range(wg[0]) & value_in_range(wg[1]) & value_in_range(wg[3]));
+                    put(side ? n + d : -1 - d, wg);
+                } else if (d == 0) {
+                    for (int g = 0; g < KH; ++g) put(side ? n + g : -1 - g, w);
+                }
+            }
+        }
+        if (out || !b.ir) sh.wide[k & 1] = 1;
+    };
+
+    for (int i = lo + tid; i < hi; i += BS) {
+        const long long c = in.c0 + i;
+        const double u[3] = {b.U[c], b.U[b.nc + c], b.U[2 * b.nc + c]};
+        publish(i, u, 1);
+    }
+    double t = 0.0, dt = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0, s_step = 0.0;
+    int steps = 0, diverged = 0;
+    bool begun = false, stop = false;   // a step awaits its end
+    unsigned k = 0;
+    for (;;) {
+        for (int st = 1; st <= nst; ++st) {
+            ++k;
+            const bool late = team && nst > 1 && begun && st != 2;   // the previous stage's team maximum comes now
+            if (team && tid < 64) {
+                const int side = tid / (KH * 6), e = tid % (KH * 6) / 2, half = tid & 1;
+                const unsigned long long *hp = nullptr, *sp = nullptr;
+                if (tid < 2 * KH * 6 && (side ? from_hi : from_lo)) hp = &tx->halo[k & 1][side ? (r + 1) % m : (r + m - 1) % m][1 - side][e][half];
+                if (late && tid < 2 * m) sp = &tx->smax[(k - 1) & 1][tid >> 1][half];
+                unsigned long long hv, sv;
+                const bool ok = words_wait(tx, hp, k, sp, k - 1, hv, sv);
+                const double w = word_join(hv), s = wave_max(word_join(sv));
+                if (hp && !half) {
+                    l.W[(e % 3) * l.ws + (side ? hi - lo + KH : 0) + e / 3] = w;
+                    if (!value_in_range(w)) sh.wide[k & 1] = 1;
+                }
+                if (tid == 63) {
+                    sh.sx[0] = s;
+                    if (!ok) sh.ok[0] = 0;
+                }
+            }
+            lds_barrier();
+            if (team && !sh.ok[0]) {
+                diverged = 2;
+                stop = true;
+                break;
+            }
+            if (late) {
+                if (st == 3 || b.scheme == 1) s2 = sh.sx[0];
+                else s3 = sh.sx[0];
+            }
+            if (st == 1) {   // the end of the step before, and whether another one follows
+                if (begun) {
+                    s_step = b.scheme == 0 ? s1 : (b.scheme == 1 ? smax(s1, s2) : smax(s1, smax(s2, s3)));
+                    steps += 1;
+                    if (!(isfinite(s_step) && isfinite(dt) && t + dt > t)) {
+                        diverged = 1;
+                        stop = true;
+                        break;
+                    }
+                    t += dt;
+                }
+                begun = true;
+                if (!(t < b.t_end && steps < b.max_steps)) {
+                    stop = true;
+                    break;
+                }
+            }
+            const bool wide = sh.wide[k & 1] != 0;
+            if (tid == 0) sh.wide[(k + 1) & 1] = 0;   // last read before this stage's first barrier, next set after its second
+            double local = 0.0;
+            for (int f = lo + tid; f <= hi; f += BS) {
+                const double* w = l.W + (f - 1 - lo + KH);
+                const bool le = f == 0 && in.halo_lo == 0, he = f == n && in.halo_hi == 0;
+                double F[4], sm;
+                if (!wide) lface<RECON, true>(b, l, w, le, he, F, sm);
+                else lface<RECON, false>(b, l, w, le, he, F, sm);
+                if (sm > local) local = sm;
+                double* y = l.F + (f - lo);
+                y[0] = F[0];
+                y[l.fs] = F[1];
+                y[2 * l.fs] = F[3];
+            }
+            // the cells' y faces, from the other end of the workgroup: a short chunk leaves these wavefronts free
+            for (int i = lo + BS - 1 - tid; i < hi; i += BS) {
+                const double* w = l.W + (i - lo + KH);
+                const double sy = !wide ? ly_speed<true>(b, w, l.ws) : ly_speed<false>(b, w, l.ws);
+                if (sy > local) local = sy;
+            }
+            // the thread's first cell, on its way while the speeds are reduced
+            double u0[3] = {}, u1[3] = {};
+            auto fetch = [&](int i) {
+                const long long c = in.c0 + i;
+#pragma unroll
+                for (int q = 0; q < 3; ++q) u0[q] = b.U[q * b.nc + c];
+                if (st > 1) {
+#pragma unroll
+                    for (int q = 0; q < 3; ++q) u1[q] = b.Ut[q * b.nc + c];
+                }
+            };
+            if (lo + tid < hi) fetch(lo + tid);
+            local = wave_max(local);
+            if ((tid & 63) == 63) sh.red[tid >> 6] = local;
+            lds_barrier();
+            double S = sh.red[0];
+#pragma unroll
+            for (int w = 1; w < BS / 64; ++w) S = fmax(S, sh.red[w]);
+            if (team) {
+                if (tid == 0) word_put(tx->smax[k & 1][r], S, k);
+                if (st == 1) {
+                    if (tid < 64) {
+                        const unsigned long long* sp = tid < 2 * m ? &tx->smax[k & 1][tid >> 1][tid & 1] : nullptr;
+                        unsigned long long hv, sv;
+                        const bool ok = words_wait(tx, nullptr, 0, sp, k, hv, sv);
+                        const double s = wave_max(word_join(sv));
+                        if (tid == 63) {
+                            sh.sx[1] = s;
+                            if (!ok) sh.ok[1] = 0;
+                        }
+                    }
+                    lds_barrier();
+                    if (!sh.ok[1]) {
+                        diverged = 2;
+                        stop = true;
+                        break;
+                    }
+                    S = sh.sx[1];
+                }
+            }
+            if (st == 1) {
+                s1 = S;
+                dt = smin(b.cfl * in.Ldt / (S + kDtEps), b.t_end - t);
+                if (b.dt_max > 0.0) dt = smin(dt, b.dt_max);
+            } else if (!team) {
+                if (st == 2) s2 = S;
+                else s3 = S;
+            }
+            // stage 1: the Euler step; later: c0 U + c1 (Ut + dt R)
+            const double c0 = b.scheme == 1 ? 0.5 : (st == 2 ? 0.75 : 1.0 / 3.0), c1 = b.scheme == 1 ? 0.5 : (st == 2 ? 0.25 : 2.0 / 3.0);
+            double* to = st == nst ? b.U : b.Ut;
+            for (int i = lo + tid; i < hi; i += BS) {
+                const double v0[3] = {u0[0], u0[1], u0[2]}, v1[3] = {u1[0], u1[1], u1[2]};
+                if (i + BS < hi) fetch(i + BS);
+                const double* y = l.F + (i - lo);
+                double u[3];
+#pragma unroll
+                for (int q = 0; q < 3; ++q) {
+                    const double R = (0.0 - (y[q * l.fs + 1] * in.Ax - y[q * l.fs] * in.Ax)) * in.inv_vol;
+                    const double e = (st == 1 ? v0[q] : v1[q]) + dt * R;
+                    u[q] = st == 1 ? e : c0 * v0[q] + c1 * e;
+                    to[q * b.nc + in.c0 + i] = u[q];
+                }
+                publish(i, u, k + 1);
+            }
+        }
+        if (stop) break;
+    }
+    if (r == 0 && tid == 0) {
+        BOut o;
+        o.t = t;
+        o.s_last = s_step;
+        o.dt_last = dt;
+        o.steps = steps;
+        o.diverged = diverged;
+        b.out[id] = o;
+    }
+    lds_barrier();
+}
+
 // Workgroups [0, team_wgs) run the teams' instances, then every workgroup takes the queued instances one at a time
 // (longest first) until none is left. Without a queue, workgroup k runs instance order[k] alone.
 // 512 and 768 threads: at most 168 VGPRs (three wavefronts per SIMD; with 768 threads a CU runs 12 wavefronts of one
@@ -495,6 +902,40 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(kEnsembleWav
             id = b.queue[k];
         }
         run_instance<BS, RECON>(b, id, r, m, ts, red, hl, hh, fx, &flag);
+        if (phase == 0) break;
+        phase = 2;
+    }
+}
+
+template <int BS, int RECON>
+__global__ __launch_bounds__(BS) void k_ensemble_lds(BP b) {
+    extern __shared__ double mem[];
+    __shared__ LdsShared sh;
+    __shared__ int slot;
+    const int wg = blockIdx.x;
+    // 0: the launch's own instance (no queue), 1: the workgroup's team, 2: the queue
+    int phase = !b.queue ? 0 : (wg < b.team_wgs ? 1 : 2);
+    for (;;) {
+        int id, r = 0, m = 1;
+        TeamXch* tx = nullptr;
+        if (phase == 0) {
+            id = b.order[wg];
+        } else if (phase == 1) {
+            int k = 0;
+            while (wg >= b.teams[k].wg0 + b.teams[k].m) ++k;
+            id = b.teams[k].inst;
+            r = wg - b.teams[k].wg0;
+            m = b.teams[k].m;
+            tx = b.xch + k;
+        } else {
+            if (threadIdx.x == 0) slot = (int)atomicAdd(b.qnext, 1u);
+            __syncthreads();
+            const int k = slot;
+            __syncthreads();
+            if (k >= b.nqueue) break;
+            id = b.queue[k];
+        }
+        run_instance_lds<BS, RECON>(b, id, r, m, tx, mem, sh);
         if (phase == 0) break;
         phase = 2;
     }
@@ -905,12 +1346,15 @@ struct fvg_batch {
     std::string err;
     // teams (1-D instances): the largest instances split over several workgroups of a cooperative launch
     int max_team = 8, min_chunk = 512, force_teams = 0;
+    bool teams_set = false;              // fvg_batch_set_teams was called
     bool coop = false;                   // the device supports cooperative launches
     std::vector<double> cost;            // estimated work per instance (N^2 x initial wave speed)
     BTeam* d_teams = nullptr;
     int* d_queue = nullptr;
     unsigned* d_qnext = nullptr;
     TeamSync* d_sync = nullptr;
+    TeamXch* d_txch = nullptr;           // exchanges of k_ensemble_lds's teams
+    int lds_cap = 0;                     // lds_cells(): cells per workgroup of k_ensemble_lds, 0 without it
     double* d_xch = nullptr;             // 2-D teams: the exchange rows (BP2::xch), grown as plans need
     long long xch_cap = 0;               // its size in doubles
     int plan_teams = 0, plan_team_wgs = 0, plan_grid = 0;   // the last launch's plan
@@ -947,13 +1391,58 @@ void free_batch(fvg_batch* b) {
     hipFree(b->d_queue);
     hipFree(b->d_qnext);
     hipFree(b->d_sync);
+    hipFree(b->d_txch);
     hipFree(b->d_xch);
     if (b->stream) hipStreamDestroy(b->stream);
     delete b;
 }
 
+size_t lds_bytes(int cap) { return sizeof(double) * 3 * (size_t)(2 * cap + 2 * KH + 1); }
+
+// The cells that a workgroup of k_ensemble_lds holds, the largest instance's: 48 bytes each, so up to 3,300 or so in the
+// 160 KB of a CU. 0 where k_ensemble runs instead: larger instances, first-order faces (they read the conservative
+// state of both cells) and an x side that is periodic on its own (a rank of a team does not hold the other end).
+int lds_cells(const fvg_batch* b) {
+    if (b->dim != 1 || b->cfg.reconstruction == FVG_RECON_NONE) return 0;
+    if ((b->cfg.bc[0] == FVG_BC_PERIODIC) != (b->cfg.bc[1] == FVG_BC_PERIODIC)) return 0;
+    int shared = 0;
+    if (hipDeviceGetAttribute(&shared, hipDeviceAttributeMaxSharedMemoryPerBlock, b->device) != hipSuccess) return 0;
+    const int cap = *std::max_element(b->n.begin(), b->n.end());
+    return lds_bytes(cap) + sizeof(LdsShared) + 64 <= (size_t)shared ? cap : 0;
+}
+
+// the launch's dynamic LDS, above the 64 KB that a kernel may take without asking
+template <int BS, int RECON>
+int lds_allow(fvg_batch* b) {
+    BCHK(b, hipFuncSetAttribute((const void*)k_ensemble_lds<BS, RECON>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes(b->lds_cap)));
+    return FVG_OK;
+}
+
 template <int BS>
-void launch_bs(fvg_batch* b, const BP& p) {
+int launch_lds(fvg_batch* b, const BP& p) {
+    const dim3 g(b->ninst), t(BS);
+    const size_t by = lds_bytes(p.cap);
+    int rc = FVG_OK;
+    switch (p.recon) {
+    case 1:
+        if ((rc = lds_allow<BS, 1>(b))) return rc;
+        hipLaunchKernelGGL((k_ensemble_lds<BS, 1>), g, t, by, b->stream, p);
+        break;
+    case 2:
+        if ((rc = lds_allow<BS, 2>(b))) return rc;
+        hipLaunchKernelGGL((k_ensemble_lds<BS, 2>), g, t, by, b->stream, p);
+        break;
+    default:
+        if ((rc = lds_allow<BS, 3>(b))) return rc;
+        hipLaunchKernelGGL((k_ensemble_lds<BS, 3>), g, t, by, b->stream, p);
+        break;
+    }
+    return rc;
+}
+
+template <int BS>
+int launch_bs(fvg_batch* b, const BP& p) {
+    if (b->lds_cap) return launch_lds<BS>(b, p);
     const dim3 g(b->ninst), t(BS);
     if (b->dim == 2) {   // the run's time, dt_max and step limit go with the 2-D parameters
         BP2 q = b->base2;
@@ -966,7 +1455,7 @@ void launch_bs(fvg_batch* b, const BP& p) {
         case 2: hipLaunchKernelGGL((k_ensemble2<BS, 2>), g, t, 0, b->stream, q); break;
         default: hipLaunchKernelGGL((k_ensemble2<BS, 3>), g, t, 0, b->stream, q); break;
         }
-        return;
+        return FVG_OK;
     }
     switch (p.recon) {
     case 0: hipLaunchKernelGGL((k_ensemble<BS, 0>), g, t, 0, b->stream, p); break;
@@ -974,29 +1463,34 @@ void launch_bs(fvg_batch* b, const BP& p) {
     case 2: hipLaunchKernelGGL((k_ensemble<BS, 2>), g, t, 0, b->stream, p); break;
     default: hipLaunchKernelGGL((k_ensemble<BS, 3>), g, t, 0, b->stream, p); break;
     }
+    return FVG_OK;
 }
 
 // The teams of a launch of `grid` resident workgroups of `bs` threads. With force_teams every instance of at least
 // 2 min_chunk cells gets min(max_team, N / min_chunk) workgroups while they last. Otherwise the plan shortens the run
 // greedily: an instance's run is modelled as steps x (a + b N / m + c [m > 1]) microseconds, with steps proportional
 // to its estimated work over N (work = N^2 x initial wave speed), a the fixed latency of a stage, b the time per cell
-// of a chunk and c the cost of the two team barriers of a stage (about 9, 0.0065 and 6 us measured on MI355X with
-// 1,024 threads; b grows as the square root of 1024 / bs). The longest modelled run takes one more workgroup while
+// of a chunk and c the cost of the team's waits in a stage (measured on MI355X: about 9, 0.0065 and 6 us for k_ensemble
+// with 1,024 threads, b growing as the square root of 1024 / bs; 4.1, 0.0037 and 1.1 us for k_ensemble_lds with 768 or
+// more, b growing as the square root of 768 / bs). The longest modelled run takes one more workgroup while
 // that shortens it without raising the bound max(longest run, total workgroup time / grid), each chunk keeps at least min_chunk cells, a
 // team at most max_team workgroups and the teams at most three quarters of the grid. The other instances form the
-// queue, longest first.
+// queue, longest first. Where fvg_batch_set_teams was not called, k_ensemble_lds takes teams of up to 16 workgroups of
+// 96 cells or more (its waits are cheap: 73 ms on the 512 instances of 128 .. 2,048 cells, 90 with 8 of 512).
 void plan_teams(const fvg_batch* b, int grid, int bs, std::vector<BTeam>& teams, std::vector<int>& queue) {
     teams.clear();
     queue.clear();
     const int ninst = (int)b->order.size();
     std::vector<int> m(b->n.size(), 1);
+    const bool lds = b->lds_cap > 0;
+    const int max_team = b->teams_set || !lds ? b->max_team : kMaxTeam, min_chunk = b->teams_set || !lds ? b->min_chunk : 96;
     auto cap = [&](int id) {   // most workgroups instance id may take
         const int n = b->n[id];
-        if (b->max_team < 2 || b->min_chunk < KH || n < 2 * b->min_chunk) return 1;
-        int k = std::min(b->max_team, std::min(kMaxTeam, n / b->min_chunk));
+        if (max_team < 2 || min_chunk < KH || n < 2 * min_chunk) return 1;
+        int k = std::min(max_team, std::min(kMaxTeam, n / min_chunk));
         if (b->dim == 2) {   // slabs of whole rows, at least KH of them and min_chunk cells
             const int nx = b->inst2[id].nx, ny = b->inst2[id].ny;
-            const int rows = std::max(KH, (b->min_chunk + nx - 1) / nx);
+            const int rows = std::max(KH, (min_chunk + nx - 1) / nx);
             k = std::min(k, ny / rows);
         }
         return std::max(1, k);
@@ -1010,8 +1504,9 @@ void plan_teams(const fvg_batch* b, int grid, int bs, std::vector<BTeam>& teams,
                 wgs += k;
             }
         }
-    } else if (b->max_team > 1 && grid > 1) {
-        const double A = 9.0, Bc = 0.0065 * std::sqrt(1024.0 / bs), C = 6.0;
+    } else if (max_team > 1 && grid > 1) {
+        const double A = lds ? 4.1 : 9.0, Bc = lds ? 0.0037 * std::sqrt(768.0 / std::min(bs, 768)) : 0.0065 * std::sqrt(1024.0 / bs),
+                     C = lds ? 1.1 : 6.0;
         auto run = [&](int id, int k) {
             const double n = b->n[id], steps = b->cost[id] / std::max(1.0, n);
             return steps * (A + Bc * n / k + (k > 1 ? C : 0.0));
@@ -1030,7 +1525,11 @@ void plan_teams(const fvg_batch* b, int grid, int bs, std::vector<BTeam>& teams,
             const auto [t, id] = heap.back();
             heap.pop_back();
             const int k = m[id] + 1, extra = (m[id] == 1 ? 2 : 1);
-            if (k > cap(id) || wgs + extra > max_wgs) break;
+            if (wgs + extra > max_wgs) break;
+            if (k > cap(id)) {
+                if (lds) continue;   // the others may be longer than modelled: their waves form after the first steps
+                break;
+            }
             const double t2 = run(id, k);
             const double total2 = total - m[id] * t + k * t2;
             const double next = heap.empty() ? 0.0 : heap.front().first;
@@ -1057,8 +1556,15 @@ void plan_teams(const fvg_batch* b, int grid, int bs, std::vector<BTeam>& teams,
 // The teamed launch of the 1-D kernel: workgroups resident at once (a cooperative launch), teams then the queue.
 template <int BS, int RECON>
 int launch_teams(fvg_batch* b, BP p) {
+    const bool lds = b->lds_cap > 0;
+    const void* kern = lds ? (const void*)k_ensemble_lds<BS, RECON> : (const void*)k_ensemble<BS, RECON>;
+    const size_t by = lds ? lds_bytes(p.cap) : 0;
+    if (lds) {
+        const int rc = lds_allow<BS, RECON>(b);
+        if (rc) return rc;
+    }
     int per_cu = 0, dev_cus = 0;
-    BCHK(b, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)k_ensemble<BS, RECON>, BS, 0));
+    BCHK(b, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, BS, by));
     BCHK(b, hipDeviceGetAttribute(&dev_cus, hipDeviceAttributeMultiprocessorCount, b->device));
     const int resident = per_cu * dev_cus;
     if (resident < 1) return bset(b, FVG_EHIP, "the ensemble kernel cannot be resident");
@@ -1071,7 +1577,8 @@ int launch_teams(fvg_batch* b, BP p) {
     if (!teams.empty()) BCHK(b, hipMemcpy(b->d_teams, teams.data(), sizeof(BTeam) * teams.size(), hipMemcpyHostToDevice));
     if (!queue.empty()) BCHK(b, hipMemcpy(b->d_queue, queue.data(), sizeof(int) * queue.size(), hipMemcpyHostToDevice));
     BCHK(b, hipMemsetAsync(b->d_qnext, 0, sizeof(unsigned), b->stream));
-    if (!teams.empty()) BCHK(b, hipMemsetAsync(b->d_sync, 0, sizeof(TeamSync) * teams.size(), b->stream));
+    if (!teams.empty() && lds) BCHK(b, hipMemsetAsync(b->d_txch, 0, sizeof(TeamXch) * teams.size(), b->stream));
+    else if (!teams.empty()) BCHK(b, hipMemsetAsync(b->d_sync, 0, sizeof(TeamSync) * teams.size(), b->stream));
     p.teams = b->d_teams;
     p.nteams = (int)teams.size();
     p.team_wgs = wgs;
@@ -1079,8 +1586,9 @@ int launch_teams(fvg_batch* b, BP p) {
     p.nqueue = (int)queue.size();
     p.qnext = b->d_qnext;
     p.sync = b->d_sync;
+    p.xch = b->d_txch;
     void* args[] = {&p};
-    BCHK(b, hipLaunchCooperativeKernel((const void*)k_ensemble<BS, RECON>, dim3(grid), dim3(BS), args, 0, b->stream));
+    BCHK(b, hipLaunchCooperativeKernel(kern, dim3(grid), dim3(BS), args, (unsigned)by, b->stream));
     b->plan_teams = (int)teams.size();
     b->plan_team_wgs = wgs;
     b->plan_grid = grid;
@@ -1187,14 +1695,16 @@ int launch_ensemble(fvg_batch* b, const BP& p, int block) {
     b->plan_teams = 0;
     b->plan_team_wgs = 0;
     b->plan_grid = b->ninst;
+    int rc = FVG_OK;
     switch (block) {
-    case 64: launch_bs<64>(b, p); break;
-    case 128: launch_bs<128>(b, p); break;
-    case 256: launch_bs<256>(b, p); break;
-    case 512: launch_bs<512>(b, p); break;
-    case 768: launch_bs<768>(b, p); break;
-    default: launch_bs<1024>(b, p); break;
+    case 64: rc = launch_bs<64>(b, p); break;
+    case 128: rc = launch_bs<128>(b, p); break;
+    case 256: rc = launch_bs<256>(b, p); break;
+    case 512: rc = launch_bs<512>(b, p); break;
+    case 768: rc = launch_bs<768>(b, p); break;
+    default: rc = launch_bs<1024>(b, p); break;
     }
+    if (rc) return rc;
     BCHK(b, hipGetLastError());
     return FVG_OK;
 }
@@ -1319,6 +1829,9 @@ int fvg_batch_create(const fvg_config* cfg_in, int ninst, const int* ncells, int
         hipMalloc(&b->d_queue, sizeof(int) * ninst) != hipSuccess || hipMalloc(&b->d_qnext, sizeof(unsigned)) != hipSuccess ||
         hipMalloc(&b->d_sync, sizeof(TeamSync) * ninst) != hipSuccess)
         return fail(FVG_ENOMEM, "hipMalloc of the ensemble buffers");
+    b->lds_cap = lds_cells(b);
+    if (b->lds_cap && hipMalloc(&b->d_txch, sizeof(TeamXch) * ninst) != hipSuccess)
+        return fail(FVG_ENOMEM, "hipMalloc of the ensemble buffers");
     int coop = 0;
     if (hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, device) == hipSuccess) b->coop = coop != 0;
     b->cost.assign(ninst, 0.0);
@@ -1344,6 +1857,8 @@ int fvg_batch_create(const fvg_config* cfg_in, int ninst, const int* ncells, int
     p.F = b->F;
     p.inst = b->d_inst;
     p.order = b->d_order;
+    p.cap = b->lds_cap;
+    p.ir = kp.ir;
     p.out = b->d_out;
     *out = b;
     return FVG_OK;
@@ -1551,6 +2066,7 @@ int fvg_batch_set_teams(fvg_batch* b, int max_team, int min_chunk, int force) {
     b->max_team = max_team;
     b->min_chunk = min_chunk;
     b->force_teams = force ? 1 : 0;
+    b->teams_set = true;
     return FVG_OK;
 }
 
