@@ -24,6 +24,7 @@ template <int NV, bool PER, typename T> __global__ void k_cells(KP);
 template <typename T> __global__ void k_cells_march(KP);
 template <int NV> __global__ void k_hancock(KP);
 template <int NV, int D, int MODE, int RECON, bool PER, typename T> __global__ void k_faces(KP);
+template <int MODE, int WHAT, bool PER, typename T> __global__ void k_xlast(KP, int, const double*, const double*, double*);
 template <int NV, int UPD, typename T> __global__ void k_update(KP, const double*, const double*, double*);
 template <int NV, int WHAT> __global__ void k_totals_partial(const double*, long long, double*);
 template <int NV, int D, int USE, bool PER, typename T> __global__ void k_faces_learned(KP);
@@ -272,9 +273,9 @@ int launch_faces_learned(fvg_ctx* c, const KP& p, bool reuse) {
 }
 
 // reuse (learned indicator, Runge-Kutta stages 2 and 3): the faces take the decisions the network made on the step's
-// first stage instead of running it again
+// first stage instead of running it again. no_x: the x faces are left to k_xlast (modes plain and learned).
 template <int NV, typename T>
-int enqueue_residual_nv(fvg_ctx* c, const double* Uin, int mode, bool audit, bool reuse) {
+int enqueue_residual_nv(fvg_ctx* c, const double* Uin, int mode, bool audit, bool reuse, bool no_x = false) {
     const KP p = make_kp(c, Uin);
     int rc;
     if ((rc = enqueue_massflow(c, p))) return rc;
@@ -288,7 +289,8 @@ int enqueue_residual_nv(fvg_ctx* c, const double* Uin, int mode, bool audit, boo
             if constexpr (NV == 5)
                 if ((rc = LFACES(k_audit, FAM_AUDIT, 2, grid_for(c->nfa[2]), kBlock))) return rc;
         }
-        if ((rc = launch_faces_learned<NV, 0, T>(c, p, reuse)) || (rc = launch_faces_learned<NV, 1, T>(c, p, reuse))) return rc;
+        if (!no_x && (rc = launch_faces_learned<NV, 0, T>(c, p, reuse))) return rc;
+        if ((rc = launch_faces_learned<NV, 1, T>(c, p, reuse))) return rc;
         if constexpr (NV == 5)
             if ((rc = launch_faces_learned<NV, 2, T>(c, p, reuse))) return rc;
 #undef LFACES
@@ -320,7 +322,8 @@ int enqueue_residual_nv(fvg_ctx* c, const double* Uin, int mode, bool audit, boo
     if (mode == MODE_HANCOCK)
         if ((rc = launch(c, FAM_HANCOCK, [&] { hipLaunchKernelGGL(k_hancock<NV>, dim3(grid_for(c->nc)), dim3(kBlock), 0, c->stream, p); })))
             return rc;
-    if ((rc = launch_faces<NV, 0, T>(c, p, mode)) || (rc = launch_faces<NV, 1, T>(c, p, mode))) return rc;
+    if (!no_x && (rc = launch_faces<NV, 0, T>(c, p, mode))) return rc;
+    if ((rc = launch_faces<NV, 1, T>(c, p, mode))) return rc;
     if constexpr (NV == 5)
         if ((rc = launch_faces<NV, 2, T>(c, p, mode))) return rc;
     return FVG_OK;
@@ -507,10 +510,43 @@ int enqueue_stage_tiles(fvg_ctx* c, const double* Uin, int upd, const double* U0
 #undef STAGE
 }
 
+// whether the x faces of this context's residuals run with the update (k_xlast): 3-D, reconstructed faces
+bool xlast_path(const fvg_ctx* c) {
+    return c->NV == 5 && !c->quad4 && !c->fused && c->cfg.reconstruction != FVG_RECON_NONE;
+}
+template <int MODE, int WHAT, typename T>
+int launch_xlast(fvg_ctx* c, const KP& p, int upd, const double* U0, const double* Ut, double* out) {
+    const dim3 g(xacc_grid(c)), b(kBlock);
+    return launch(c, FAM_FACES_X, [&] {
+        if (p.wrap[0]) hipLaunchKernelGGL((k_xlast<MODE, WHAT, true, T>), g, b, 0, c->stream, p, upd, U0, Ut, out);
+        else hipLaunchKernelGGL((k_xlast<MODE, WHAT, false, T>), g, b, 0, c->stream, p, upd, U0, Ut, out);
+    });
+}
+// One stage of the 3-D residual of Uin (mode plain or learned): stored into out (UPD_RESIDUAL), or combined into the stage
+// output; out is not Uin. reuse as in enqueue_residual_nv.
+template <typename T>
+int enqueue_xlast_t(fvg_ctx* c, const double* Uin, int mode, bool audit, bool reuse, int upd, const double* U0, const double* Ut, double* out) {
+    const KP p = make_kp(c, Uin);
+    int rc;
+    if ((rc = enqueue_residual_nv<5, T>(c, Uin, mode, audit, reuse, true))) return rc;
+    if (mode == MODE_LEARNED)
+        return reuse ? launch_xlast<MODE_LEARNED, LF_KEPT, T>(c, p, upd, U0, Ut, out) : launch_xlast<MODE_LEARNED, LF_STORE, T>(c, p, upd, U0, Ut, out);
+    switch (p.recon) {
+    case FVG_RECON_MUSCL: return launch_xlast<MODE_PLAIN, FVG_RECON_MUSCL, T>(c, p, upd, U0, Ut, out);
+    case FVG_RECON_WENO3: return launch_xlast<MODE_PLAIN, FVG_RECON_WENO3, T>(c, p, upd, U0, Ut, out);
+    default: return launch_xlast<MODE_PLAIN, FVG_RECON_WENO5, T>(c, p, upd, U0, Ut, out);
+    }
+}
+int enqueue_xlast(fvg_ctx* c, const double* Uin, int mode, bool audit, bool reuse, int upd, const double* U0, const double* Ut, double* out) {
+    return c->fp32 ? enqueue_xlast_t<float>(c, Uin, mode, audit, reuse, upd, U0, Ut, out)
+                   : enqueue_xlast_t<double>(c, Uin, mode, audit, reuse, upd, U0, Ut, out);
+}
+
 // The residual of Uin stored into R (Rb for fvg_residual): fused passes, one 2-D stage, or separate face and update passes
 int residual_into(fvg_ctx* c, const double* Uin, int mode, bool audit, double* R) {
     if (mode == MODE_PLAIN && stage_tiles(c)) return enqueue_stage_tiles(c, Uin, UPD_RESIDUAL, nullptr, nullptr, R);
     if (fused_path(c)) return enqueue_fused(c, Uin, mode, audit, false, UPD_RESIDUAL, nullptr, nullptr, R);
+    if (mode != MODE_HANCOCK && xlast_path(c)) return enqueue_xlast(c, Uin, mode, audit, false, UPD_RESIDUAL, nullptr, nullptr, R);
     int rc = enqueue_residual(c, Uin, mode, audit);
     return rc ? rc : enqueue_update(c, UPD_RESIDUAL, nullptr, nullptr, R);
 }
@@ -572,12 +608,15 @@ int enqueue_step(fvg_ctx* c, int link = 0) {
     c->stage = 0;
     const int mode = plain_mode(c);
     if (c->learned && (rc = enqueue_indicator(c, CTL_AUDIT_BEGIN))) return rc;
-    if (fused || stage_tiles(c)) {
+    const bool xlast = xlast_path(c);
+    if (fused || xlast || stage_tiles(c)) {
         // stage 1: R into Rb, dt from its wave speed, then the first update; stages 2-3 finish their combination in
         // the last face pass (the SSP-RK3 stage-2 output goes to Rb, which stage 1's R no longer needs)
         auto stage = [&](int k, const double* Uin, int upd, double* out) {
             c->stage = k;
-            const int r = fused ? enqueue_fused(c, Uin, mode, false, c->learned, upd, c->U, Uin, out) : enqueue_stage_tiles(c, Uin, upd, c->U, Uin, out);
+            const int r = fused   ? enqueue_fused(c, Uin, mode, false, c->learned, upd, c->U, Uin, out)
+                          : xlast ? enqueue_xlast(c, Uin, mode, false, c->learned, upd, c->U, Uin, out)
+                                  : enqueue_stage_tiles(c, Uin, upd, c->U, Uin, out);
             c->stage = 0;
             return r;
         };

@@ -1358,7 +1358,105 @@ __global__ __launch_bounds__(256) void k_update(KP p, const double* __restrict__
 }
 
 // ------------------------------------------------------------------------------------------------------------
-// Fused residual passes (the default kernel sequence): the face fluxes never go to HBM. Every face is computed
+// The x faces and the update of a 3-D stage in one pass, after the y and z faces (k_faces, k_faces_learned): a wavefront
+// holds 64 consecutive faces in face order, the next face's fluxes come from the next lane, and the 63 cells between
+// them take their balance (k_update) and stage combination at once; wavefronts overlap by one face. The x fluxes, 72
+// bytes of a cell in FP64, are neither written nor read again, and the update's memory traffic runs under other
+// wavefronts' FP64 work, which bounds the faces. out is not the stage input (a boundary face reads cells of it).
+// Measured, WENO5-Z viscous: 256^3 FP64 0.92 (x faces) + 1.07 (update) -> 1.41 ms, 192^3 FP32 fluxes 0.183 + 0.220 ->
+// 0.266 ms; with the first stage's k_axpy (0.34 and 0.14 ms) a step takes a tenth less time, at 160 x 64 x 48 a twentieth.
+// The faces in the rows' slab order (row_block) measured the same.
+// upd: the stage, UPD_RESIDUAL (R itself: the step's dt comes from this residual) to UPD_RK3_3.
+// ------------------------------------------------------------------------------------------------------------
+
+// The fluxes of x face f in range form IR as store_face stores them; its wave speed.
+template <int MODE, int WHAT, bool PER, typename T, bool IR>
+__device__ __forceinline__ double xlast_face(const KP& p, bool active, long long f, int i, int j, int k, T* Fc, T* Fv) {
+    T sm = T(0);
+    if constexpr (MODE == MODE_LEARNED) {
+        learned_face<5, 0, WHAT, T, IR, PER>(p, active, f, i, j, k, i, p.nx, Fc, sm);
+        if (!active) return 0.0;
+    } else {
+        if (!active) return 0.0;
+        T UL[5], UR[5];
+        face_states<5, 0, MODE, T, IR, WHAT, PER>(p, i, j, k, i, p.nx, UL, UR);
+        face_flux<5, IR>(p.rs, UL, UR, 0, Fc, sm);
+    }
+    if (p.viscous) viscous_face<5, 0, T, IR, PER>(p, i, j, k, i, p.nx, Fv);
+    if constexpr (std::is_same<T, float>::value) {
+        const float A = float(p.Ax);
+#pragma unroll
+        for (int q = 0; q < 5; ++q) Fc[q] = Fc[q] * A;
+        if (p.viscous)
+#pragma unroll
+            for (int q = 1; q < 5; ++q) Fc[q] -= Fv[q - 1];
+    }
+    return double(sm);
+}
+
+// WHAT: the reconstruction (MODE_PLAIN) or LF_STORE / LF_KEPT (MODE_LEARNED); PER as in k_faces
+template <int MODE, int WHAT, bool PER, typename T>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_xlast(KP p, int upd, const double* __restrict__ U0,
+                                                                                      const double* __restrict__ Ut, double* __restrict__ out) {
+    if (p.st->done) return;   // uniform: the whole grid leaves
+    const long long nf = (long long)(p.nx + 1) * p.ny * p.nz;
+    const int lane = threadIdx.x & 63;
+    const long long f = (xcd_block() * (blockDim.x >> 6) + (threadIdx.x >> 6)) * 63 + lane;
+    const bool active = f < nf;
+    int i = 0, j = 0, k = 0, t;
+    if (active) face_coords<5, 0>(p, f, i, j, k, t);
+    constexpr bool F64 = std::is_same<T, double>::value;
+    T Fc[5] = {}, Fv[4] = {};
+    double local = 0.0;
+    double sm;
+    if (F64 && in_range(p)) sm = xlast_face<MODE, WHAT, PER, T, F64>(p, active, f, i, j, k, Fc, Fv);
+    else sm = xlast_face<MODE, WHAT, PER, T, false>(p, active, f, i, j, k, Fc, Fv);
+    if (sm > local) local = sm;
+    T Gc[5], Gv[4];
+#pragma unroll
+    for (int q = 0; q < 5; ++q) Gc[q] = __shfl_down(Fc[q], 1, 64);
+    if (F64 && p.viscous)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) Gv[q] = __shfl_down(Fv[q], 1, 64);
+    if (active && lane < 63 && i < p.nx) {   // the cell between this face and the next
+        const long long c = cidx(p, i, j, k), plane = (long long)p.nx * p.ny;
+        const long long fy = ((long long)k * (p.ny + 1) + j) * p.nx + i, fz = c;
+        const double dt = p.st->dt;
+#pragma unroll
+        for (int q = 0; q < 5; ++q) {
+            const T* Fy = (const T*)p.Fc[1] + q * p.nfa[1];
+            const T* Fz = (const T*)p.Fc[2] + q * p.nfa[2];
+            double R;
+            if constexpr (F64) {
+                R = (((0.0 - (Gc[q] * p.Ax - Fc[q] * p.Ax)) - (Fy[fy + p.nx] * p.Ay - Fy[fy] * p.Ay)) - (Fz[fz + plane] * p.Az - Fz[fz] * p.Az)) *
+                    p.inv_vol;
+                if (p.viscous) {
+                    double v = 0.0;   // the zero viscous flux of the density slot
+                    if (q > 0) {
+                        const T* Vy = (const T*)p.Fv[1] + (q - 1) * p.nfa[1];
+                        const T* Vz = (const T*)p.Fv[2] + (q - 1) * p.nfa[2];
+                        v = (((0.0 + (Gv[q > 0 ? q - 1 : 0] - Fv[q > 0 ? q - 1 : 0])) + (Vy[fy + p.nx] - Vy[fy])) + (Vz[fz + plane] - Vz[fz])) * p.inv_vol;
+                    }
+                    R = R + v;
+                }
+            } else {
+                double d = (double(Gc[q]) - double(Fc[q])) + (double(Fy[fy + p.nx]) - double(Fy[fy]));
+                d += double(Fz[fz + plane]) - double(Fz[fz]);
+                R = -d * p.inv_vol;
+            }
+            const long long x = q * p.nc + c;
+            double o = R;
+            if (upd == UPD_RK2_2) o = 0.5 * U0[x] + 0.5 * (Ut[x] + dt * R);
+            else if (upd == UPD_RK3_2) o = 0.75 * U0[x] + 0.25 * (Ut[x] + dt * R);
+            else if (upd == UPD_RK3_3) o = (1.0 / 3.0) * U0[x] + (2.0 / 3.0) * (Ut[x] + dt * R);
+            out[x] = o;
+        }
+    }
+    block_max_slot(p, local, SPD_CONV);
+}
+
+// ------------------------------------------------------------------------------------------------------------
+// Fused residual passes (opt-in, fvg_set_fused): the face fluxes never go to HBM. Every face is computed
 // once (up to one face per line segment or wavefront) and its difference with the next face of the same axis is
 // added at once to the cell between them, in the reference's order of the divergence (Simulation.cpp:1022-1037,
 // 1293-1310; viscous balance Physics.cpp:196-204, 746-752):
