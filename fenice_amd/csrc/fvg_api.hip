@@ -41,10 +41,9 @@ __global__ void k_totals_final(const double*, int, long long, int, double*);
 __global__ void k_control(KP, int, int);
 __global__ void k_set_state(DevState*, DevState);
 __global__ void k_publish_state(const DevState*, DevState*);
-__global__ void k_massflow(KP);
+template <int NV> __global__ void k_sides(KP, int);
 __global__ void k_hancock_step2d(KP, const double*, double*);
 template <int RECON, bool VISC, bool PER> __global__ void k_stage2d(KP, int, const double*, const double*, double*);
-template <int NV, int SIDE> __global__ void k_nrbc(KP);
 __global__ void k_riemann_batch(RiemannParams, const double*, const double*, const int*, long long, double*, double*);
 }   // namespace fvg
 
@@ -111,8 +110,8 @@ struct fvg_ctx {
     hipGraphExec_t graph[2] = {nullptr, nullptr};
     int parity = 0;                    // swaps of U and Ut so far, mod 2
     bool quad4 = false;                // flux_quadrature = fourth
-    bool massflow = false;             // a mass-flow inlet side: k_massflow runs before every k_cells
-    int nrbc_sides = 0;                // bit s: side s is non-reflecting (k_nrbc runs for it before every k_cells)
+    bool massflow = false;             // a mass-flow inlet side: k_sides runs before every k_cells
+    int nrbc_sides = 0;                // bit s: side s is non-reflecting (k_sides runs for it before every k_cells)
     double* nrbc = nullptr;            // KP::nrbc
     double *Wc = nullptr, *q4_UL = nullptr, *q4_UR = nullptr, *q4_Fp = nullptr;
     unsigned char *q4_good = nullptr, *q4_pt = nullptr;
@@ -196,35 +195,17 @@ KP make_kp(fvg_ctx* c, const double* Uin) {
 
 // the mass-flow targets and the non-reflecting ghosts of the stage input, which the ghost states of k_cells and the
 // face passes read
-int enqueue_massflow(fvg_ctx* c, const KP& p) {
-    int rc = FVG_OK;
-    if (c->massflow && (rc = launch(c, FAM_CONTROL, [&] { hipLaunchKernelGGL(k_massflow, dim3(6), dim3(1024), 0, c->stream, p); })))
-        return rc;
-    for (int s = 0; s < 6 && !rc; ++s) {
-        if (!(c->nrbc_sides >> s & 1)) continue;
-        const long long n = s < 2 ? (long long)c->cfg.ny * c->cfg.nz : (s < 4 ? (long long)c->cfg.nx * c->cfg.nz : (long long)c->cfg.nx * c->cfg.ny);
-        const dim3 g(grid_for(n)), b(kBlock);
-        rc = launch(c, FAM_CONTROL, [&] {
-            if (c->NV == 4) {
-                switch (s) {
-                case 0: hipLaunchKernelGGL((k_nrbc<4, 0>), g, b, 0, c->stream, p); break;
-                case 1: hipLaunchKernelGGL((k_nrbc<4, 1>), g, b, 0, c->stream, p); break;
-                case 2: hipLaunchKernelGGL((k_nrbc<4, 2>), g, b, 0, c->stream, p); break;
-                default: hipLaunchKernelGGL((k_nrbc<4, 3>), g, b, 0, c->stream, p); break;
-                }
-            } else {
-                switch (s) {
-                case 0: hipLaunchKernelGGL((k_nrbc<5, 0>), g, b, 0, c->stream, p); break;
-                case 1: hipLaunchKernelGGL((k_nrbc<5, 1>), g, b, 0, c->stream, p); break;
-                case 2: hipLaunchKernelGGL((k_nrbc<5, 2>), g, b, 0, c->stream, p); break;
-                case 3: hipLaunchKernelGGL((k_nrbc<5, 3>), g, b, 0, c->stream, p); break;
-                case 4: hipLaunchKernelGGL((k_nrbc<5, 4>), g, b, 0, c->stream, p); break;
-                default: hipLaunchKernelGGL((k_nrbc<5, 5>), g, b, 0, c->stream, p); break;
-                }
-            }
-        });
-    }
-    return rc;
+int enqueue_sides(fvg_ctx* c, const KP& p) {
+    if (!c->massflow && !c->nrbc_sides) return FVG_OK;
+    long long n = 1;   // the boundary cells of the largest non-reflecting side
+    for (int s = 0; s < 6; ++s)
+        if (c->nrbc_sides >> s & 1)
+            n = std::max(n, s < 2 ? (long long)c->cfg.ny * c->cfg.nz : (s < 4 ? (long long)c->cfg.nx * c->cfg.nz : (long long)c->cfg.nx * c->cfg.ny));
+    const dim3 g(grid_for(n), c->NV == 5 ? 6 : 4);
+    return launch(c, FAM_CONTROL, [&] {
+        if (c->NV == 5) hipLaunchKernelGGL(k_sides<5>, g, dim3(kBlock), 0, c->stream, p, c->nrbc_sides);
+        else hipLaunchKernelGGL(k_sides<4>, g, dim3(kBlock), 0, c->stream, p, c->nrbc_sides);
+    });
 }
 
 // the primitives and gradients, in the variant of the mesh's sides
@@ -278,7 +259,7 @@ template <int NV, typename T>
 int enqueue_residual_nv(fvg_ctx* c, const double* Uin, int mode, bool audit, bool reuse, bool no_x = false) {
     const KP p = make_kp(c, Uin);
     int rc;
-    if ((rc = enqueue_massflow(c, p))) return rc;
+    if ((rc = enqueue_sides(c, p))) return rc;
     if ((rc = launch_cells<NV, T>(c, p))) return rc;
     if (mode == MODE_LEARNED) {
 #define LFACES(KERNEL, FAM, D, GRID, BLOCK) \
@@ -343,7 +324,7 @@ template <int NV>
 int enqueue_hancock_residual(fvg_ctx* c, const double* Uin) {
     const KP p = make_kp(c, Uin);
     int rc;
-    if ((rc = enqueue_massflow(c, p))) return rc;
+    if ((rc = enqueue_sides(c, p))) return rc;
     if ((rc = launch_cells<NV, double>(c, p))) return rc;
     if ((rc = launch(c, FAM_HANCOCK, [&] { hipLaunchKernelGGL(k_hancock<NV>, dim3(grid_for(c->nc)), dim3(kBlock), 0, c->stream, p); })))
         return rc;
@@ -442,7 +423,7 @@ int enqueue_fused_nv(fvg_ctx* c, const double* Uin, int mode, bool audit, bool r
                      double* out) {
     const KP p = make_kp(c, Uin);
     int rc;
-    if ((rc = enqueue_massflow(c, p))) return rc;
+    if ((rc = enqueue_sides(c, p))) return rc;
     if ((rc = launch_cells<NV, T>(c, p))) return rc;
     if constexpr (std::is_same<T, double>::value) {
         if (mode == MODE_HANCOCK) {
@@ -497,7 +478,7 @@ bool stage_tiles(const fvg_ctx* c) {
 int enqueue_stage_tiles(fvg_ctx* c, const double* Uin, int upd, const double* U0, const double* Ut, double* out) {
     const KP p = make_kp(c, Uin);
     int rc;
-    if ((rc = enqueue_massflow(c, p))) return rc;
+    if ((rc = enqueue_sides(c, p))) return rc;
     const dim3 g((c->cfg.nx + kStageTile - 1) / kStageTile, (c->cfg.ny + kStageTile - 1) / kStageTile);
     auto go = [&](auto kernel) { return launch(c, FAM_STAGE2D, [&] { hipLaunchKernelGGL(kernel, g, dim3(512), 0, c->stream, p, upd, U0, Ut, out); }); };
     const bool per = p.wrap[0] && p.wrap[1], visc = p.viscous != 0;
@@ -1355,7 +1336,7 @@ int fvg_indicator_samples(fvg_ctx* c, int axis, float* X, float* dep, long long 
     KP p = make_kp(c, c->U);
     p.viscous = 0;   // only the primitives are needed: no gradients, and no speed maxima left behind in the slots
     const dim3 gc(cells_grid(c)), bc(cells_block(c)), gf((unsigned)((nfaces + kBlock - 1) / kBlock)), b(kBlock);
-    if (int rc = enqueue_massflow(c, p)) {
+    if (int rc = enqueue_sides(c, p)) {
         hipFree(dX);
         hipFree(dd);
         return rc;

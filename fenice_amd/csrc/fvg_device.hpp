@@ -434,7 +434,7 @@ __device__ __forceinline__ int bc_of(const BcParams& b, int side) {
 }
 
 // side: 0 left, 1 right, 2 bottom, 3 top, 4 front, 5 back. Periodic and non-reflecting sides never reach here; a
-// mass-flow side reads its target velocity from b.ut (set by k_massflow before the residual's first pass).
+// mass-flow side reads its target velocity from b.ut (set by k_sides before the residual's first pass).
 template <int NV>
 __device__ __forceinline__ void ghost_state(const Eos& e, const BcParams& b, int side, const double* Ui, double* Ug) {
     const int bc = bc_of(b, side);

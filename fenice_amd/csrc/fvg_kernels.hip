@@ -31,34 +31,22 @@ __device__ __forceinline__ void end_step(DevState* s) {
     }
 }
 
-template __global__ void k_nrbc<4, 0>(KP);
-template __global__ void k_nrbc<4, 1>(KP);
-template __global__ void k_nrbc<4, 2>(KP);
-template __global__ void k_nrbc<4, 3>(KP);
-template __global__ void k_nrbc<5, 0>(KP);
-template __global__ void k_nrbc<5, 1>(KP);
-template __global__ void k_nrbc<5, 2>(KP);
-template __global__ void k_nrbc<5, 3>(KP);
-template __global__ void k_nrbc<5, 4>(KP);
-template __global__ void k_nrbc<5, 5>(KP);
-
-// The mass-flow inlet velocity of every mass-flow side (apply_side, Boundaries.cpp:285-294): rho_in u_in over the
-// mean density of the side's boundary cells, floored at 1e-5. One block of kMassflowThreads per side; the densities
-// are summed in the reference's boundary order (Core.hpp:121-151) by one thread, a chunk of kMassflowChunk values
-// loaded into LDS by the whole block at a time, so that the sum has the reference's bits. The result goes to
-// DevState::ut, which the ghost states of the residual read.
-constexpr int kMassflowThreads = 1024, kMassflowChunk = 4096;
-__global__ __launch_bounds__(kMassflowThreads) void k_massflow(KP p) {
-    __shared__ double rho[kMassflowChunk];
-    const int side = blockIdx.x;
-    if (bc_of(p.bp, side) != 4 || (side >= 4 && !p.is3d) || p.st->done) return;   // uniform over the block
+// The mass-flow inlet velocity of a mass-flow side (apply_side, Boundaries.cpp:285-294): rho_in u_in over the mean
+// density of the side's boundary cells, floored at 1e-5, into DevState::ut, which the ghost states of the residual read.
+// The densities are summed in the reference's boundary order (Core.hpp:121-151) by one thread, so that the sum has the
+// reference's bits: a chain of n dependent additions, about 17 cycles each. The block loads a chunk into LDS at a time
+// and the thread reads the next values into registers while it adds the ones before them. 64 x 48 boundary cells: 30 us
+// when the additions waited for the reads and 6 for the launch of the non-reflecting side, 26 for both now.
+constexpr int kMassflowChunk = 4096, kMassflowAhead = 32;
+__device__ void massflow_side(const KP& p, int side, double* rho) {
     const long long nx = p.nx, ny = p.ny, nz = p.nz;
     const long long n = side < 2 ? ny * nz : (side < 4 ? nx * nz : nx * ny);
     double sum = 0.0;
     for (long long base = 0; base < n; base += kMassflowChunk) {
-        for (int l = threadIdx.x; l < kMassflowChunk; l += blockDim.x) {
+        const int m = n - base < kMassflowChunk ? (int)(n - base) : kMassflowChunk;
+        const int whole = (m + 2 * kMassflowAhead - 1) / (2 * kMassflowAhead) * (2 * kMassflowAhead);
+        for (int l = threadIdx.x; l < whole + kMassflowAhead; l += blockDim.x) {
             const long long k = base + l;
-            if (k >= n) break;
             long long c;
             switch (side) {
             case 0: c = k * nx; break;
@@ -68,13 +56,24 @@ __global__ __launch_bounds__(kMassflowThreads) void k_massflow(KP p) {
             case 4: c = k; break;
             default: c = (nz - 1) * ny * nx + k; break;
             }
-            rho[l] = smax(p.U[c], kEosEps);   // the density of cons_to_prim
+            rho[l] = l < m ? smax(p.U[c], kEosEps) : 0.0;   // the density of cons_to_prim; + 0 leaves the sum as it is
         }
         __syncthreads();
         if (threadIdx.x == 0) {
-            const int m = n - base < kMassflowChunk ? (int)(n - base) : kMassflowChunk;
-#pragma unroll 16
-            for (int l = 0; l < m; ++l) sum += rho[l];   // in order: the loads run ahead of the chain of adds
+            double a[kMassflowAhead], b[kMassflowAhead];
+#pragma unroll
+            for (int q = 0; q < kMassflowAhead; ++q) a[q] = rho[q];
+#pragma unroll 1
+            for (int l = 0; l < whole; l += 2 * kMassflowAhead) {
+#pragma unroll
+                for (int q = 0; q < kMassflowAhead; ++q) b[q] = rho[l + kMassflowAhead + q];
+#pragma unroll
+                for (int q = 0; q < kMassflowAhead; ++q) sum += a[q];
+#pragma unroll
+                for (int q = 0; q < kMassflowAhead; ++q) a[q] = rho[l + 2 * kMassflowAhead + q];
+#pragma unroll
+                for (int q = 0; q < kMassflowAhead; ++q) sum += b[q];
+            }
         }
         __syncthreads();
     }
@@ -83,6 +82,33 @@ __global__ __launch_bounds__(kMassflowThreads) void k_massflow(KP p) {
         p.st->ut[side] = (p.bp.rho_in * p.bp.u_in) / rho_avg;
     }
 }
+
+// What the sides need before a residual's first pass, from the stage input: block (0, s) the target velocity of a
+// mass-flow side s, blocks (x, s) the ghosts of a non-reflecting side's boundary cells (bit s of nrbc).
+template <int NV>
+__global__ __launch_bounds__(256) void k_sides(KP p, int nrbc) {
+    __shared__ double rho[kMassflowChunk + kMassflowAhead];
+    if (p.st->done) return;
+    const int side = blockIdx.y;
+    if (!(nrbc >> side & 1)) {
+        if (blockIdx.x == 0 && bc_of(p.bp, side) == 4) massflow_side(p, side, rho);
+        return;
+    }
+    switch (side) {
+    case 0: nrbc_cell<NV, 0>(p); break;
+    case 1: nrbc_cell<NV, 1>(p); break;
+    case 2: nrbc_cell<NV, 2>(p); break;
+    case 3: nrbc_cell<NV, 3>(p); break;
+    case 4:
+        if constexpr (NV == 5) nrbc_cell<NV, 4>(p);
+        break;
+    default:
+        if constexpr (NV == 5) nrbc_cell<NV, 5>(p);
+        break;
+    }
+}
+template __global__ void k_sides<4>(KP, int);
+template __global__ void k_sides<5>(KP, int);
 
 // The maximum over the 64 slots of one quantity (bit patterns of non-negative doubles order as integers); clears them.
 // Every lane of the wavefront calls it and gets the maximum.

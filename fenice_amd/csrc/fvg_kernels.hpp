@@ -22,7 +22,7 @@ struct DevState {
     double s1, s2, s3, s_step, lagged;
     long long reverted;
     int done, diverged, steps, max_steps;
-    double ut[6];   // mass-flow inlet velocity per side of the current residual (k_massflow)
+    double ut[6];   // mass-flow inlet velocity per side of the current residual (k_sides)
     // nonzero: a value k_cells stored for the residual's stencils (a primitive of the FP64 planes or, with the
     // fourth-order quadrature, a value of the padded conservative planes) is outside value_in_range, so the kernels
     // take the IEEE divisions and roots. k_cells only sets it; k_update (the end of every residual of the separate
@@ -100,7 +100,7 @@ struct KP {
     double *q4_UL, *q4_UR, *q4_Fp;
     unsigned char *q4_good, *q4_pt;
     long long q4_n;
-    // non-reflecting sides: the ghost state of each boundary cell of the stage input (k_nrbc), NV planes per side
+    // non-reflecting sides: the ghost state of each boundary cell of the stage input (k_sides), NV planes per side
     // of the side's boundary cells, side s from element nrbc_off[s] (null without such a side)
     double* nrbc;
     long long nrbc_off[6];

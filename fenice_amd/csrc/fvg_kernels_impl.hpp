@@ -140,7 +140,7 @@ __device__ __forceinline__ void stencil_prim(const KP& p, int d, int i, int j, i
 // neighbours of apply_side, Boundaries.cpp:155-198, 314-360): a characteristic outlet whose ghost differs from the
 // cell only in the incoming acoustic wave, relaxed towards p_out with the transverse terms weighted by 1 - beta.
 // Tangential derivatives are central differences of the primitives, wrapped across a periodic axis, one-sided at
-// the ends of the others. k_nrbc computes it once per stage into the side's plane of KP::nrbc, which the face
+// the ends of the others. k_sides computes it once per stage into the side's plane of KP::nrbc, which the face
 // kernels read.
 template <int NV, int SIDE>
 __device__ __forceinline__ void nrbc_ghost(const KP& p, int i, int j, int k, double* ug) {
@@ -233,7 +233,7 @@ __device__ __forceinline__ void outside_first_order(const KP& p, int d, int side
         load_cons<NV>(p, cidx_d(p, d, i, j, k, (side & 1) ? 0 : ncell(p, d) - 1), ug);
         return;
     }
-    if (bc == 8) {   // the non-reflecting ghost k_nrbc stored for this boundary cell
+    if (bc == 8) {   // the non-reflecting ghost k_sides stored for this boundary cell
         const long long n = side_cells(p, side), kb = side_index(p, side, i, j, k);
         const double* g = p.nrbc + nrbc_off_of(p, side);
 #pragma unroll
@@ -619,12 +619,12 @@ __global__ __launch_bounds__(256) void k_cells_march(KP p) {
     block_max_slot(p, local, SPD_VISC);
 }
 
-// k_nrbc: the non-reflecting ghosts of side SIDE's boundary cells (thread per cell, in the side's boundary order),
-// from the stage input, before the passes that read them
+// the non-reflecting ghosts of side SIDE's boundary cells (thread per cell, in the side's boundary order), from the stage
+// input, before the passes that read them (k_sides)
 template <int NV, int SIDE>
-__global__ __launch_bounds__(256) void k_nrbc(KP p) {
+__device__ __forceinline__ void nrbc_cell(const KP& p) {
     const long long n = side_cells(p, SIDE), kb = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (kb >= n || p.st->done) return;
+    if (kb >= n) return;
     int i, j, k;
     if (SIDE < 2) {
         i = SIDE == 0 ? 0 : p.nx - 1;
