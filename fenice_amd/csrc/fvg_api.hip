@@ -35,7 +35,8 @@ template <int NV, int D, typename T> __global__ void k_audit(KP);
 template <int NV, int D, typename T> __global__ void k_samples(KP, float*, float*);
 template <int NV, int D, int R> __global__ void k4_states(KP);
 template <int NV, int D> __global__ void k4_points(KP);
-template <int NV, int D> __global__ void k4_fluxes(KP);
+template <int NV, int D, bool PER> __global__ void k4_fluxes(KP);
+template <bool PER> __global__ void k4_xlast(KP, int, const double*, const double*, double*);
 __global__ void k_indicator_control(KP, int);
 __global__ void k_totals_final(const double*, int, long long, int, double*);
 __global__ void k_control(KP, int, int);
@@ -233,10 +234,15 @@ int launch_faces(fvg_ctx* c, const KP& p, int mode) {
         return launch(c, FAM_FACES_X + D, [&] {
             hipLaunchKernelGGL((k_faces<NV, D, MODE_FIRST_ORDER, 0, false, T>), dim3(faces_grid(c, D)), dim3(faces_block(c, D)), 0, c->stream, p);
         });
-    switch (p.recon) {
-    case FVG_RECON_MUSCL: return launch_faces_recon<NV, D, MODE_PLAIN, FVG_RECON_MUSCL, T>(c, p);
-    case FVG_RECON_WENO3: return launch_faces_recon<NV, D, MODE_PLAIN, FVG_RECON_WENO3, T>(c, p);
-    default: return launch_faces_recon<NV, D, MODE_PLAIN, FVG_RECON_WENO5, T>(c, p);
+    if constexpr (NV == 5 && D == 0) {   // the seed residual of a MUSCL-Hancock run; k_xlast takes the others
+        if constexpr (std::is_same<T, double>::value) return launch_faces_recon<NV, D, MODE_PLAIN, FVG_RECON_MUSCL, T>(c, p);
+        else return set_err(c, FVG_ELOGIC, "no separate x faces");
+    } else {
+        switch (p.recon) {
+        case FVG_RECON_MUSCL: return launch_faces_recon<NV, D, MODE_PLAIN, FVG_RECON_MUSCL, T>(c, p);
+        case FVG_RECON_WENO3: return launch_faces_recon<NV, D, MODE_PLAIN, FVG_RECON_WENO3, T>(c, p);
+        default: return launch_faces_recon<NV, D, MODE_PLAIN, FVG_RECON_WENO5, T>(c, p);
+        }
     }
 }
 template <int NV, int D, typename T>
@@ -254,7 +260,8 @@ int launch_faces_learned(fvg_ctx* c, const KP& p, bool reuse) {
 }
 
 // reuse (learned indicator, Runge-Kutta stages 2 and 3): the faces take the decisions the network made on the step's
-// first stage instead of running it again. no_x: the x faces are left to k_xlast (modes plain and learned).
+// first stage instead of running it again. no_x: the plain x faces are left to k_xlast, as the
+// learned and fourth-order x fluxes of a 3-D mesh always are (k_xlast, k4_xlast).
 template <int NV, typename T>
 int enqueue_residual_nv(fvg_ctx* c, const double* Uin, int mode, bool audit, bool reuse, bool no_x = false) {
     const KP p = make_kp(c, Uin);
@@ -270,7 +277,8 @@ int enqueue_residual_nv(fvg_ctx* c, const double* Uin, int mode, bool audit, boo
             if constexpr (NV == 5)
                 if ((rc = LFACES(k_audit, FAM_AUDIT, 2, grid_for(c->nfa[2]), kBlock))) return rc;
         }
-        if (!no_x && (rc = launch_faces_learned<NV, 0, T>(c, p, reuse))) return rc;
+        if constexpr (NV == 4)
+            if ((rc = launch_faces_learned<NV, 0, T>(c, p, reuse))) return rc;
         if ((rc = launch_faces_learned<NV, 1, T>(c, p, reuse))) return rc;
         if constexpr (NV == 5)
             if ((rc = launch_faces_learned<NV, 2, T>(c, p, reuse))) return rc;
@@ -287,13 +295,26 @@ int enqueue_residual_nv(fvg_ctx* c, const double* Uin, int mode, bool audit, boo
         if (w5) hipLaunchKernelGGL((k4_states<NV, D, 3>), dim3(grid_for(c->nfa[D])), dim3(kBlock), 0, c->stream, p); \
         else hipLaunchKernelGGL((k4_states<NV, D, 2>), dim3(grid_for(c->nfa[D])), dim3(kBlock), 0, c->stream, p);    \
     })
+#define Q4_FLUXES(D)                                                                                                           \
+    launch(c, FAM_Q4_FLUXES, [&] {                                                                                             \
+        if (p.wrap[D]) hipLaunchKernelGGL((k4_fluxes<NV, D, true>), dim3(grid_for(c->nfa[D])), dim3(kBlock), 0, c->stream, p); \
+        else hipLaunchKernelGGL((k4_fluxes<NV, D, false>), dim3(grid_for(c->nfa[D])), dim3(kBlock), 0, c->stream, p);          \
+    })
+#define Q4_POINTS(D) \
+    if ((rc = Q4_STATES(D)) || (rc = Q4(k4_points, FAM_Q4_POINTS, D))) return rc;
 #define Q4_AXIS(D) \
-    if ((rc = Q4_STATES(D)) || (rc = Q4(k4_points, FAM_Q4_POINTS, D)) || (rc = Q4(k4_fluxes, FAM_Q4_FLUXES, D))) return rc;
-            Q4_AXIS(0)
-            Q4_AXIS(1)
-            if constexpr (NV == 5) {
+    Q4_POINTS(D)   \
+    if ((rc = Q4_FLUXES(D))) return rc;
+            if constexpr (NV == 4) {
+                Q4_AXIS(0)
+                Q4_AXIS(1)
+            } else {   // the x faces last, for k4_xlast: the axes share their buffers
+                Q4_AXIS(1)
                 Q4_AXIS(2)
+                Q4_POINTS(0)
             }
+#undef Q4_POINTS
+#undef Q4_FLUXES
 #undef Q4_AXIS
 #undef Q4_STATES
 #undef Q4
@@ -491,9 +512,9 @@ int enqueue_stage_tiles(fvg_ctx* c, const double* Uin, int upd, const double* U0
 #undef STAGE
 }
 
-// whether the x faces of this context's residuals run with the update (k_xlast): 3-D, reconstructed faces
+// whether the x faces of this context's residuals run with the update (k_xlast, k4_xlast): 3-D, reconstructed faces
 bool xlast_path(const fvg_ctx* c) {
-    return c->NV == 5 && !c->quad4 && !c->fused && c->cfg.reconstruction != FVG_RECON_NONE;
+    return c->NV == 5 && !fused_path(c) && c->cfg.reconstruction != FVG_RECON_NONE;
 }
 template <int MODE, int WHAT, typename T>
 int launch_xlast(fvg_ctx* c, const KP& p, int upd, const double* U0, const double* Ut, double* out) {
@@ -503,13 +524,20 @@ int launch_xlast(fvg_ctx* c, const KP& p, int upd, const double* U0, const doubl
         else hipLaunchKernelGGL((k_xlast<MODE, WHAT, false, T>), g, b, 0, c->stream, p, upd, U0, Ut, out);
     });
 }
-// One stage of the 3-D residual of Uin (mode plain or learned): stored into out (UPD_RESIDUAL), or combined into the stage
+// One stage of the 3-D residual of Uin (mode plain, learned or fourth): stored into out (UPD_RESIDUAL), or combined into the stage
 // output; out is not Uin. reuse as in enqueue_residual_nv.
 template <typename T>
 int enqueue_xlast_t(fvg_ctx* c, const double* Uin, int mode, bool audit, bool reuse, int upd, const double* U0, const double* Ut, double* out) {
     const KP p = make_kp(c, Uin);
     int rc;
     if ((rc = enqueue_residual_nv<5, T>(c, Uin, mode, audit, reuse, true))) return rc;
+    if constexpr (std::is_same<T, double>::value)
+        if (mode == MODE_FOURTH)
+            return launch(c, FAM_Q4_FLUXES, [&] {
+                const dim3 g(xacc_grid(c)), b(kBlock);
+                if (p.wrap[0]) hipLaunchKernelGGL(k4_xlast<true>, g, b, 0, c->stream, p, upd, U0, Ut, out);
+                else hipLaunchKernelGGL(k4_xlast<false>, g, b, 0, c->stream, p, upd, U0, Ut, out);
+            });
     if (mode == MODE_LEARNED)
         return reuse ? launch_xlast<MODE_LEARNED, LF_KEPT, T>(c, p, upd, U0, Ut, out) : launch_xlast<MODE_LEARNED, LF_STORE, T>(c, p, upd, U0, Ut, out);
     switch (p.recon) {

@@ -25,7 +25,7 @@ template __global__ void k_cells_march<float>(KP);
     template __global__ void k_faces<NV, D, MODE_FIRST_ORDER, 0, false, float>(KP);
 FVG_AXIS(4, 0)
 FVG_AXIS(4, 1)
-FVG_AXIS(5, 0)
+template __global__ void k_faces<5, 0, MODE_FIRST_ORDER, 0, false, float>(KP);   // k_xlast takes the others
 FVG_AXIS(5, 1)
 FVG_AXIS(5, 2)
 

@@ -56,6 +56,24 @@ template <int NV, int D> struct Trans {
     static constexpr int t1 = D == 2 ? 1 : 2;
 };
 
+// the transverse neighbours of face f (f itself where there is none), and whether all are there and flagged as f is. All
+// flags are read at once: a chain of reads, each waiting for the flag before it, is what these short passes would wait for.
+template <int NV, int D>
+__device__ __forceinline__ bool q4_neighbours(const KP& p, const unsigned char* flag, long long f, int i, int j, int k, long long (*nb)[2]) {
+    using TR = Trans<NV, D>;
+    const int ct[2] = {coord(TR::t0, i, j, k), coord(TR::t1, i, j, k)};
+    int ok = flag[f];
+#pragma unroll
+    for (int u = 0; u < TR::n; ++u)
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            const long long x = q4_nbr<D>(p, f, ct[u], u ? TR::t1 : TR::t0, 2 * s - 1);
+            nb[u][s] = x < 0 ? f : x;
+            ok &= int(x >= 0) & int(flag[nb[u][s]]);
+        }
+    return ok != 0;
+}
+
 template <int NV>
 __device__ __forceinline__ void q4_load(const double* planes, long long n, long long f, double* u) {
 #pragma unroll
@@ -168,18 +186,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
         q4_load<NV>(p.q4_UL, p.q4_n, f, al);
         q4_load<NV>(p.q4_UR, p.q4_n, f, ar);
         bool pt = false;
-        if (p.q4_good[f]) {
+        {
             long long nb[2][2];
-            const int ct0 = coord(TR::t0, i, j, k), ct1 = coord(TR::t1, i, j, k);
-            nb[0][0] = q4_nbr<D>(p, f, ct0, TR::t0, -1);
-            nb[0][1] = q4_nbr<D>(p, f, ct0, TR::t0, 1);
-            bool ok = nb[0][0] >= 0 && nb[0][1] >= 0 && p.q4_good[nb[0][0]] && p.q4_good[nb[0][1]];
-            if constexpr (TR::n == 2) {
-                nb[1][0] = q4_nbr<D>(p, f, ct1, TR::t1, -1);
-                nb[1][1] = q4_nbr<D>(p, f, ct1, TR::t1, 1);
-                ok = ok && nb[1][0] >= 0 && nb[1][1] >= 0 && p.q4_good[nb[1][0]] && p.q4_good[nb[1][1]];
-            }
-            if (ok) {
+            if (q4_neighbours<NV, D>(p, p.q4_good, f, i, j, k, nb)) {
                 double pl[NV], pr[NV];
 #pragma unroll
                 for (int q = 0; q < NV; ++q) {
@@ -215,35 +224,26 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     block_max_slot(p, local, SPD_CONV);
 }
 
+// the corrected flux of face f
 template <int NV, int D>
-__global__ __launch_bounds__(256) void k4_fluxes(KP p) {
+__device__ __forceinline__ void q4_flux(const KP& p, long long f, int i, int j, int k, double* F) {
     using TR = Trans<NV, D>;
-    const long long f = xcd_block() * blockDim.x + threadIdx.x;
-    if (f >= p.nfa[D] || p.st->done) return;
-    int i, j, k, t;
-    face_coords<NV, D>(p, f, i, j, k, t);
-    double F[NV];
     q4_load<NV>(p.q4_Fp, p.q4_n, f, F);
-    if (p.q4_pt[f]) {
-        long long nb[2][2];
-        const int ct0 = coord(TR::t0, i, j, k), ct1 = coord(TR::t1, i, j, k);
-        nb[0][0] = q4_nbr<D>(p, f, ct0, TR::t0, -1);
-        nb[0][1] = q4_nbr<D>(p, f, ct0, TR::t0, 1);
-        bool full = nb[0][0] >= 0 && nb[0][1] >= 0 && p.q4_pt[nb[0][0]] && p.q4_pt[nb[0][1]];
-        if constexpr (TR::n == 2) {
-            nb[1][0] = q4_nbr<D>(p, f, ct1, TR::t1, -1);
-            nb[1][1] = q4_nbr<D>(p, f, ct1, TR::t1, 1);
-            full = full && nb[1][0] >= 0 && nb[1][1] >= 0 && p.q4_pt[nb[1][0]] && p.q4_pt[nb[1][1]];
-        }
+    long long nb[2][2];
+    const bool pt = p.q4_pt[f] != 0, full = q4_neighbours<NV, D>(p, p.q4_pt, f, i, j, k, nb);
+    double C[NV];   // of the neighbours' fluxes, read with the flags
+#pragma unroll
+    for (int q = 0; q < NV; ++q) {
+        const double* P = p.q4_Fp + q * p.q4_n;
+        double d = 0.0;
+#pragma unroll
+        for (int u = 0; u < TR::n; ++u) d += P[nb[u][1]] - 2.0 * F[q] + P[nb[u][0]];
+        C[q] = d;
+    }
+    if (pt) {
         if (full) {
 #pragma unroll
-            for (int q = 0; q < NV; ++q) {
-                const double* P = p.q4_Fp + q * p.q4_n;
-                double d = 0.0;
-#pragma unroll
-                for (int u = 0; u < TR::n; ++u) d += P[nb[u][1]] - 2.0 * F[q] + P[nb[u][0]];
-                F[q] = F[q] + d / 24.0;
-            }
+            for (int q = 0; q < NV; ++q) F[q] = F[q] + C[q] / 24.0;
         } else {   // a point value without the full correction: the flux of the averaged states
             double ul[NV], ur[NV], sm;
             q4_load<NV>(p.q4_UL, p.q4_n, f, ul);
@@ -251,18 +251,62 @@ __global__ __launch_bounds__(256) void k4_fluxes(KP p) {
             face_flux<NV>(p.rs, ul, ur, D, F, sm);
         }
     }
-    store_face<NV, D, double>(p, f, i, j, k, t, ncell(p, D), F);
 }
+
+// PER as in k_faces: the viscous face flux without boundary code
+template <int NV, int D, bool PER>
+__global__ __launch_bounds__(256) void k4_fluxes(KP p) {
+    const long long f = xcd_block() * blockDim.x + threadIdx.x;
+    if (f >= p.nfa[D] || p.st->done) return;
+    int i, j, k, t;
+    face_coords<NV, D>(p, f, i, j, k, t);
+    double F[NV];
+    q4_flux<NV, D>(p, f, i, j, k, F);
+    if (in_range(p)) store_face<NV, D, double, true, PER>(p, f, i, j, k, t, ncell(p, D), F);
+    else store_face<NV, D, double, false, PER>(p, f, i, j, k, t, ncell(p, D), F);
+}
+
+// the x faces' k4_fluxes with the update, after the other axes (k_xlast). 96^3, a stage's corrected fluxes and update: 153 +
+// 68 -> 177 us, and 7 of the first stage's k_axpy; reading the flags at once (q4_neighbours) is 2 of it and 2 of k4_points.
+template <bool PER>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k4_xlast(KP p, int upd, const double* __restrict__ U0,
+                                                                                       const double* __restrict__ Ut, double* __restrict__ out) {
+    if (p.st->done) return;   // uniform: the whole grid leaves
+    const int lane = threadIdx.x & 63;
+    const long long f = (xcd_block() * (blockDim.x >> 6) + (threadIdx.x >> 6)) * 63 + lane;
+    const bool active = f < p.nfa[0];
+    int i = 0, j = 0, k = 0, t;
+    double F[5] = {}, Fv[4] = {};
+    if (active) {
+        face_coords<5, 0>(p, f, i, j, k, t);
+        q4_flux<5, 0>(p, f, i, j, k, F);
+        if (p.viscous) {
+            if (in_range(p)) viscous_face<5, 0, double, true, PER>(p, i, j, k, i, p.nx, Fv);
+            else viscous_face<5, 0, double, false, PER>(p, i, j, k, i, p.nx, Fv);
+        }
+    }
+    xlast_cell<double>(p, active, lane, i, j, k, F, Fv, upd, U0, Ut, out);
+}
+
 
 #define FVG_INST_Q4(NV, D)                              \
     template __global__ void k4_states<NV, D, 2>(KP); \
     template __global__ void k4_states<NV, D, 3>(KP); \
-    template __global__ void k4_points<NV, D>(KP);    \
-    template __global__ void k4_fluxes<NV, D>(KP);
+    template __global__ void k4_points<NV, D>(KP);
+
+#define FVG_INST_Q4F(NV, D)                              \
+    template __global__ void k4_fluxes<NV, D, true>(KP); \
+    template __global__ void k4_fluxes<NV, D, false>(KP);
 FVG_INST_Q4(4, 0)
 FVG_INST_Q4(4, 1)
 FVG_INST_Q4(5, 0)
 FVG_INST_Q4(5, 1)
 FVG_INST_Q4(5, 2)
+FVG_INST_Q4F(4, 0)
+FVG_INST_Q4F(4, 1)
+FVG_INST_Q4F(5, 1)
+FVG_INST_Q4F(5, 2)
+template __global__ void k4_xlast<true>(KP, int, const double*, const double*, double*);
+template __global__ void k4_xlast<false>(KP, int, const double*, const double*, double*);
 
 }   // namespace fvg

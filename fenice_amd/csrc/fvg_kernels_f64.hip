@@ -25,7 +25,10 @@ template __global__ void k_cells_march<double>(KP);
     template __global__ void k_faces<NV, D, MODE_FIRST_ORDER, 0, false, double>(KP);
 FVG_AXIS(4, 0)
 FVG_AXIS(4, 1)
-FVG_AXIS(5, 0)
+// x faces of a 3-D mesh: first order and the seed of a MUSCL-Hancock run (k_xlast takes the others)
+template __global__ void k_faces<5, 0, MODE_PLAIN, 1, true, double>(KP);
+template __global__ void k_faces<5, 0, MODE_PLAIN, 1, false, double>(KP);
+template __global__ void k_faces<5, 0, MODE_FIRST_ORDER, 0, false, double>(KP);
 FVG_AXIS(5, 1)
 FVG_AXIS(5, 2)
 

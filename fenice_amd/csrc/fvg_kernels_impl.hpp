@@ -1394,24 +1394,12 @@ __device__ __forceinline__ double xlast_face(const KP& p, bool active, long long
     return double(sm);
 }
 
-// WHAT: the reconstruction (MODE_PLAIN) or LF_STORE / LF_KEPT (MODE_LEARNED); PER as in k_faces
-template <int MODE, int WHAT, bool PER, typename T>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_xlast(KP p, int upd, const double* __restrict__ U0,
-                                                                                      const double* __restrict__ Ut, double* __restrict__ out) {
-    if (p.st->done) return;   // uniform: the whole grid leaves
-    const long long nf = (long long)(p.nx + 1) * p.ny * p.nz;
-    const int lane = threadIdx.x & 63;
-    const long long f = (xcd_block() * (blockDim.x >> 6) + (threadIdx.x >> 6)) * 63 + lane;
-    const bool active = f < nf;
-    int i = 0, j = 0, k = 0, t;
-    if (active) face_coords<5, 0>(p, f, i, j, k, t);
+// The cell right of each lane's x face (fluxes Fc, Fv as store_face stores them; the next lane's are the cell's right
+// face): its balance and stage combination. Every lane of the wavefront calls it.
+template <typename T>
+__device__ __forceinline__ void xlast_cell(const KP& p, bool active, int lane, int i, int j, int k, const T* Fc, const T* Fv, int upd,
+                                           const double* __restrict__ U0, const double* __restrict__ Ut, double* __restrict__ out) {
     constexpr bool F64 = std::is_same<T, double>::value;
-    T Fc[5] = {}, Fv[4] = {};
-    double local = 0.0;
-    double sm;
-    if (F64 && in_range(p)) sm = xlast_face<MODE, WHAT, PER, T, F64>(p, active, f, i, j, k, Fc, Fv);
-    else sm = xlast_face<MODE, WHAT, PER, T, false>(p, active, f, i, j, k, Fc, Fv);
-    if (sm > local) local = sm;
     T Gc[5], Gv[4];
 #pragma unroll
     for (int q = 0; q < 5; ++q) Gc[q] = __shfl_down(Fc[q], 1, 64);
@@ -1452,6 +1440,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
             out[x] = o;
         }
     }
+}
+
+// WHAT: the reconstruction (MODE_PLAIN) or LF_STORE / LF_KEPT (MODE_LEARNED); PER as in k_faces
+template <int MODE, int WHAT, bool PER, typename T>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_xlast(KP p, int upd, const double* __restrict__ U0,
+                                                                                      const double* __restrict__ Ut, double* __restrict__ out) {
+    if (p.st->done) return;   // uniform: the whole grid leaves
+    const long long nf = (long long)(p.nx + 1) * p.ny * p.nz;
+    const int lane = threadIdx.x & 63;
+    const long long f = (xcd_block() * (blockDim.x >> 6) + (threadIdx.x >> 6)) * 63 + lane;
+    const bool active = f < nf;
+    int i = 0, j = 0, k = 0, t;
+    if (active) face_coords<5, 0>(p, f, i, j, k, t);
+    constexpr bool F64 = std::is_same<T, double>::value;
+    T Fc[5] = {}, Fv[4] = {};
+    double local = 0.0;
+    double sm;
+    if (F64 && in_range(p)) sm = xlast_face<MODE, WHAT, PER, T, F64>(p, active, f, i, j, k, Fc, Fv);
+    else sm = xlast_face<MODE, WHAT, PER, T, false>(p, active, f, i, j, k, Fc, Fv);
+    if (sm > local) local = sm;
+    xlast_cell<T>(p, active, lane, i, j, k, Fc, Fv, upd, U0, Ut, out);
     block_max_slot(p, local, SPD_CONV);
 }
 
