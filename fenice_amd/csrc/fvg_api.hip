@@ -495,9 +495,11 @@ bool stage_tiles(const fvg_ctx* c) {
     return c->NV == 4 && !c->fp32 && !c->learned && !c->quad4 && !c->fused && c->cfg.reconstruction != FVG_RECON_NONE &&
            c->cfg.ny / kStageTile < 65535;   // the grid's y extent
 }
-// One stage of the 2-D residual of Uin: stored into out (UPD_RESIDUAL), or combined into the stage output; out is not Uin
-int enqueue_stage_tiles(fvg_ctx* c, const double* Uin, int upd, const double* U0, const double* Ut, double* out) {
-    const KP p = make_kp(c, Uin);
+// One stage of the 2-D residual of Uin: stored into out (UPD_RESIDUAL), or combined into the stage output; out is neither
+// Uin nor R0 (KP::R0; only without sides that k_sides prepares: it reads Uin)
+int enqueue_stage_tiles(fvg_ctx* c, const double* Uin, int upd, const double* U0, const double* Ut, double* out, const double* R0 = nullptr) {
+    KP p = make_kp(c, Uin);
+    p.R0 = R0;
     int rc;
     if ((rc = enqueue_sides(c, p))) return rc;
     const dim3 g((c->cfg.nx + kStageTile - 1) / kStageTile, (c->cfg.ny + kStageTile - 1) / kStageTile);
@@ -631,8 +633,15 @@ int enqueue_step(fvg_ctx* c, int link = 0) {
         };
         if ((rc = residual_into(c, c->U, mode, c->learned, c->Rb))) return rc;
         if ((rc = enqueue_control(c, CTL_STAGE1_DT, ts))) return rc;
-        if ((rc = enqueue_axpy(c, c->U, c->Rb, ts == FVG_TS_EULER ? c->U : c->Ut))) return rc;
-        if (ts == FVG_TS_SSPRK2) {
+        // one pass less where the second stage's launch can form its input itself
+        const bool summed = !fused && !xlast && ts == FVG_TS_SSPRK3 && !c->massflow && !c->nrbc_sides;
+        if (!summed && (rc = enqueue_axpy(c, c->U, c->Rb, ts == FVG_TS_EULER ? c->U : c->Ut))) return rc;
+        if (summed) {
+            c->stage = 1;
+            rc = enqueue_stage_tiles(c, c->U, UPD_RK3_2, c->U, nullptr, c->Ut, c->Rb);
+            c->stage = 0;
+            if (rc || (rc = stage(2, c->Ut, UPD_RK3_3, c->U))) return rc;
+        } else if (ts == FVG_TS_SSPRK2) {
             if ((rc = stage(1, c->Ut, UPD_RK2_2, c->U))) return rc;
         } else if (ts == FVG_TS_SSPRK3) {
             if ((rc = stage(1, c->Ut, UPD_RK3_2, c->Rb))) return rc;

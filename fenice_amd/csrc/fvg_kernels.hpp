@@ -81,6 +81,7 @@ struct KP {
     // buffers (plane sets)
     // W, G, Fc and Fv hold doubles in the FP64 mode and floats in the FP32-flux mode (flux_precision)
     const double* U;    // stage input state (always FP64)
+    const double* R0;   // k_stage2d: the stage input is U + dt R0, never stored (null: U)
     void* W;            // primitives of U
     void* G;            // viscous cell gradients (3-D: 9 planes G[a][b] at 3a+b; 2-D: dudx, dudy, dvdx, dvdy)
     double* HS;         // MUSCL-Hancock predicted states: (2*ndim) * NV planes, state s = 2*axis + high (FP64 only)

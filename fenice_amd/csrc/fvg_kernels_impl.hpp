@@ -44,6 +44,13 @@ __device__ __forceinline__ bool in_range(const KP& p) { return p.ir != 0 && __bu
 template <int NV> __device__ __forceinline__ void load_cons(const KP& p, long long c, double* u) {
 #pragma unroll
     for (int q = 0; q < NV; ++q) u[q] = p.U[q * p.nc + c];
+#ifdef FVG_SUMMED_INPUT   // the unit of k_stage2d only: the test would cost the other kernels registers
+    if (p.R0) {
+        const double dt = p.st->dt;
+#pragma unroll
+        for (int q = 0; q < NV; ++q) u[q] = u[q] + dt * p.R0[q * p.nc + c];
+    }
+#endif
 }
 // element of cell (i, j, k) in the padded primitive planes (each coordinate from -PH)
 __device__ __forceinline__ long long pidx(const KP& p, int i, int j, int k) {

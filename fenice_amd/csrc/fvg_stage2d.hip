@@ -9,9 +9,12 @@
 // 15 x 16 y faces. It repeats 1/15 of the faces. Two blocks are resident on a CU (four wavefronts per SIMD, the
 // registers' limit), so one block's loads run under the other's arithmetic.
 // A stage never writes its own input (neighbouring tiles still read it): the first stage stores its residual, since
-// its step size is not known before every tile is done.
+// its step size is not known before every tile is done. The second SSP-RK3 stage forms the first one's result, U + dt R,
+// as it loads it (KP::R0) instead of reading what a pass of its own stored (a step of the 64^2 cavity 81 -> 77 us, of
+// 2048^2 1,340 -> 1,294).
 // Measured per step (SSP-RK3): viscous MUSCL cavity 32^2 125 -> 81 us, 64^2 118 -> 79, 400^2 170 -> 132; periodic WENO5-Z
 // 100 x 90 70 -> 44 us, 511 x 700 206 -> 159, 2048^2 1,798 -> 1,353.
+#define FVG_SUMMED_INPUT
 #include "fvg_kernels_impl.hpp"
 
 namespace fvg {
@@ -256,7 +259,17 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
         switch (upd) {   // uniform
         case UPD_RESIDUAL: combine<4, UPD_RESIDUAL>(p, c, R, U0, Ut, out); break;
         case UPD_RK2_2: combine<4, UPD_RK2_2>(p, c, R, U0, Ut, out); break;
-        case UPD_RK3_2: combine<4, UPD_RK3_2>(p, c, R, U0, Ut, out); break;
+        case UPD_RK3_2:
+            if (p.R0) {   // Ut = U + dt R0 as load_cons makes it
+                const double dt = p.st->dt;
+                double ut[4];
+                load_cons<4>(p, c, ut);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) out[q * p.nc + c] = 0.75 * U0[q * p.nc + c] + 0.25 * (ut[q] + dt * R[q]);
+            } else {
+                combine<4, UPD_RK3_2>(p, c, R, U0, Ut, out);
+            }
+            break;
         default: combine<4, UPD_RK3_3>(p, c, R, U0, Ut, out); break;
         }
     }
