@@ -711,7 +711,7 @@ int ensure_graph(fvg_ctx* c) {
 }
 
 // The device state set from and published to the host by one-wavefront kernels: two small copies and the wait took 14 us
-// of a step() call, these 8.
+// of a step() call.
 int write_state(fvg_ctx* c, const DevState& s) {
     *c->st_host = s;
     hipLaunchKernelGGL(k_set_state, dim3(1), dim3(64), 0, c->stream, c->st, s);

@@ -1354,6 +1354,7 @@ struct fvg_batch {
     unsigned* d_qnext = nullptr;
     TeamSync* d_sync = nullptr;
     TeamXch* d_txch = nullptr;           // exchanges of k_ensemble_lds's teams
+    int txch_teams = 0;                  // their number
     int lds_cap = 0;                     // lds_cells(): cells per workgroup of k_ensemble_lds, 0 without it
     double* d_xch = nullptr;             // 2-D teams: the exchange rows (BP2::xch), grown as plans need
     long long xch_cap = 0;               // its size in doubles
@@ -1571,6 +1572,7 @@ int launch_teams(fvg_batch* b, BP p) {
     std::vector<BTeam> teams;
     std::vector<int> queue;
     plan_teams(b, resident, BS, teams, queue);
+    if (lds && (int)teams.size() > b->txch_teams) return bset(b, FVG_ELOGIC, "more teams than exchanges");
     int wgs = 0;
     for (const BTeam& t : teams) wgs += t.m;
     const int grid = std::min(resident, wgs + (int)queue.size());
@@ -1830,7 +1832,10 @@ int fvg_batch_create(const fvg_config* cfg_in, int ninst, const int* ncells, int
         hipMalloc(&b->d_sync, sizeof(TeamSync) * ninst) != hipSuccess)
         return fail(FVG_ENOMEM, "hipMalloc of the ensemble buffers");
     b->lds_cap = lds_cells(b);
-    if (b->lds_cap && hipMalloc(&b->d_txch, sizeof(TeamXch) * ninst) != hipSuccess)
+    int cus = 0;   // a team takes two or more of the resident workgroups, at most 32 of which fit a CU
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || cus < 1) return fail(FVG_EHIP, "no CU count");
+    b->txch_teams = std::min(ninst, 32 * cus);
+    if (b->lds_cap && hipMalloc(&b->d_txch, sizeof(TeamXch) * b->txch_teams) != hipSuccess)
         return fail(FVG_ENOMEM, "hipMalloc of the ensemble buffers");
     int coop = 0;
     if (hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, device) == hipSuccess) b->coop = coop != 0;

@@ -112,7 +112,7 @@ __device__ __forceinline__ double recip_rho(double rho) {
     return r;
 }
 __device__ __forceinline__ float recip_rho(float rho) { return dv(1.0f, rho); }
-// x / c for a constant c > 0 with inv = RN(1 / c): Markstein's correction as in quot6 (with a correctly rounded
+// x / c for a constant c > 0 with inv = RN(1 / c): Markstein's correction (with a correctly rounded
 // reciprocal the corrected quotient is the IEEE one for every significand of c); FP32: the product
 template <bool IR> __host__ __device__ __forceinline__ double by_const(double x, double c, double inv) {
     if constexpr (IR) {

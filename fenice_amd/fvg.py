@@ -302,7 +302,7 @@ class Solver:
         return X, d
 
     def set_fused(self, on: bool):
-        """Runge-Kutta stages 2-3: the last axis' faces fused with the update (on) or separate passes (off, the
+        """Fused passes without face fluxes in device memory (on) or the sequence of the mesh and scheme (off, the
         default). Same bits."""
         self._c(lib().fvg_set_fused(self._h, int(on)))
 

@@ -230,10 +230,10 @@ int fvg_set_timing(fvg_ctx* ctx, int on);
 int fvg_set_graphs(fvg_ctx* ctx, int on);
 /* Kernel sequence of the residual (no counterpart in the reference): 1, fused passes, in which no face flux goes to
  * device memory: the x faces' differences go straight into per-cell partial sums, the y faces' are added to them,
- * and the last axis' pass finishes the residual and applies the stage combination; 0 (default), separate face
- * passes storing the fluxes and one update pass. The same bits either way; on MI355X the separate passes measured
- * as fast for FP64 fluxes and faster for FP32 fluxes and the learned indicator. The fourth-order quadrature always
- * takes its own passes. */
+ * and the last axis' pass finishes the residual and applies the stage combination; 0 (default), the sequence of the
+ * mesh and scheme: one launch per stage (2-D, FP64), face passes that store their fluxes with the update in the x faces
+ * (3-D), or face passes and an update. The same bits either way; the default is the faster one on MI355X. The
+ * fourth-order quadrature always takes its own passes. */
 int fvg_set_fused(fvg_ctx* ctx, int on);
 
 /* Known-answer entry: the Riemann flux of n faces with host AoS conservative states (5 doubles per face),
