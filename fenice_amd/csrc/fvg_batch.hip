@@ -231,7 +231,7 @@ __device__ __forceinline__ void bface(const BP& b, const BInst& in, const double
         roundtrip<4>(b.rs.eos, UL);
         roundtrip<4>(b.rs.eos, UR);
     }
-    face_flux<4>(b.rs, UL, UR, 0, F, sm);
+    face_flux<4, false, true>(b.rs, UL, UR, 0, F, sm);
 }
 
 // wave speed of the two (equal) y faces of cell i: the speed face_flux(u, u, y) returns for the cell's face state u,
@@ -244,7 +244,7 @@ __device__ __forceinline__ double by_speed(const BP& b, const double* w, double 
     if constexpr (RECON != 0) {   // the face state is the round trip p2c(c2p(u))
         double u2[4], w2[4], inv2;
         p2c<4>(b.rs.eos, w, u2);
-        c2p<4>(b.rs.eos, u2, w2, &inv2);
+        c2p<4, false, true>(b.rs.eos, u2, w2, &inv2);
         return sound_speed_inv(b.rs.eos, w2[3], inv2);
     }
     return sound_speed_inv(b.rs.eos, w[3], inv);
@@ -348,7 +348,7 @@ __device__ void run_instance(const BP& b, int id, int r, int m, TeamSync* ts, do
             for (int i = ch.lo + (int)threadIdx.x; i < ch.hi; i += BS) {
                 double u[4], w[4], inv;
                 bload_cons(b, in, Us, i, u);
-                c2p<4>(b.rs.eos, u, w, &inv);
+                c2p<4, false, true>(b.rs.eos, u, w, &inv);
                 const long long c = in.c0 + i;
                 b.W[c] = w[0];
                 b.W[b.nc + c] = w[1];
