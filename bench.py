@@ -27,16 +27,16 @@ sys.path.insert(0, ROOT)
 HBM_PEAK_GBS = 8000.0          # MI355X HBM3E, published
 FP64_VECTOR_PEAK_TFLOPS = 78.6  # MI355X FP64 vector, published (FMA counted as 2)
 BYTES_PER_CELL_STAGE_RK3_3D = 8.0 * 5 * (2 + 3 + 3) / 3.0   # 106.7 B: stage input, U^n on stages 2-3, output
-# HBM bytes of one stage of the 256^3 workload (k_cells + k_faces x/y/z + k_update, the update averaged over the
-# three SSP-RK3 stages), from two rocprofv3 --pmc runs (FETCH_SIZE x 2.0, WRITE_SIZE x 1.0, the factors a 1 GiB
+# HBM bytes of one stage of the 256^3 workload (k_cells, the y and z faces, the x faces with the update and the first
+# stage's k_axpy, averaged over the three SSP-RK3 stages), from two rocprofv3 --pmc runs (FETCH_SIZE x 2.0, WRITE_SIZE x 1.0, the factors a 1 GiB
 # device copy reads in the same runs); the runs and per-kernel figures are in the profile files named here. These
 # are figures of those counter runs, not of the run that prints them.
-MEASURED_STAGE_TRAFFIC = {("fp64", 256): (16.888e9, "profiles/tgv256_weno5_rk3_fp64.md"),
-                          ("fp32", 256): (7.678e9, "profiles/tgv256_weno5_rk3_fp32.md")}
-# VALU instructions per wavefront (SQ_INSTS_VALU / SQ_WAVES, one face or cell per lane) of each kernel of the
+MEASURED_STAGE_TRAFFIC = {("fp64", 256): (15.275e9, "profiles/tgv256_weno5_rk3_fp64.md"),
+                          ("fp32", 256): (7.919e9, "profiles/tgv256_weno5_rk3_fp32.md")}
+# VALU instructions per 64 faces or cells (SQ_INSTS_VALU / SQ_WAVES, one face per lane, 16 cells per lane in k_cells) of each kernel of the
 # workload, from the same counter runs; with this run's event time of the kernel they give its VALU issue rate. A
 # wave64 VALU instruction occupies a SIMD for 4 cycles; MI355X has 1,024 SIMDs at up to 2.4 GHz.
-VALU_PER_WAVE = {"fp64": ({"k_cells": 578, "k_faces_x": 1893, "k_faces_y": 1902, "k_faces_z": 1873}, "profiles/tgv256_weno5_rk3_fp64.md")}
+VALU_PER_WAVE = {"fp64": ({"k_cells": 346, "k_faces_x": 1684, "k_faces_y": 1540, "k_faces_z": 1476}, "profiles/tgv256_weno5_rk3_fp64.md")}
 SIMDS, CLOCK_HZ = 1024, 2.4e9
 
 from fenice_amd.workloads import taylor_green as tgv_state  # noqa: E402
@@ -566,7 +566,8 @@ def main():
     valu = None
     vt, vsrc = VALU_PER_WAVE.get(a.flux, ({}, ""))
     if n == 256 and a.indicator == "none" and dom[0] in vt:
-        waves = ((n + 1) * n * n + 63) // 64 if dom[0].startswith("k_faces") else cells // 64
+        nf = (n + 1) * n * n   # the x faces' wavefronts overlap by one face
+        waves = (nf + 61) // 63 if dom[0] == "k_faces_x" else (nf + 63) // 64 if dom[0].startswith("k_faces") else cells // 64
         avg_s = dom[1][0] / dom[1][1] * 1e-3
         issue = vt[dom[0]] * waves * 4.0 / (SIMDS * CLOCK_HZ * avg_s)
         valu = {"kernel": dom[0], "instr_per_wave": vt[dom[0]], "waves": waves, "avg_ms": round(avg_s * 1e3, 4),
