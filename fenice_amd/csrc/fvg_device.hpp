@@ -67,6 +67,12 @@ __host__ __device__ __forceinline__ bool range_fits_quot6(double v) {
 // at least 2^-458 and the last quotient at least 2^-570; van Leer's 2 a b is at least 2^-906. The Riemann solver
 // divides by densities and pressures of at least 1e-10 and by speed differences of at least 1e-14; its contact
 // speed, whose numerator may be any small number, keeps the IEEE division.
+// The advanced states of MUSCL-Hancock are not reconstructed values: they move with the half step, which a caller may
+// choose (fvg_residual). An admissible one has a density above 1e-10 and an energy whose product with it bounds the
+// momenta, so with both at most 2^200 (state_moderate, also DevState::wide) the momenta are at most 2^201, the
+// velocities 2^235, the pressure 2^220, the sound speed between 2^-117 and 2^127, the contact speed's numerator at most
+// 2^672 and its quotient 2^719, so that no speed is NaN; the solver's other denominators lie between 2^-47 and 2^720
+// and its numerators are zero or at least 2^-204.
 __device__ __forceinline__ double rcp_refined(double b) {   // the compiler's reciprocal: two Newton steps
     double r = __builtin_amdgcn_rcp(b);
     r = __builtin_fma(r, __builtin_fma(-b, r, 1.0), r);
@@ -138,6 +144,9 @@ __host__ __device__ __forceinline__ bool value_in_range(double v) {
     const double m = v < 0.0 ? -v : v;
     return (v == 0.0) | ((m >= 0x1p-400) & (m <= 0x1p+100));   // no short-circuit branches
 }
+
+// an admissible conservative state of MUSCL-Hancock's face fluxes, see above
+__host__ __device__ __forceinline__ bool state_moderate(const double* u) { return (u[0] <= 0x1p+200) & (u[3] <= 0x1p+200); }
 
 // the absolute floor of the WENO regularisation: 1e-300 in FP64 (Schemes.cpp:331, 343); the smallest power of ten
 // above FLT_MIN in FP32, where 1e-300 would round to zero and 0/0 would reach the weights of an all-zero stencil

@@ -26,7 +26,7 @@ struct Tile {
     double W[4][WY][WX];
     double S[4][4][SY][SX];          // advanced states: low x, high x, low y, high y side of the cell
     double Fx[4][TY][TX + 1], Fy[4][TY + 1][TX];
-    int wide[8];
+    int wide[8], wide_states[8];
 };
 
 // coordinate g (from -2) of a periodic axis of n cells; n may be smaller than the tile
@@ -35,9 +35,10 @@ __device__ __forceinline__ int wrapped(int g, int n) {
     return g < n ? g : g % n;
 }
 
-// the advanced states of the cell at (lx, ly) of the S arrays; returns how many were inadmissible and kept
+// the advanced states of the cell at (lx, ly) of the S arrays; returns how many were inadmissible and kept; wide is set
+// when an advanced one is not state_moderate
 template <bool IR>
-__device__ __forceinline__ int advance_states(const KP& p, Tile& s, int lx, int ly, double half_dt) {
+__device__ __forceinline__ int advance_states(const KP& p, Tile& s, int lx, int ly, double half_dt, bool& wide) {
     constexpr int NV = 4;
     double st[4][NV];
 #pragma unroll
@@ -67,6 +68,7 @@ __device__ __forceinline__ int advance_states(const KP& p, Tile& s, int lx, int 
         for (int q = 0; q < NV; ++q) nw[q] = st[k][q] - dd[q];
         const bool ok = admissible<NV>(p, nw);
         kept += ok ? 0 : 1;
+        wide |= ok & !state_moderate(nw);
 #pragma unroll
         for (int q = 0; q < NV; ++q) s.S[k][q][ly][lx] = ok ? nw[q] : st[k][q];
     }
@@ -130,15 +132,22 @@ __global__ __launch_bounds__(512) void k_hancock_step2d(KP p, const double* __re
     int nwide = 0;   // every value this tile reads is in range, or none of the in-range operations is used
 #pragma unroll
     for (int k = 0; k < 8; ++k) nwide |= s.wide[k];
-    const bool ir = p.ir != 0 && __builtin_amdgcn_readfirstlane(nwide) == 0;
+    bool ir = p.ir != 0 && __builtin_amdgcn_readfirstlane(nwide) == 0;
+    wide = false;
     if (t < SX * SY) {
         const int lx = t % SX, ly = t / SX;
-        const int kept = ir ? advance_states<true>(p, s, lx, ly, half_dt) : advance_states<false>(p, s, lx, ly, half_dt);
+        const int kept = ir ? advance_states<true>(p, s, lx, ly, half_dt, wide) : advance_states<false>(p, s, lx, ly, half_dt, wide);
         const int gi = i0 + lx - 1, gj = j0 + ly - 1;
         if (kept && lx >= 1 && lx <= TX && ly >= 1 && ly <= TY && gi < p.nx && gj < p.ny)
             atomicAdd((unsigned long long*)&p.st->reverted, (unsigned long long)kept);
     }
+    const bool any_state = __any(wide);
+    if ((t & 63) == 0) s.wide_states[t >> 6] = any_state;
     __syncthreads();
+    nwide = 0;
+#pragma unroll
+    for (int k = 0; k < SX * SY / 64; ++k) nwide |= s.wide_states[k];
+    ir = ir && __builtin_amdgcn_readfirstlane(nwide) == 0;
     double speed = 0.0;   // a face beyond the mesh in a ragged tile is a face of the wrapped cells
     const int h = t & 255;
     if (t < 256) {

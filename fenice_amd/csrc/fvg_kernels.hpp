@@ -25,10 +25,12 @@ struct DevState {
     int done, diverged, steps, max_steps;
     double ut[6];   // mass-flow inlet velocity per side of the current residual (k_sides)
     // nonzero: a value k_cells stored for the residual's stencils (a primitive of the FP64 planes or, with the
-    // fourth-order quadrature, a value of the padded conservative planes) is outside value_in_range, so the kernels
-    // take the IEEE divisions and roots. k_cells only sets it; k_update (the end of every residual of the separate
-    // passes) and k_control (after a residual's faces or between steps) clear it, never between a k_cells and the
-    // kernels that read its planes.
+    // fourth-order quadrature, a value of the padded conservative planes) is outside value_in_range, or a state that
+    // k_hancock advanced is not state_moderate, so the kernels take the IEEE divisions and roots. k_cells and k_hancock
+    // only set it; k_update (the end of every residual of the separate passes) and k_control (after a residual's faces
+    // or between steps) clear it, never between a k_cells and the kernels that read its planes. The stages that
+    // k_xlast and k4_xlast end have no k_update: a flag set in the second one holds for the third, which then takes the
+    // slower form of the same bits.
     int wide;
 };
 

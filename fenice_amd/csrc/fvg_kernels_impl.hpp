@@ -37,8 +37,9 @@ __device__ __forceinline__ int vper_of(const KP& p, int a) { return a == 0 ? p.v
 __device__ __forceinline__ int wrap_of(const KP& p, int a) { return a == 0 ? p.wrap[0] : (a == 1 ? p.wrap[1] : p.wrap[2]); }
 
 __device__ __forceinline__ double inv_hstep(const KP& p, int d) { return d == 0 ? p.inv_h[0] : (d == 1 ? p.inv_h[1] : p.inv_h[2]); }
-// whether the residual's FP64 operands are in range (fvg_device.hpp): uniform over the launch, since k_cells finished
-// before it and nothing else sets the flag
+// whether the residual's FP64 operands are in range (fvg_device.hpp): uniform over a launch of the faces, since k_cells
+// and k_hancock, which alone set the flag, finished before it (in k_hancock, whose own operands k_cells has settled,
+// both forms give the same bits)
 __device__ __forceinline__ bool in_range(const KP& p) { return p.ir != 0 && __builtin_amdgcn_readfirstlane(p.st->wide) == 0; }
 
 template <int NV> __device__ __forceinline__ void load_cons(const KP& p, long long c, double* u) {
@@ -676,7 +677,7 @@ __device__ __forceinline__ bool admissible(const KP& p, const double* u) {
     return (u[0] > kEosEps) && (0.5 * (u[1] * u[1] + u[2] * u[2] + u4 * u4) < u[0] * (u[3] - p.rs.eos.p_inf));
 }
 template <int NV, bool IR>
-__device__ __forceinline__ unsigned long long hancock_cell(const KP& p, long long c) {
+__device__ __forceinline__ unsigned long long hancock_cell(const KP& p, long long c, bool& wide) {
     constexpr int ND = NV - 2, NS = 2 * ND;
     unsigned long long reverted = 0;
     {
@@ -733,6 +734,7 @@ __device__ __forceinline__ unsigned long long hancock_cell(const KP& p, long lon
             for (int q = 0; q < NV; ++q) nw[q] = st[s][q] - dd[q];
             const bool ok = admissible<NV>(p, nw);
             reverted += ok ? 0 : 1;
+            wide |= ok & !state_moderate(nw);
 #pragma unroll
             for (int q = 0; q < NV; ++q) p.HS[((long long)s * NV + q) * p.nc + c] = ok ? nw[q] : st[s][q];
         }
@@ -743,7 +745,9 @@ template <int NV>
 __global__ __launch_bounds__(256) void k_hancock(KP p) {
     const long long c = xcd_block() * blockDim.x + threadIdx.x;
     if (c >= p.nc || p.st->done) return;
-    const unsigned long long reverted = in_range(p) ? hancock_cell<NV, true>(p, c) : hancock_cell<NV, false>(p, c);
+    bool wide = false;   // a state that the faces take is not state_moderate
+    const unsigned long long reverted = in_range(p) ? hancock_cell<NV, true>(p, c, wide) : hancock_cell<NV, false>(p, c, wide);
+    if (wide) p.st->wide = 1;
     if (reverted) atomicAdd((unsigned long long*)&p.st->reverted, reverted);
 }
 
