@@ -489,11 +489,29 @@ int enqueue_axpy(fvg_ctx* c, const double* U0, const double* R, double* out) {
 // whether the residuals of this context take the fused passes (the fourth-order quadrature keeps its own passes)
 bool fused_path(const fvg_ctx* c) { return c->fused && !c->quad4; }
 
+// Whether tiles of side `tile` suit the mesh: a tile costs about the same however few of its rows are cells, so a long
+// mesh of few rows is better off with the separate passes, which pack cells and faces into wavefronts. Up to 1,024
+// tiles (two rounds of two blocks per CU) the launches that the tiles save decide; with three rows of tiles or more,
+// most of them are full. Columns need no such rule: a narrow mesh leaves the separate passes' wavefronts as empty.
+// share: the rows of the tiles that must be cells. Measured, microseconds a step, tiles against separate passes:
+//   k_stage2d, periodic WENO5-Z: 10^6 x 1 2,695 / 487, 250,000 x 4 946 / 455, 100,000 x 8 438 / 352, x 10 448 / 421,
+//     x 12 453 / 487, 60,000 x 16 459 / 395, 50,000 x 20 440 / 412, 40,000 x 24 370 / 396, 30,000 x 31 379 / 389,
+//     20,000 x 1 (1,334 tiles) 77 / 60, 10,000 x 4 (667) 60 / 69; 8 x 100,000 462 / 548;
+//   viscous MUSCL: 10^6 x 1 3,833 / 604, 100,000 x 8 407 / 340, x 12 420 / 486, 50,000 x 20 429 / 405, x 24 350 / 388;
+//   inviscid MUSCL: 10^6 x 1 1,949 / 428, 100,000 x 8 282 / 251, x 10 284 / 301, 50,000 x 20 287 / 291;
+//   k_hancock_step2d: 10^6 x 2 1,126 / 300, 250,000 x 4 301 / 153, 100,000 x 8 134 / 110, x 10 132 / 136, 60,000 x 15
+//     159 / 121, 50,000 x 20 136 / 133, 40,000 x 28 113 / 152; 4 x 250,000 304 / 396.
+bool tiles_suit(const fvg_ctx* c, int tile, double share) {
+    const long long cols = (c->cfg.nx + tile - 1) / tile, rows = (c->cfg.ny + tile - 1) / tile;
+    return cols * rows <= 1024 || rows > 2 || c->cfg.ny >= share * (double)(rows * tile);
+}
+
 // whether the Runge-Kutta stages of this context run as one launch each (k_stage2d): 2-D, FP64 fluxes, reconstructed
-// faces. Faster than the separate passes at every size measured (see the kernel).
+// faces, a mesh that suits its tiles
 bool stage_tiles(const fvg_ctx* c) {
+    const bool light = c->cfg.reconstruction == FVG_RECON_MUSCL && !c->cfg.use_viscous;
     return c->NV == 4 && !c->fp32 && !c->learned && !c->quad4 && !c->fused && c->cfg.reconstruction != FVG_RECON_NONE &&
-           c->cfg.ny / kStageTile < 65535;   // the grid's y extent
+           tiles_suit(c, kStageTile, light ? 0.65 : 0.72) && c->cfg.ny / kStageTile < 65535;   // the grid's y extent
 }
 // One stage of the 2-D residual of Uin: stored into out (UPD_RESIDUAL), or combined into the stage output; out is neither
 // Uin nor R0 (KP::R0; only without sides that k_sides prepares: it reads Uin)
@@ -568,10 +586,11 @@ int plain_mode(const fvg_ctx* c) {
     return c->cfg.reconstruction == FVG_RECON_NONE ? MODE_FIRST_ORDER : MODE_PLAIN;
 }
 
-// MUSCL-Hancock steps of a periodic, inviscid 2-D mesh in one launch (k_hancock_step2d)
+// MUSCL-Hancock steps of a periodic, inviscid 2-D mesh in one launch (k_hancock_step2d), where the mesh suits its tiles
 bool hancock_tiles(const fvg_ctx* c) {
     return c->NV == 4 && c->cfg.time_scheme == FVG_TS_HANCOCK && c->cfg.reconstruction == FVG_RECON_MUSCL && !c->cfg.use_viscous &&
-           c->base.wrap[0] && c->base.wrap[1] && !c->fused && c->cfg.ny / kHancockTile < 65535;   // the grid's y extent
+           c->base.wrap[0] && c->base.wrap[1] && !c->fused && tiles_suit(c, kHancockTile, 0.7) &&
+           c->cfg.ny / kHancockTile < 65535;   // the grid's y extent
 }
 int enqueue_hancock_tiles(fvg_ctx* c) {
     const KP p = make_kp(c, c->U);
