@@ -34,18 +34,21 @@ __device__ __forceinline__ void end_step(DevState* s) {
 // The mass-flow inlet velocity of a mass-flow side (apply_side, Boundaries.cpp:285-294): rho_in u_in over the mean
 // density of the side's boundary cells, floored at 1e-5, into DevState::ut, which the ghost states of the residual read.
 // The densities are summed in the reference's boundary order (Core.hpp:121-151) by one thread, so that the sum has the
-// reference's bits: a chain of n dependent additions, about 17 cycles each. The block loads a chunk into LDS at a time
-// and the thread reads the next values into registers while it adds the ones before them. 64 x 48 boundary cells: 30 us
-// when the additions waited for the reads and 6 for the launch of the non-reflecting side, 26 for both now.
-constexpr int kMassflowChunk = 4096, kMassflowAhead = 32;
-__device__ void massflow_side(const KP& p, int side, double* rho) {
+// reference's bits: a chain of n dependent additions, about 17 cycles each. The block loads the first chunk into LDS;
+// then the thread adds one chunk, reading the next values into registers while it adds the ones before them, and the
+// other wavefronts load the next one. 64 x 48 boundary cells: 30 us when the additions waited for the reads and 6 for
+// the launch of the non-reflecting side, 26 for both now. A step of 512 x 16 x 512 with a side of 262,144 cells: 6,860 us
+// by a block of 1,024 threads that loaded and added in turn, 7,690 by 256 such threads, 5,760 now; of 16 x 256 x 256
+// 2,490, 2,300 and 1,930.
+constexpr int kMassflowChunk = 2048, kMassflowAhead = 32;
+__device__ void massflow_side(const KP& p, int side, double (*rho)[kMassflowChunk + kMassflowAhead]) {
     const long long nx = p.nx, ny = p.ny, nz = p.nz;
     const long long n = side < 2 ? ny * nz : (side < 4 ? nx * nz : nx * ny);
-    double sum = 0.0;
-    for (long long base = 0; base < n; base += kMassflowChunk) {
-        const int m = n - base < kMassflowChunk ? (int)(n - base) : kMassflowChunk;
-        const int whole = (m + 2 * kMassflowAhead - 1) / (2 * kMassflowAhead) * (2 * kMassflowAhead);
-        for (int l = threadIdx.x; l < whole + kMassflowAhead; l += blockDim.x) {
+    auto cells = [&](long long base) { return n - base < kMassflowChunk ? (int)(n - base) : kMassflowChunk; };
+    auto whole = [](int m) { return (m + 2 * kMassflowAhead - 1) / (2 * kMassflowAhead) * (2 * kMassflowAhead); };
+    auto load = [&](double* to, long long base, int first, int threads) {   // the chunk from base on, zeros behind it
+        const int m = cells(base), end = whole(m) + kMassflowAhead;
+        for (int l = first; l < end; l += threads) {
             const long long k = base + l;
             long long c;
             switch (side) {
@@ -56,24 +59,37 @@ __device__ void massflow_side(const KP& p, int side, double* rho) {
             case 4: c = k; break;
             default: c = (nz - 1) * ny * nx + k; break;
             }
-            rho[l] = l < m ? smax(p.U[c], kEosEps) : 0.0;   // the density of cons_to_prim; + 0 leaves the sum as it is
+            to[l] = l < m ? smax(p.U[c], kEosEps) : 0.0;   // the density of cons_to_prim; + 0 leaves the sum as it is
         }
-        __syncthreads();
-        if (threadIdx.x == 0) {
+    };
+    double sum = 0.0;
+    int cur = 1;
+#pragma unroll 1
+    for (long long base = -kMassflowChunk; base < n; base += kMassflowChunk, cur ^= 1) {   // before the first chunk, every thread loads
+        const int first = base < 0 ? 0 : 64;
+        if (base >= 0 && threadIdx.x == 0) {
+            const double* v = (const double*)__builtin_assume_aligned(rho[cur], 16);
+            const int end = whole(cells(base));
             double a[kMassflowAhead], b[kMassflowAhead];
 #pragma unroll
-            for (int q = 0; q < kMassflowAhead; ++q) a[q] = rho[q];
+            for (int q = 0; q < kMassflowAhead; ++q) a[q] = v[q];
 #pragma unroll 1
-            for (int l = 0; l < whole; l += 2 * kMassflowAhead) {
+            for (int l = 0; l < end; l += 2 * kMassflowAhead) {
 #pragma unroll
-                for (int q = 0; q < kMassflowAhead; ++q) b[q] = rho[l + kMassflowAhead + q];
+                for (int q = 0; q < kMassflowAhead; ++q) b[q] = v[l + kMassflowAhead + q];
+                __builtin_amdgcn_sched_barrier(0);   // the reads stay ahead of the additions before them
 #pragma unroll
                 for (int q = 0; q < kMassflowAhead; ++q) sum += a[q];
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int q = 0; q < kMassflowAhead; ++q) a[q] = rho[l + 2 * kMassflowAhead + q];
+                for (int q = 0; q < kMassflowAhead; ++q) a[q] = v[l + 2 * kMassflowAhead + q];
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int q = 0; q < kMassflowAhead; ++q) sum += b[q];
+                __builtin_amdgcn_sched_barrier(0);
             }
+        } else if ((int)threadIdx.x >= first && base + kMassflowChunk < n) {
+            load(rho[cur ^ 1], base + kMassflowChunk, threadIdx.x - first, blockDim.x - first);
         }
         __syncthreads();
     }
@@ -87,7 +103,7 @@ __device__ void massflow_side(const KP& p, int side, double* rho) {
 // mass-flow side s, blocks (x, s) the ghosts of a non-reflecting side's boundary cells (bit s of nrbc).
 template <int NV>
 __global__ __launch_bounds__(256) void k_sides(KP p, int nrbc) {
-    __shared__ double rho[kMassflowChunk + kMassflowAhead];
+    __shared__ __align__(16) double rho[2][kMassflowChunk + kMassflowAhead];
     if (p.st->done) return;
     const int side = blockIdx.y;
     if (!(nrbc >> side & 1)) {
