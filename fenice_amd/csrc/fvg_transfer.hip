@@ -5,7 +5,9 @@
 // separate copy; host threads fill or drain the slots (one thread copies 12-30 GB/s, and 5-14 GB/s into pages that a
 // caller has just allocated, so large arrays take several). Measured (up / down): 256^3 Taylor-Green, 671 MB,
 // 18 / 15 ms (36 / 44 GB/s), 206 / 216 ms with the conversion on one host thread through a pageable vector; 2048^2
-// Kelvin-Helmholtz, 134 MB, 3.9 / 4.3 ms against 42 / 43; 101 x 75 x 52, 15.8 MB, 0.5 / 0.5 ms against 2.4 / 4.4.
+// Kelvin-Helmholtz, 134 MB, 3.9 / 4.3 ms against 42 / 43; 101 x 75 x 52, 15.8 MB, 0.5 / 0.5 ms against 2.4 / 4.4. A
+// single chunk is latency: it waits for the stream itself, without an event (164 KB 19 / 20 us, 24-28 / 21-24 with one,
+// 21-30 / 20-22 by pageable copies; 40 KB 16 / 16, 16-20 / 16-19, 14-15 / 13).
 #include "fvg_transfer.hpp"
 
 #include <algorithm>
@@ -67,7 +69,7 @@ hipError_t HostCopy::lane(int j, int nlanes, hipStream_t stream, double* host, l
         else if (ncomp == 4) convert<4>(stream, up, slot[s], n, planes, stride, first(c), map);
         else convert<3>(stream, up, slot[s], n, planes, stride, first(c), map);
         const hipError_t e = hipGetLastError();
-        return e != hipSuccess ? e : hipEventRecord(done[s], stream);
+        return e != hipSuccess || nchunks == 1 ? e : hipEventRecord(done[s], stream);
     };
     hipError_t e = hipSuccess;
     if (up) {
@@ -85,7 +87,7 @@ hipError_t HostCopy::lane(int j, int nlanes, hipStream_t stream, double* host, l
         int k = 0;
         for (long long c = j; c < nchunks && e == hipSuccess; c += nlanes, ++k) {
             const int s = kSlotsPerThread * j + k % kSlotsPerThread;
-            e = hipEventSynchronize(done[s]);
+            e = nchunks == 1 ? hipStreamSynchronize(stream) : hipEventSynchronize(done[s]);
             if (e != hipSuccess) break;
             std::memcpy(host + first(c) * ncomp, slot[s], (size_t)cells(c) * ncomp * sizeof(double));
             if (const long long next = c + (long long)kSlotsPerThread * nlanes; next < nchunks) e = launch(next, s);
@@ -144,7 +146,8 @@ hipError_t HostCopy::run(int device, hipStream_t stream, double* host, long long
     for (int j = 1; j < started; ++j) th[j].join();
     for (int j = 0; j < nlanes; ++j)
         if (err[j] != hipSuccess && e == hipSuccess) e = err[j];
-    const hipError_t es = hipStreamSynchronize(stream);   // also after a failed lane: no kernel may outlive the call
+    // also after a failed lane: no kernel may outlive the call
+    const hipError_t es = nchunks == 1 && !up && e == hipSuccess ? hipSuccess : hipStreamSynchronize(stream);
     if (e == hipSuccess) e = es;
     if (e != hipSuccess) what = "host copy of a state";
     return e;
