@@ -12,7 +12,7 @@
 
 #include <algorithm>
 #include <cstring>
-#include <system_error>
+#include <exception>
 #include <thread>
 
 namespace fvg {
@@ -137,7 +137,7 @@ hipError_t HostCopy::run(int device, hipStream_t stream, double* host, long long
                 err[j] = hipSetDevice(device);
                 if (err[j] == hipSuccess) err[j] = lane(j, nlanes, stream, host, ncells, ncomp, planes, stride, map, up, chunk);
             });
-        } catch (const std::system_error&) {   // no more threads: this one takes the other lanes
+        } catch (const std::exception&) {   // no more threads, or no memory for one: this one takes the other lanes
             break;
         }
     }
