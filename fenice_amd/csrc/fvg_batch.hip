@@ -1349,6 +1349,7 @@ struct fvg_batch {
     bool teams_set = false;              // fvg_batch_set_teams was called
     bool coop = false;                   // the device supports cooperative launches
     std::vector<double> cost;            // estimated work per instance (N^2 x initial wave speed)
+    std::vector<double> rate;            // estimated steps per unit of time
     BTeam* d_teams = nullptr;
     int* d_queue = nullptr;
     unsigned* d_qnext = nullptr;
@@ -1359,6 +1360,7 @@ struct fvg_batch {
     double* d_xch = nullptr;             // 2-D teams: the exchange rows (BP2::xch), grown as plans need
     long long xch_cap = 0;               // its size in doubles
     int plan_teams = 0, plan_team_wgs = 0, plan_grid = 0;   // the last launch's plan
+    int plan_lds = 0;                    // its cells in LDS (0: k_ensemble or k_ensemble2)
 };
 
 namespace {
@@ -1399,9 +1401,11 @@ void free_batch(fvg_batch* b) {
 }
 
 size_t lds_bytes(int cap) { return sizeof(double) * 3 * (size_t)(2 * cap + 2 * KH + 1); }
+// the cells that fit in `bytes` of LDS beside the kernel's own (about 200 bytes; LDS is given out in larger units)
+int lds_most(int bytes) { return (int)((bytes - 2048) / (int)(sizeof(double) * 3) - 2 * KH - 1) / 2; }
 
-// The cells that a workgroup of k_ensemble_lds holds, the largest instance's: 48 bytes each, so up to 3,300 or so in the
-// 160 KB of a CU. 0 where k_ensemble runs instead: larger instances, first-order faces (they read the conservative
+// The cells that a workgroup of k_ensemble_lds holds, the largest instance's: 48 bytes each, so up to about 3,400 in the
+// 160 KB of a CU. 0 where only k_ensemble can run: larger instances, first-order faces (they read the conservative
 // state of both cells) and an x side that is periodic on its own (a rank of a team does not hold the other end).
 int lds_cells(const fvg_batch* b) {
     if (b->dim != 1 || b->cfg.reconstruction == FVG_RECON_NONE) return 0;
@@ -1410,61 +1414,6 @@ int lds_cells(const fvg_batch* b) {
     if (hipDeviceGetAttribute(&shared, hipDeviceAttributeMaxSharedMemoryPerBlock, b->device) != hipSuccess) return 0;
     const int cap = *std::max_element(b->n.begin(), b->n.end());
     return lds_bytes(cap) + sizeof(LdsShared) + 64 <= (size_t)shared ? cap : 0;
-}
-
-// the launch's dynamic LDS, above the 64 KB that a kernel may take without asking
-template <int BS, int RECON>
-int lds_allow(fvg_batch* b) {
-    BCHK(b, hipFuncSetAttribute((const void*)k_ensemble_lds<BS, RECON>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes(b->lds_cap)));
-    return FVG_OK;
-}
-
-template <int BS>
-int launch_lds(fvg_batch* b, const BP& p) {
-    const dim3 g(b->ninst), t(BS);
-    const size_t by = lds_bytes(p.cap);
-    int rc = FVG_OK;
-    switch (p.recon) {
-    case 1:
-        if ((rc = lds_allow<BS, 1>(b))) return rc;
-        hipLaunchKernelGGL((k_ensemble_lds<BS, 1>), g, t, by, b->stream, p);
-        break;
-    case 2:
-        if ((rc = lds_allow<BS, 2>(b))) return rc;
-        hipLaunchKernelGGL((k_ensemble_lds<BS, 2>), g, t, by, b->stream, p);
-        break;
-    default:
-        if ((rc = lds_allow<BS, 3>(b))) return rc;
-        hipLaunchKernelGGL((k_ensemble_lds<BS, 3>), g, t, by, b->stream, p);
-        break;
-    }
-    return rc;
-}
-
-template <int BS>
-int launch_bs(fvg_batch* b, const BP& p) {
-    if (b->lds_cap) return launch_lds<BS>(b, p);
-    const dim3 g(b->ninst), t(BS);
-    if (b->dim == 2) {   // the run's time, dt_max and step limit go with the 2-D parameters
-        BP2 q = b->base2;
-        q.t_end = p.t_end;
-        q.dt_max = p.dt_max;
-        q.max_steps = p.max_steps;
-        switch (q.recon) {
-        case 0: hipLaunchKernelGGL((k_ensemble2<BS, 0>), g, t, 0, b->stream, q); break;
-        case 1: hipLaunchKernelGGL((k_ensemble2<BS, 1>), g, t, 0, b->stream, q); break;
-        case 2: hipLaunchKernelGGL((k_ensemble2<BS, 2>), g, t, 0, b->stream, q); break;
-        default: hipLaunchKernelGGL((k_ensemble2<BS, 3>), g, t, 0, b->stream, q); break;
-        }
-        return FVG_OK;
-    }
-    switch (p.recon) {
-    case 0: hipLaunchKernelGGL((k_ensemble<BS, 0>), g, t, 0, b->stream, p); break;
-    case 1: hipLaunchKernelGGL((k_ensemble<BS, 1>), g, t, 0, b->stream, p); break;
-    case 2: hipLaunchKernelGGL((k_ensemble<BS, 2>), g, t, 0, b->stream, p); break;
-    default: hipLaunchKernelGGL((k_ensemble<BS, 3>), g, t, 0, b->stream, p); break;
-    }
-    return FVG_OK;
 }
 
 // The teams of a launch of `grid` resident workgroups of `bs` threads. With force_teams every instance of at least
@@ -1478,12 +1427,13 @@ int launch_bs(fvg_batch* b, const BP& p) {
 // team at most max_team workgroups and the teams at most three quarters of the grid. The other instances form the
 // queue, longest first. Where fvg_batch_set_teams was not called, k_ensemble_lds takes teams of up to 16 workgroups of
 // 96 cells or more (its waits are cheap: 73 ms on the 512 instances of 128 .. 2,048 cells, 90 with 8 of 512).
-void plan_teams(const fvg_batch* b, int grid, int bs, std::vector<BTeam>& teams, std::vector<int>& queue) {
+// most: the cells that a workgroup may hold (0: any number); false where that takes more workgroups than a team or the
+// teams may have.
+bool plan_teams(const fvg_batch* b, bool lds, int most, int grid, int bs, std::vector<BTeam>& teams, std::vector<int>& queue) {
     teams.clear();
     queue.clear();
     const int ninst = (int)b->order.size();
     std::vector<int> m(b->n.size(), 1);
-    const bool lds = b->lds_cap > 0;
     const int max_team = b->teams_set || !lds ? b->max_team : kMaxTeam, min_chunk = b->teams_set || !lds ? b->min_chunk : 96;
     auto cap = [&](int id) {   // most workgroups instance id may take
         const int n = b->n[id];
@@ -1505,6 +1455,8 @@ void plan_teams(const fvg_batch* b, int grid, int bs, std::vector<BTeam>& teams,
                 wgs += k;
             }
         }
+        for (int id = 0; id < ninst; ++id)
+            if (most > 0 && b->n[id] > (long long)m[id] * most) return false;
     } else if (max_team > 1 && grid > 1) {
         const double A = lds ? 4.1 : 9.0, Bc = lds ? 0.0037 * std::sqrt(768.0 / std::min(bs, 768)) : 0.0065 * std::sqrt(1024.0 / bs),
                      C = lds ? 1.1 : 6.0;
@@ -1513,35 +1465,48 @@ void plan_teams(const fvg_batch* b, int grid, int bs, std::vector<BTeam>& teams,
             return steps * (A + Bc * n / k + (k > 1 ? C : 0.0));
         };
         double total = 0.0;
-        std::vector<std::pair<double, int>> heap;   // (modelled run, instance), longest on top
+        // (modelled run, instance), longest on top, of the instances that may take one more workgroup; the longest of
+        // the others stays below them (it ends the plan of k_ensemble and k_ensemble2)
+        std::vector<std::pair<double, int>> heap;
+        std::pair<double, int> stuck{-1.0, -1};
+        const int max_wgs = grid * 3 / 4;
         for (int id = 0; id < ninst; ++id) {
-            const double t = run(id, 1);
-            total += t;
-            heap.push_back({t, id});
+            const int k = cap(id);
+            if (most > 0 && b->n[id] > most) {
+                m[id] = (b->n[id] + most - 1) / most;
+                wgs += m[id];
+                if (m[id] > k || wgs > max_wgs) return false;
+            }
+            const double t = run(id, m[id]);
+            total += m[id] * t;
+            if (m[id] < k) heap.push_back({t, id});
+            else stuck = std::max(stuck, {t, id});
         }
         std::make_heap(heap.begin(), heap.end());
-        const int max_wgs = grid * 3 / 4;
         while (!heap.empty()) {
             std::pop_heap(heap.begin(), heap.end());
             const auto [t, id] = heap.back();
             heap.pop_back();
+            // k_ensemble_lds goes on: the others may be longer than modelled, their waves form after the first steps
+            if (!lds && stuck > std::pair<double, int>{t, id}) break;
             const int k = m[id] + 1, extra = (m[id] == 1 ? 2 : 1);
             if (wgs + extra > max_wgs) break;
-            if (k > cap(id)) {
-                if (lds) continue;   // the others may be longer than modelled: their waves form after the first steps
-                break;
-            }
             const double t2 = run(id, k);
             const double total2 = total - m[id] * t + k * t2;
-            const double next = heap.empty() ? 0.0 : heap.front().first;
             // taken while the bound does not rise (equal runs: the others follow) and this run gets shorter
-            if (!(t2 < t) || std::max(std::max(next, t2), total2 / grid) > std::max(t, total / grid)) break;
+            if (!(t2 < t) || std::max(t2, total2 / grid) > std::max(t, total / grid)) break;
             wgs += extra;
             m[id] = k;
             total = total2;
-            heap.push_back({t2, id});
-            std::push_heap(heap.begin(), heap.end());
+            if (k < cap(id)) {
+                heap.push_back({t2, id});
+                std::push_heap(heap.begin(), heap.end());
+            } else {
+                stuck = std::max(stuck, {t2, id});
+            }
         }
+    } else if (most > 0 && *std::max_element(b->n.begin(), b->n.end()) > most) {
+        return false;
     }
     wgs = 0;
     for (int id : b->order) {
@@ -1552,26 +1517,148 @@ void plan_teams(const fvg_batch* b, int grid, int bs, std::vector<BTeam>& teams,
             queue.push_back(id);
         }
     }
+    return true;
+}
+
+// Which kernel runs a 1-D ensemble whose instances all fit in LDS, and with how much LDS per workgroup. k_ensemble_lds
+// is the faster one per workgroup, but its workgroups all take the LDS of the largest chunk: one long instance among
+// many short ones, whole, leaves a CU a workgroup or two where registers would allow three of 256 threads, six of 128 or
+// twelve of 64, and short instances do not fill it. So where the LDS is what limits the residency, the plan that splits
+// the long instances until the most workgroups fit that teams allow, or else one of k_ensemble, is weighed against the
+// plan without a limit by this model: a stage takes a fixed time and one per pass of the workgroup over its cells
+// and faces; the workgroups of a CU overlap, less well the more there are, down to the time the cells' arithmetic takes,
+// and slow the longest run down while they are there.
+// Measured at 64, 128 and 256 threads, MUSCL (ms: k_ensemble / k_ensemble_lds with the LDS of the largest instance / this
+// rule): 4,000 instances of 128 cells and one of 3,000, 60 steps 4.8 / 13.5 / 2.1, 4.8 / 8.9 / 2.6, 5.5 / 6.9 / 3.4, to
+// t = 0.03 31.6 / 31.6 / 16.6, 18.1 / 23.9 / 10.7, 13.0 / 16.0 / 7.8; 20,000 of 16 and one of 3,300 to t = 0.03
+// 30.4 / 14.7 / 11.5, 19.8 / 11.0 / 7.1, 14.4 / 10.8 / 5.2; 500 of 128 .. 2,048 to t = 0.03 1,056 / 277 / 115,
+// 566 / 146 / 78, 357 / 91 / 91; 600 of 3,000, 60 steps (no team is left to split them) 22.6 / 32.6 / 22.6,
+// 13.3 / 17.2 / 13.4, 12.2 / 9.0 / 8.9, to t = 0.03 1,370 / 797 / 794, 799 / 418 / 417, 446 / 215 / 213. The model is
+// good to about a tenth, so another plan has to promise 5 % to be taken, and k_ensemble 10 %.
+struct StageModel {
+    double fixed, pass, cell, team;   // microseconds: per stage, per pass, per cell with a full CU, per stage of a team
+};
+StageModel stage_model(bool lds, int recon) {   // measured on MI355X, by reconstruction
+    if (lds) return recon == 1 ? StageModel{1.8, 1.95, 0.0065, 1.1} : (recon == 2 ? StageModel{1.8, 2.2, 0.0083, 1.1} : StageModel{1.8, 2.75, 0.0107, 1.1});
+    return recon == 1 ? StageModel{2.4, 2.8, 0.0105, 6.0} : (recon == 2 ? StageModel{2.4, 3.1, 0.012, 6.0} : StageModel{2.4, 4.75, 0.0172, 6.0});
+}
+
+struct Launch {
+    int cap = 0;                  // cells of a workgroup of k_ensemble_lds; 0: k_ensemble
+    int resident = 0;             // workgroups resident at once
+    std::vector<BTeam> teams;     // without teams every instance has its workgroup and both lists are empty
+    std::vector<int> queue;
+};
+
+// the modelled stages' time of a launch, in microseconds
+double modelled_time(const fvg_batch* b, const BP& p, const Launch& l, int bs, int cus) {
+    const StageModel s = stage_model(l.cap > 0, p.recon);
+    const double per_cu = (double)l.resident / cus, crowd = 1.0 + 0.2 * (per_cu - 1.0) * std::min(1.0, bs / 128.0);
+    double longest = 0.0, total = 0.0;
+    auto add = [&](int id, int m) {
+        const double chunk = std::ceil((double)b->n[id] / m);
+        const double steps = std::min((double)p.max_steps, p.t_end * std::max(b->rate[id], p.dt_max > 0.0 ? 1.0 / p.dt_max : 0.0));
+        const double t = s.fixed + s.pass * 0.5 * (std::ceil((chunk + 1.0) / bs) + std::ceil(chunk / bs)) + (m > 1 ? s.team : 0.0);
+        longest = std::max(longest, steps * t);
+        total += steps * m * std::max(crowd * t / per_cu, s.cell * chunk);
+    };
+    for (const BTeam& t : l.teams) add(t.inst, t.m);
+    for (int id : l.queue) add(id, 1);
+    if (l.teams.empty() && l.queue.empty())
+        for (int id : b->order) add(id, 1);
+    total /= cus;
+    return std::max(longest, total) + (1.0 - 1.0 / crowd) * std::min(longest, total);
+}
+
+// the kernel and, with teams, the plan of a launch of BS threads per workgroup
+template <int BS, int RECON>
+int choose_launch(fvg_batch* b, const BP& p, bool teams, Launch& best) {
+    const void* kern_lds = (const void*)k_ensemble_lds<BS, RECON>;
+    int cus = 0, shared = 0, most_wgs = 0;
+    BCHK(b, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, b->device));
+    // a plan whose workgroups hold at most `most` cells (k_ensemble_lds; 0: k_ensemble), `limit`: whether that binds it
+    auto plan = [&](int most, bool limit, Launch& l, bool& ok) -> int {
+        int per_cu = 0;
+        l.cap = most;
+        if (most > 0) BCHK(b, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern_lds, BS, lds_bytes(most)));
+        else BCHK(b, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)k_ensemble<BS, RECON>, BS, 0));
+        l.resident = per_cu * cus;
+        if (l.resident < 1) return bset(b, FVG_EHIP, "the ensemble kernel cannot be resident");
+        ok = !teams || plan_teams(b, most > 0, limit ? most : 0, l.resident, BS, l.teams, l.queue);
+        return FVG_OK;
+    };
+    bool ok = true;
+    int rc = FVG_OK;
+    if (b->lds_cap) BCHK(b, hipFuncSetAttribute(kern_lds, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes(b->lds_cap)));
+    if ((rc = plan(b->lds_cap, false, best, ok)) || !best.cap) return rc;
+    BCHK(b, hipOccupancyMaxActiveBlocksPerMultiprocessor(&most_wgs, kern_lds, BS, 0));
+    if (best.resident >= most_wgs * cus) return FVG_OK;   // the registers' limit, not the LDS
+    Launch other;
+    ok = false;
+    if (teams) {
+        BCHK(b, hipDeviceGetAttribute(&shared, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, b->device));
+        for (int wgs = most_wgs; wgs >= 1 && !ok; wgs = wgs == 3 ? 2 : wgs / 2) {
+            const int most = lds_most(shared / wgs);
+            if (most < KH || most >= b->lds_cap) continue;
+            other = Launch();
+            if ((rc = plan(most, true, other, ok))) return rc;
+        }
+    }
+    if (!ok) {
+        other = Launch();
+        if ((rc = plan(0, false, other, ok))) return rc;
+    }
+    if (modelled_time(b, p, other, BS, cus) < (other.cap ? 0.95 : 0.9) * modelled_time(b, p, best, BS, cus)) best = std::move(other);
+    return FVG_OK;
+}
+
+template <int BS>
+int launch_bs(fvg_batch* b, const BP& p) {
+    const dim3 g(b->ninst), t(BS);
+    if (b->dim == 2) {   // the run's time, dt_max and step limit go with the 2-D parameters
+        BP2 q = b->base2;
+        q.t_end = p.t_end;
+        q.dt_max = p.dt_max;
+        q.max_steps = p.max_steps;
+        switch (q.recon) {
+        case 0: hipLaunchKernelGGL((k_ensemble2<BS, 0>), g, t, 0, b->stream, q); break;
+        case 1: hipLaunchKernelGGL((k_ensemble2<BS, 1>), g, t, 0, b->stream, q); break;
+        case 2: hipLaunchKernelGGL((k_ensemble2<BS, 2>), g, t, 0, b->stream, q); break;
+        default: hipLaunchKernelGGL((k_ensemble2<BS, 3>), g, t, 0, b->stream, q); break;
+        }
+        return FVG_OK;
+    }
+    auto go = [&](auto recon) -> int {
+        constexpr int R = decltype(recon)::value;
+        Launch l;
+        const int rc = choose_launch<BS, R>(b, p, false, l);
+        if (rc) return rc;
+        b->plan_lds = l.cap;
+        if (l.cap) hipLaunchKernelGGL((k_ensemble_lds<BS, R>), g, t, lds_bytes(l.cap), b->stream, p);
+        else hipLaunchKernelGGL((k_ensemble<BS, R>), g, t, 0, b->stream, p);
+        return FVG_OK;
+    };
+    switch (p.recon) {
+    case 0: hipLaunchKernelGGL((k_ensemble<BS, 0>), g, t, 0, b->stream, p); return FVG_OK;
+    case 1: return go(std::integral_constant<int, 1>{});
+    case 2: return go(std::integral_constant<int, 2>{});
+    default: return go(std::integral_constant<int, 3>{});
+    }
 }
 
 // The teamed launch of the 1-D kernel: workgroups resident at once (a cooperative launch), teams then the queue.
 template <int BS, int RECON>
 int launch_teams(fvg_batch* b, BP p) {
-    const bool lds = b->lds_cap > 0;
+    Launch l;
+    const int rc = choose_launch<BS, RECON>(b, p, true, l);
+    if (rc) return rc;
+    const bool lds = l.cap > 0;
+    p.cap = l.cap;
     const void* kern = lds ? (const void*)k_ensemble_lds<BS, RECON> : (const void*)k_ensemble<BS, RECON>;
     const size_t by = lds ? lds_bytes(p.cap) : 0;
-    if (lds) {
-        const int rc = lds_allow<BS, RECON>(b);
-        if (rc) return rc;
-    }
-    int per_cu = 0, dev_cus = 0;
-    BCHK(b, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, BS, by));
-    BCHK(b, hipDeviceGetAttribute(&dev_cus, hipDeviceAttributeMultiprocessorCount, b->device));
-    const int resident = per_cu * dev_cus;
-    if (resident < 1) return bset(b, FVG_EHIP, "the ensemble kernel cannot be resident");
-    std::vector<BTeam> teams;
-    std::vector<int> queue;
-    plan_teams(b, resident, BS, teams, queue);
+    const int resident = l.resident;
+    const std::vector<BTeam>& teams = l.teams;
+    const std::vector<int>& queue = l.queue;
     if (lds && (int)teams.size() > b->txch_teams) return bset(b, FVG_ELOGIC, "more teams than exchanges");
     int wgs = 0;
     for (const BTeam& t : teams) wgs += t.m;
@@ -1594,6 +1681,7 @@ int launch_teams(fvg_batch* b, BP p) {
     b->plan_teams = (int)teams.size();
     b->plan_team_wgs = wgs;
     b->plan_grid = grid;
+    b->plan_lds = p.cap;
     return FVG_OK;
 }
 
@@ -1616,7 +1704,7 @@ int launch_teams2(fvg_batch* b, const BP& p) {
     if (resident < 1) return bset(b, FVG_EHIP, "the ensemble kernel cannot be resident");
     std::vector<BTeam> teams;
     std::vector<int> queue;
-    plan_teams(b, resident, BS, teams, queue);
+    plan_teams(b, false, 0, resident, BS, teams, queue);
     int wgs = 0;
     long long xn = 0;
     for (BTeam& t : teams) {
@@ -1674,6 +1762,7 @@ bool teamed(const fvg_batch* b, const BP& p) {
 }
 
 int launch_ensemble(fvg_batch* b, const BP& p, int block) {
+    b->plan_lds = 0;
     if (teamed(b, p) && b->dim == 2) {
         switch (block) {
         case 64: return launch_teams2_bs<64>(b, p);
@@ -1840,6 +1929,7 @@ int fvg_batch_create(const fvg_config* cfg_in, int ninst, const int* ncells, int
     int coop = 0;
     if (hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, device) == hipSuccess) b->coop = coop != 0;
     b->cost.assign(ninst, 0.0);
+    b->rate.assign(ninst, 0.0);
     if (hipMemcpy(b->d_inst, b->inst.data(), sizeof(BInst) * ninst, hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(b->d_order, b->order.data(), sizeof(int) * ninst, hipMemcpyHostToDevice) != hipSuccess)
         return fail(FVG_EHIP, "hipMemcpy of the instance table");
@@ -2007,6 +2097,8 @@ int fvg_batch_upload(fvg_batch* b, const double* U, long long ncells, int ncomp)
     std::vector<double> cost(b->ninst);
     BCHK(b, hipMemcpyAsync(cost.data(), b->d_speed, sizeof(double) * b->ninst, hipMemcpyDeviceToHost, b->stream));
     BCHK(b, hipStreamSynchronize(b->stream));
+    if (b->dim == 1)
+        for (int i = 0; i < b->ninst; ++i) b->rate[i] = cost[i] / (b->cfg.cfl * b->inst[i].Ldt);
     for (int i = 0; i < b->ninst; ++i)
         cost[i] = (double)b->n[i] * (b->dim == 2 ? std::max(b->inst2[i].nx, b->inst2[i].ny) : b->n[i]) * (cost[i] + 1e-3);
     std::stable_sort(b->order.begin(), b->order.end(), [&](int a, int c) { return cost[a] > cost[c]; });
@@ -2083,6 +2175,12 @@ int fvg_batch_get_plan(const fvg_batch* b, int* nteams, int* team_wgs, int* grid
     return FVG_OK;
 }
 
+int fvg_batch_get_lds(const fvg_batch* b, int* cells) {
+    if (!b || !cells) return FVG_EINVAL;
+    *cells = b->plan_lds;
+    return FVG_OK;
+}
+
 int fvg_batch_get_block(const fvg_batch* b, int* block) {
     if (!b || !block) return FVG_EINVAL;
     *block = b->block;
@@ -2133,7 +2231,10 @@ int fvg_batch_tune(fvg_batch* b, double t_probe, int max_steps, const char* cach
     // within the first steps): the queue order and the teams of later runs take N x probe steps as the work
     std::vector<BOut> o(b->ninst);
     BCHK(b, hipMemcpy(o.data(), b->d_out, sizeof(BOut) * b->ninst, hipMemcpyDeviceToHost));
-    for (int i = 0; i < b->ninst; ++i) b->cost[i] = (double)b->n[i] * std::max(1, o[i].steps);
+    for (int i = 0; i < b->ninst; ++i) {
+        b->cost[i] = (double)b->n[i] * std::max(1, o[i].steps);
+        if (b->dim == 1 && o[i].t > 0.0) b->rate[i] = o[i].steps / o[i].t;
+    }
     std::stable_sort(b->order.begin(), b->order.end(), [&](int a, int c) { return b->cost[a] > b->cost[c]; });
     BCHK(b, hipMemcpy(b->d_order, b->order.data(), sizeof(int) * b->ninst, hipMemcpyHostToDevice));
     BCHK(b, hipMemcpyAsync(b->U, b->Usave, cb, hipMemcpyDeviceToDevice, b->stream));

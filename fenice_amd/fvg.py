@@ -120,6 +120,7 @@ def lib():
         L.fvg_batch_tune.argtypes = [C.c_void_p, C.c_double, C.c_int, C.c_char_p, _I, _I]
         L.fvg_batch_set_teams.argtypes = [C.c_void_p, C.c_int, C.c_int, C.c_int]
         L.fvg_batch_get_plan.argtypes = [C.c_void_p, _I, _I, _I]
+        L.fvg_batch_get_lds.argtypes = [C.c_void_p, _I]
         F = C.POINTER(C.c_float)
         L.fvg_indicator_set.argtypes = [C.c_void_p, F, C.c_int, C.c_float]
         L.fvg_indicator_stats.argtypes = [C.c_void_p, C.POINTER(C.c_ulonglong), _I, _I]
@@ -429,6 +430,13 @@ class Ensemble:
         a, b, c = C.c_int(), C.c_int(), C.c_int()
         self._c(lib().fvg_batch_get_plan(self._h, C.byref(a), C.byref(b), C.byref(c)))
         return a.value, b.value, c.value
+
+    @property
+    def lds_cells(self) -> int:
+        """Cells that a workgroup of the last run held in LDS (0: the run kept them in global memory)."""
+        n = C.c_int()
+        self._c(lib().fvg_batch_get_lds(self._h, C.byref(n)))
+        return n.value
 
     def tune(self, t_probe: float, max_steps: int, cache_path: str | None = None):
         """Autotune the workgroup size on a probe run (the state is restored); returns (block, from_cache)."""

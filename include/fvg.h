@@ -315,16 +315,20 @@ int fvg_batch_tune(fvg_batch* b, double t_probe, int max_steps, const char* cach
 /* Teams of 1-D and 2-D instances (no reference counterpart: the reference runs one process per instance). The
  * largest instances run on several workgroups of one cooperative launch, each over its own chunk of at least
  * min_chunk cells, the team's workgroups waiting for each other in every stage; the other instances are taken one at a time, longest
- * first, by any workgroup. An instance gets a team when its estimated work is at least twice the average per resident
- * workgroup (as many workgroups as averages, at most max_team; teams use at most half of the workgroups); with
- * force, every instance of at least 2 min_chunk cells gets min(max_team, N / min_chunk). The chunks of a 2-D
- * instance are slabs of whole rows, at least 3 rows and min_chunk cells each. Results do not depend on the teams. Waits at a team barrier are bounded: a team that times out makes fvg_batch_run return FVG_EHIP.
+ * first, by any workgroup. The plan shortens the longest modelled run by one workgroup at a time, while that does not
+ * raise the bound of the whole launch, up to max_team workgroups for an instance and three quarters of the resident
+ * ones for all; with force, every instance of at least 2 min_chunk cells gets min(max_team, N / min_chunk). The chunks
+ * of a 2-D instance are slabs of whole rows, at least 3 rows and min_chunk cells each. Results do not depend on the
+ * teams. Waits at a team barrier are bounded: a team that times out makes fvg_batch_run return FVG_EHIP.
  * max_team = 1, first-order faces or a device without cooperative launches: one workgroup per instance.
  * Until this is called: max_team 8, min_chunk 512, force 0; 1-D instances that all fit in LDS (about 3,400 cells)
- * take up to 16 workgroups of at least 96 cells. max_team <= 16, min_chunk >= 3. */
+ * take up to 16 workgroups of at least 96 cells, also to leave room in LDS for more workgroups.
+ * max_team <= 16, min_chunk >= 3. */
 int fvg_batch_set_teams(fvg_batch* b, int max_team, int min_chunk, int force);
 /* The last fvg_batch_run's launch: teams, workgroups in teams, workgroups launched. */
 int fvg_batch_get_plan(const fvg_batch* b, int* nteams, int* team_wgs, int* grid);
+/* The cells that a workgroup of the last fvg_batch_run's launch held in LDS; 0: it kept them in global memory. */
+int fvg_batch_get_lds(const fvg_batch* b, int* cells);
 
 #ifdef __cplusplus
 }
