@@ -1841,6 +1841,8 @@ std::string tune_key(const fvg_batch* b) {
     std::ostringstream s;
     s << arch << "|" << b->ninst << "|" << b->nc << "|" << std::hex << h << std::dec << "|" << b->cfg.reconstruction << "|"
       << b->cfg.limiter << "|" << b->cfg.riemann << "|" << b->cfg.time_scheme;
+    // the kernels that a launch chooses from (the sides decide too whether LDS is one) and the teams it may form
+    s << "|lds" << b->lds_cap << "|teams" << (b->coop ? 1 : 0) << b->teams_set << "," << b->max_team << "," << b->min_chunk << "," << b->force_teams;
     return s.str();
 }
 

@@ -309,7 +309,7 @@ int fvg_batch_set_block(fvg_batch* b, int block);
 int fvg_batch_get_block(const fvg_batch* b, int* block);
 /* Autotuner: time every workgroup size on a probe run of the uploaded state (to t_probe, at most max_steps),
  * keep the fastest and restore the state. With cache_path, a line "key block ms" per tuned workload (device
- * architecture, instance sizes, scheme) is appended, and a later call for the same key reads it instead of
+ * architecture, instance sizes, scheme, kernel and team settings) is appended, and a later call for the same key reads it instead of
  * measuring (*from_cache = 1). */
 int fvg_batch_tune(fvg_batch* b, double t_probe, int max_steps, const char* cache_path, int* block, int* from_cache);
 /* Teams of 1-D and 2-D instances (no reference counterpart: the reference runs one process per instance). The

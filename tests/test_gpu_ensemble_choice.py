@@ -70,3 +70,22 @@ def test_sizes_of_the_lds_tests():
     for teams in ((1, 512, False), (3, 100, True)):
         assert launch(n[:1], U[:3400], 1024, 2, teams)[2] == 3400
         assert launch(n, U, 1024, 2, teams)[2] == 0
+
+
+def test_tuned_block_is_kept_for_the_same_kernel_and_teams(tmp_path):
+    say("ensemble choice: tuner's cache")
+    n, U = states([64] * 40)
+    cache = tmp_path / "tune.txt"
+
+    def tune(teams=None):
+        with fvg.Ensemble(fvg.config_from_keys(ensemble_keys()), n) as e:
+            if teams:
+                e.set_teams(*teams)
+            e.upload(U)
+            return e.tune(0.002, 20, str(cache))[1]
+
+    assert not tune() and tune()
+    assert not tune(teams=(1, 512)) and tune(teams=(1, 512)) and not tune(teams=(4, 20)) and not tune(teams=(4, 20, True))
+    key, rest = cache.read_text().splitlines()[0].split(" ", 1)
+    cache.write_text(key[:key.index("|lds")] + " " + rest + "\n")   # a line that does not say which kernel it was for
+    assert not tune()
