@@ -57,5 +57,15 @@ def build(verbose: bool = False) -> str:
     return LIB
 
 
+def build_check() -> str:
+    """tests/libarith_check.so: the known-answer kernel of the in-range FP64 operations, with the library's flags."""
+    tests = os.path.join(ROOT, "tests")
+    lib = os.path.join(tests, "libarith_check.so")
+    _run([HIPCC, "-x", "hip", *COMMON, *DEVICE, "-shared", os.path.join(tests, "arith_check.hip"), "-o", lib + ".tmp"])
+    os.replace(lib + ".tmp", lib)
+    return lib
+
+
 if __name__ == "__main__":
     print(build(verbose=True))
+    print(build_check())

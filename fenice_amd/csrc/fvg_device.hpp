@@ -42,7 +42,7 @@ __device__ __forceinline__ float sq(float a) { return __builtin_amdgcn_sqrtf(a);
 // or 2/3, which puts x/6 at least 1/6 ulp from every midpoint, so the result is the IEEE quotient. Zeros keep their
 // sign. Below the range the quotient may be subnormal and a midpoint (x = 9 2^-1074 gives 2^-1074, the division
 // 2 2^-1074); above it, or for non-finite x, the FMA can overflow or give NaN: callers keep the IEEE division there
-// (range_fits_quot6).
+// (value_in_range below, whose bounds are narrower than those that quot6 needs, range_fits_quot6).
 __host__ __device__ __forceinline__ double quot6(double x) {
     constexpr double a = 1.0 / 6.0, b = 0x1p-54 / 6.0;
     return __builtin_fma(x, a, x * b);
@@ -59,7 +59,9 @@ __host__ __device__ __forceinline__ bool range_fits_quot6(double v) {
 // in them. When neither operand needs the scaling (denominator and its reciprocal normal, quotient normal or zero,
 // |numerator| >= 2^-969 or zero), scaling multiplies by one and the same reciprocal, Newton steps and correction
 // give the same bits without it: 57 cycles with the fixup (which keeps zeros, infinities and NaN as IEEE has them), 52
-// without it, 53 for the square root.
+// without it, 53 for the square root. (The compiler's division, and so these, misses the IEEE quotient by one ulp for a
+// few operands within 2^-53 ulp of a midpoint with a divisor just below a power of two, for instance
+// 0x1.6666666666663p+52 / 0x1.ffffffffffffbp+52.)
 // The kernels take these forms when every primitive that k_cells stored is zero or between 2^-400 and 2^100 in
 // magnitude (value_in_range; DevState::wide) and the configuration's constants are moderate (KP::ir). Then, with
 // WENO5-Z (eps at least 2^-42 of the stencil's mean square): differences are zero or at least 2^-453, the smoothness
