@@ -230,6 +230,7 @@ int launch_faces_recon(fvg_ctx* c, const KP& p) {
 }
 template <int NV, int D, typename T>
 int launch_faces(fvg_ctx* c, const KP& p, int mode) {
+    if (!c->Fc[D]) return set_err(c, FVG_ELOGIC, "no planes of the face fluxes");
     if (mode == MODE_FIRST_ORDER)
         return launch(c, FAM_FACES_X + D, [&] {
             hipLaunchKernelGGL((k_faces<NV, D, MODE_FIRST_ORDER, 0, false, T>), dim3(faces_grid(c, D)), dim3(faces_block(c, D)), 0, c->stream, p);
@@ -343,6 +344,7 @@ int enqueue_hancock_faces(fvg_ctx* c, const KP& p) {
 
 template <int NV>
 int enqueue_hancock_residual(fvg_ctx* c, const double* Uin) {
+    if (!c->Fc[0]) return set_err(c, FVG_ELOGIC, "no planes of the face fluxes");
     const KP p = make_kp(c, Uin);
     int rc;
     if ((rc = enqueue_sides(c, p))) return rc;
@@ -372,6 +374,7 @@ int enqueue_control(fvg_ctx* c, int op, int arg) {
 
 template <int NV, typename T>
 int enqueue_update_nv(fvg_ctx* c, int upd, const double* U0, const double* Ut, double* out) {
+    if (!c->Fc[0]) return set_err(c, FVG_ELOGIC, "no planes of the face fluxes");
     const KP p = c->base;
     const dim3 g(cells_grid(c)), b(cells_block(c));
     return launch(c, FAM_UPDATE, [&] {
@@ -803,11 +806,14 @@ int checked_alloc(fvg_ctx* c, P** p, size_t n, size_t elem = sizeof(double)) {
 }
 
 // the face-flux planes of the separate face and update passes: per axis NV convective planes (FP32 fluxes: the
-// combined flux) and, with FP64 fluxes and viscosity, NV - 1 viscous planes
-int alloc_face_fluxes(fvg_ctx* c, const fvg_config& cfg) {
+// combined flux) and, with FP64 fluxes and viscosity, NV - 1 viscous planes. Those of the x faces of a 3-D mesh, 72 bytes
+// a cell in FP64 (1.2 GB at 256^3), only where k_xlast and k4_xlast do not keep them in registers (x_planes): first-order
+// and MUSCL-Hancock runs, and from the first residual with a predictor on.
+int alloc_face_fluxes(fvg_ctx* c, const fvg_config& cfg, bool x_planes) {
     const size_t fe = c->fp32 ? sizeof(float) : sizeof(double);
     int rc = FVG_OK;
     for (int d = 0; d < c->ND; ++d) {
+        if (d == 0 && c->NV == 5 && !x_planes) continue;
         if (!c->Fc[d]) rc = rc ? rc : checked_alloc(c, &c->Fc[d], (size_t)c->NV * c->nfa[d], fe);
         if (cfg.use_viscous && !c->fp32 && !c->Fv[d]) rc = rc ? rc : checked_alloc(c, &c->Fv[d], (size_t)(c->NV - 1) * c->nfa[d], fe);
     }
@@ -1050,7 +1056,7 @@ int fvg_create(const fvg_config* cfg_in, int device, fvg_ctx** out) {
     c->quad4 = cfg.flux_quadrature == FVG_QUAD_FOURTH;
     // the face-flux planes of the separate passes (the default, and the fourth-order quadrature's); the accumulators
     // of the fused passes are allocated when fvg_set_fused switches to them
-    rc = rc ? rc : alloc_face_fluxes(c, cfg);
+    rc = rc ? rc : alloc_face_fluxes(c, cfg, cfg.reconstruction == FVG_RECON_NONE || cfg.time_scheme == FVG_TS_HANCOCK);
     const long long q4_n = std::max({c->nfa[0], c->nfa[1], c->nfa[2]});
     if (c->quad4) {   // the padded conservative state and one axis' face states, flags and point-value fluxes
         rc = rc ? rc : checked_alloc(c, &c->Wc, (size_t)NV * npad);
@@ -1187,6 +1193,11 @@ int fvg_residual(fvg_ctx* c, double half_dt, double* R, int ncomp, double* s_max
     if (hancock && !c->HS) {
         if ((rc = checked_alloc(c, &c->HS, (size_t)2 * c->ND * c->NV * c->nc))) return rc;
         c->base.HS = c->HS;
+    }
+    if (hancock && !c->Fc[0]) {
+        if ((rc = alloc_face_fluxes(c, c->cfg, true))) return rc;
+        c->base.Fc[0] = c->Fc[0];
+        c->base.Fv[0] = c->Fv[0];
     }
     s.half_dt = hancock ? half_dt : 0.0;
     if ((rc = write_state(c, s))) return rc;
