@@ -231,6 +231,7 @@ def cpu_ensemble_worker(procs: int, steps: int) -> dict:
     import multiprocessing as mp
     from fenice_amd.workloads import riemann_ensemble
     ninst = len(riemann_ensemble()[0])
+    C.CDLL(os.path.join(ROOT, "oracle", "_ref", "libfenice_ref.so"))   # an error here, not in every worker the pool would start anew
     with mp.get_context("fork").Pool(procs, initializer=_ens_init) as pool:
         pool.map(_ens_run, [(i, 1) for i in range(procs)])   # warm every process (library, instances)
         t0 = time.perf_counter()
