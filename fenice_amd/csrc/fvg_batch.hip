@@ -172,7 +172,7 @@ __device__ __forceinline__ void boutside(const BP& b, const BInst& in, const dou
 
 // face f (between cells f - 1 and f) of the instance: the reconstruction (RECON = fvg_recon) and Riemann solve
 // of the face pass
-template <int RECON>
+template <int BS, int RECON>
 __device__ __forceinline__ void bface(const BP& b, const BInst& in, const double* Us, const Chunk& ch, int f, double* F, double& sm) {
     const int n = in.n;
     const bool lo = f == 0, hi = f == n;
@@ -231,7 +231,7 @@ __device__ __forceinline__ void bface(const BP& b, const BInst& in, const double
         roundtrip<4>(b.rs.eos, UL);
         roundtrip<4>(b.rs.eos, UR);
     }
-    face_flux<4, false, true>(b.rs, UL, UR, 0, F, sm);
+    face_flux<4, false, true, (RECON != 0 && BS < 1024)>(b.rs, UL, UR, 0, F, sm);
 }
 
 // wave speed of the two (equal) y faces of cell i: the speed face_flux(u, u, y) returns for the cell's face state u,
@@ -380,7 +380,7 @@ __device__ void run_instance(const BP& b, int id, int r, int m, TeamSync* ts, do
             // x faces (k_faces)
             for (int f = ch.lo + (int)threadIdx.x; f <= ch.hi; f += BS) {
                 double F[4], sm;
-                bface<RECON>(b, in, Us, ch, f, F, sm);
+                bface<BS, RECON>(b, in, Us, ch, f, F, sm);
                 if (sm > local) local = sm;
                 if (extra && f == ch.hi) {
                     fx[0] = F[0];

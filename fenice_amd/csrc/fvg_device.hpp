@@ -233,13 +233,39 @@ struct RiemannParams {
     double blend;
 };
 
+// the flux of a state normal to axis, and the side's factor of its star state and that state
+template <int NV, typename T>
+__device__ __forceinline__ void state_flux(const T* W, T E, int axis, T* F) {
+    const int mn = mom(axis);
+    const T rho = W[0], p = W[3], Vn = W[mn];
+    F[0] = rho * Vn;
+#pragma unroll
+    for (int a = 0; a < NV - 2; ++a) F[mom(a)] = rho * W[mom(a)] * Vn;
+    F[mn] = F[mn] + p;
+    F[3] = Vn * (rho * E + p);
+}
+template <int NV, bool IR, typename T>
+__device__ __forceinline__ void star_state(const T* W, T E, T S, T S_M, int axis, T* Us) {
+    const T rho = W[0], p = W[3], Vn = W[mom(axis)];
+    const T f = dvx<IR>(rho * (S - Vn), safe_denom<IR>(S - S_M));
+    Us[0] = f;
+#pragma unroll
+    for (int a = 0; a < NV - 2; ++a) Us[mom(a)] = f * (a == axis ? S_M : W[mom(a)]);
+    Us[3] = f * (E + (S_M - Vn) * (S_M + dvx<IR>(p, rho * safe_denom<IR>(S - Vn))));
+}
+
 // HLLC with Einfeldt bounds, the contact speed of Toro (10.37) and the shock blend toward HLL
 // (Schemes.cpp:116-200). vel index a = 0, 1, 2 maps to W[1], W[2], W[4].
 // The flux of a face comes from one side of its contact: the side is picked first, by selecting its eleven or so
 // inputs, and only that side's flux, star state and two of its quotients are computed; the reference computes both
 // and picks the result. Which side its four successive conditions leave: the right one when S_R < 0 or
 // S_M < 0 <= S_R, else the left one, and zero when none of them holds (NaN speeds).
-template <int NV, bool IR = false, typename T>
+// BOTH: as the reference, for k_ensemble, which waits for a face's chain of operations rather than for their number:
+// all that does not need the contact speed is on its way beside its quotient (1,024 instances to t = 0.03: 2.34-2.36 s,
+// 2.38-2.42 with one side; 600 of 4,000 cells, 60 steps: MUSCL at 768 threads 12.0 ms against 12.6, WENO5 at 256 32.5
+// against 33.6). Its first-order faces and 1,024-thread workgroups, which spill, take one (4.5 against 4.8 ms; MUSCL 13.8
+// against 14.2).
+template <int NV, bool IR = false, bool BOTH = false, typename T>
 __device__ __forceinline__ void hllc_core(const RiemannParams& rs, const T* WL, const T* WR, const T* UL, const T* UR, T inv_L,
                                           T inv_R, T c_L, T c_R, int axis, T* F, T& smax_out) {
     const T rho_L = WL[0], p_L = WL[3];
@@ -251,56 +277,58 @@ __device__ __forceinline__ void hllc_core(const RiemannParams& rs, const T* WL, 
     const T num = rho_R * Vn_R * (S_R - Vn_R) - rho_L * Vn_L * (S_L - Vn_L) + p_L - p_R;
     const T den = rho_R * (S_R - Vn_R) - rho_L * (S_L - Vn_L);
     const T S_M = dv(num, safe_denom<IR>(den));
-    const bool right = (S_R < T(0)) | ((S_M < T(0)) & (S_R >= T(0)));
-    const bool star = right ? S_R >= T(0) : (S_L < T(0)) & (S_M >= T(0));
-    const bool none = !IR & !right & !star & !(S_L >= T(0));   // not with finite speeds
-    T W[NV], U[NV];
-#pragma unroll
-    for (int q = 0; q < NV; ++q) {
-        W[q] = right ? WR[q] : WL[q];
-        U[q] = right ? UR[q] : UL[q];
-    }
-    const T S = right ? S_R : S_L;
-    const T rho = W[0], p = W[3], Vn = W[mn];
-    const T E = U[3] * (right ? inv_R : inv_L);
     T Fo[NV];
-    Fo[0] = rho * Vn;
-#pragma unroll
-    for (int a = 0; a < NV - 2; ++a) Fo[mom(a)] = rho * W[mom(a)] * Vn;
-    Fo[mn] = Fo[mn] + p;
-    Fo[3] = Vn * (rho * E + p);
-    const T f = dvx<IR>(rho * (S - Vn), safe_denom<IR>(S - S_M));
-    T Us[NV];
-    Us[0] = f;
-#pragma unroll
-    for (int a = 0; a < NV - 2; ++a) Us[mom(a)] = f * (a == axis ? S_M : W[mom(a)]);
-    Us[3] = f * (E + (S_M - Vn) * (S_M + dvx<IR>(p, rho * safe_denom<IR>(S - Vn))));
-#pragma unroll
-    for (int q = 0; q < NV; ++q) {
-        const T s = Fo[q] + S * (Us[q] - U[q]);
-        Fo[q] = star ? s : Fo[q];
-    }
-    if (none)
+    if constexpr (BOTH) {
+        T FL[NV], FR[NV], UsL[NV], UsR[NV];
+        const T E_L = UL[3] * inv_L, E_R = UR[3] * inv_R;
+        state_flux<NV>(WL, E_L, axis, FL);
+        state_flux<NV>(WR, E_R, axis, FR);
+        star_state<NV, IR>(WL, E_L, S_L, S_M, axis, UsL);
+        star_state<NV, IR>(WR, E_R, S_R, S_M, axis, UsR);
 #pragma unroll
         for (int q = 0; q < NV; ++q) Fo[q] = T(0);
+        if (S_L >= T(0))
+#pragma unroll
+            for (int q = 0; q < NV; ++q) Fo[q] = FL[q];
+        if (S_L < T(0) && S_M >= T(0))
+#pragma unroll
+            for (int q = 0; q < NV; ++q) Fo[q] = FL[q] + S_L * (UsL[q] - UL[q]);
+        if (S_M < T(0) && S_R >= T(0))
+#pragma unroll
+            for (int q = 0; q < NV; ++q) Fo[q] = FR[q] + S_R * (UsR[q] - UR[q]);
+        if (S_R < T(0))
+#pragma unroll
+            for (int q = 0; q < NV; ++q) Fo[q] = FR[q];
+    } else {
+        const bool right = (S_R < T(0)) | ((S_M < T(0)) & (S_R >= T(0)));
+        const bool star = right ? S_R >= T(0) : (S_L < T(0)) & (S_M >= T(0));
+        const bool none = !IR & !right & !star & !(S_L >= T(0));   // not with finite speeds
+        T W[NV], U[NV], Us[NV];
+#pragma unroll
+        for (int q = 0; q < NV; ++q) {
+            W[q] = right ? WR[q] : WL[q];
+            U[q] = right ? UR[q] : UL[q];
+        }
+        const T S = right ? S_R : S_L, E = U[3] * (right ? inv_R : inv_L);
+        state_flux<NV>(W, E, axis, Fo);
+        star_state<NV, IR>(W, E, S, S_M, axis, Us);
+#pragma unroll
+        for (int q = 0; q < NV; ++q) {
+            const T s = Fo[q] + S * (Us[q] - U[q]);
+            Fo[q] = star ? s : Fo[q];
+        }
+        if (none)
+#pragma unroll
+            for (int q = 0; q < NV; ++q) Fo[q] = T(0);
+    }
     if (rs.blend > 0.0) {
         const T blend = T(rs.blend);
         const T s = dvx<IR>(fabs(p_R - p_L), nmin<IR>(p_L, p_R));
         if (s > blend) {
             const T phi = smin(dv(s - blend, blend), T(1.0));
-            const T E_L = UL[3] * inv_L, E_R = UR[3] * inv_R;
             T FL[NV], FR[NV];
-            FL[0] = rho_L * Vn_L;
-            FR[0] = rho_R * Vn_R;
-#pragma unroll
-            for (int a = 0; a < NV - 2; ++a) {
-                FL[mom(a)] = rho_L * WL[mom(a)] * Vn_L;
-                FR[mom(a)] = rho_R * WR[mom(a)] * Vn_R;
-            }
-            FL[mn] = FL[mn] + p_L;
-            FR[mn] = FR[mn] + p_R;
-            FL[3] = Vn_L * (rho_L * E_L + p_L);
-            FR[3] = Vn_R * (rho_R * E_R + p_R);
+            state_flux<NV>(WL, UL[3] * inv_L, axis, FL);
+            state_flux<NV>(WR, UR[3] * inv_R, axis, FR);
             T Fh[NV];
             if (S_L >= T(0)) {
 #pragma unroll
@@ -324,7 +352,7 @@ __device__ __forceinline__ void hllc_core(const RiemannParams& rs, const T* WL, 
 
 // RiemannSolver::face_flux (Schemes.cpp:108-113, 202-229). One hllc_core for both solvers (its code is inlined once):
 // the low-Mach variant blends the velocities first.
-template <int NV, bool IR = false, bool PLAIN = false, typename T>
+template <int NV, bool IR = false, bool PLAIN = false, bool BOTH = false, typename T>
 __device__ __forceinline__ void face_flux(const RiemannParams& rs, const T* UL0, const T* UR0, int axis, T* F, T& sm) {
     T WL[NV], WR[NV], UL[NV], UR[NV], inv_L, inv_R;
 #pragma unroll
@@ -336,6 +364,11 @@ __device__ __forceinline__ void face_flux(const RiemannParams& rs, const T* UL0,
     c2p<NV, IR, PLAIN>(rs.eos, UR, WR, &inv_R);
     const T c_L = sound_speed_inv<IR>(rs.eos, WL[3], inv_L);
     const T c_R = sound_speed_inv<IR>(rs.eos, WR[3], inv_R);
+    if constexpr (BOTH)
+        if (!rs.lowmach) {
+            hllc_core<NV, IR, true>(rs, WL, WR, UL0, UR0, inv_L, inv_R, c_L, c_R, axis, F, sm);
+            return;
+        }
     if (rs.lowmach) {
         T ML2 = WL[1] * WL[1] + WL[2] * WL[2], MR2 = WR[1] * WR[1] + WR[2] * WR[2];
         if constexpr (NV == 5) {
@@ -356,7 +389,7 @@ __device__ __forceinline__ void face_flux(const RiemannParams& rs, const T* UL0,
         p2c<NV, IR>(rs.eos, WL, UL);
         p2c<NV, IR>(rs.eos, WR, UR);
     }
-    hllc_core<NV, IR>(rs, WL, WR, UL, UR, inv_L, inv_R, c_L, c_R, axis, F, sm);
+    hllc_core<NV, IR, BOTH>(rs, WL, WR, UL, UR, inv_L, inv_R, c_L, c_R, axis, F, sm);
 }
 
 // ---- limiters (Schemes.hpp:90-117) and WENO-Z (Schemes.cpp:323-353) ----
