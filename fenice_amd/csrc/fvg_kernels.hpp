@@ -9,7 +9,8 @@
 // (stencil, reconstruction, Riemann solve, viscous face flux; block maximum of the wave speed then one 64-bit
 // atomicMax) -> k_control (time step on the device) -> k_update (flux divergence, viscous balance and the
 // stage combination of the time scheme, fused). On 3-D meshes k_xlast takes the x faces and the update in one pass; on 2-D
-// meshes with FP64 fluxes k_stage2d takes a whole stage, k_hancock_step2d a whole periodic MUSCL-Hancock step.
+// meshes with FP64 fluxes, but for long ones of few rows, k_stage2d takes a whole stage, k_hancock_step2d a whole
+// periodic MUSCL-Hancock step.
 #pragma once
 
 #include "fvg_learned.hpp"
